@@ -2732,8 +2732,8 @@ clexmc_status clexmc_wave_pick_device(clexmc_handle *h, int n_rows, const float 
   return CLEXMC_OK;
 }
 
-static TrainArgs train_args(clexmc_handle *h, int n, const int8_t *dX, const float *dy, const float *dt, float *dH,
-                            float *ddl, float *dloss, float *dgrad) {
+static TrainArgs train_args(clexmc_handle *h, int n, const int8_t *dX, const float *dy, const float *dt, int n_part,
+                            double *dpart, float *dgrad, float *dloss) {
   TrainArgs t;
   t.n = n;
   t.n_env = h->n_env;
@@ -2744,14 +2744,12 @@ static TrainArgs train_args(clexmc_handle *h, int n, const int8_t *dX, const flo
   t.b1 = h->d_mlp_params + kHidden * kEnvMax;
   t.W2 = h->d_mlp_params + kHidden * kEnvMax + kHidden;
   t.b2 = h->d_mlp_params + kHidden * kEnvMax + 2 * kHidden;
-  t.H = dH;
-  t.dl = ddl;
-  t.loss = dloss;
+  t.n_part = n_part;
+  t.part = dpart;
   t.grad = dgrad;
+  t.loss = dloss;
   return t;
 }
-
-
 
 clexmc_status clexmc_mlp_gradients(clexmc_handle *h, int n, const int8_t *X, const float *y, const float *t,
                                    float *grad_out, float *loss_out) {
@@ -2760,29 +2758,24 @@ clexmc_status clexmc_mlp_gradients(clexmc_handle *h, int n, const int8_t *X, con
   HIP_TRY(hipSetDevice(h->device));
   DevBufs B;
   int8_t *dX;
-  float *dy, *dt = nullptr, *dH, *ddl, *dloss, *dg;
+  float *dy, *dt = nullptr, *dg;
+  double *dpart;
+  const int n_part = mlp_train_parts(n, h->n_cu);
   HIP_TRY(B.alloc(&dX, (size_t)n * kEnvMax));
   HIP_TRY(B.alloc(&dy, n));
   if (t) {
     HIP_TRY(B.alloc(&dt, n));
     HIP_TRY(hipMemcpy(dt, t, sizeof(float) * n, hipMemcpyHostToDevice));
   }
-  HIP_TRY(B.alloc(&dH, (size_t)n * kHidden));
-  HIP_TRY(B.alloc(&ddl, n));
-  HIP_TRY(B.alloc(&dloss, n));
-  HIP_TRY(B.alloc(&dg, kNParams));
+  HIP_TRY(B.alloc(&dpart, (size_t)n_part * mlp_part_bytes() / sizeof(double)));
+  HIP_TRY(B.alloc(&dg, kNParams + 1));
   HIP_TRY(hipMemcpy(dX, X, (size_t)n * kEnvMax, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(dy, y, sizeof(float) * n, hipMemcpyHostToDevice));
-  HIP_TRY(launch_mlp_train_step(train_args(h, n, dX, dy, dt, dH, ddl, dloss, dg), h->stream));
+  AdamArgs none{};
+  HIP_TRY(launch_mlp_train_step(train_args(h, n, dX, dy, dt, n_part, dpart, dg, dg + kNParams), none, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   HIP_TRY(hipMemcpy(grad_out, dg, sizeof(float) * kNParams, hipMemcpyDeviceToHost));
-  if (loss_out) {
-    std::vector<float> l(n);
-    HIP_TRY(hipMemcpy(l.data(), dloss, sizeof(float) * n, hipMemcpyDeviceToHost));
-    double acc = 0.0;
-    for (float v : l) acc += v;
-    *loss_out = (float)(acc / n);
-  }
+  if (loss_out) HIP_TRY(hipMemcpy(loss_out, dg + kNParams, sizeof(float), hipMemcpyDeviceToHost));
   return CLEXMC_OK;
 }
 
@@ -2839,14 +2832,14 @@ clexmc_status clexmc_mlp_train(clexmc_handle *h, int n_per_chain, int n_steps, f
   ARG_CHECK(n < (1u << 24), "training batch too large");
   DevBufs B;
   int8_t *dX;
-  float *dy, *dt, *dH, *ddl, *dloss, *dg;
+  float *dy, *dt, *dloss;
+  double *dpart;
+  const int n_part = mlp_train_parts((int)n, h->n_cu);
   HIP_TRY(B.alloc(&dX, n * kEnvMax));
   HIP_TRY(B.alloc(&dy, n));
   HIP_TRY(B.alloc(&dt, n));
-  HIP_TRY(B.alloc(&dH, n * kHidden));
-  HIP_TRY(B.alloc(&ddl, n));
-  HIP_TRY(B.alloc(&dloss, n));
-  HIP_TRY(B.alloc(&dg, kNParams));
+  HIP_TRY(B.alloc(&dpart, (size_t)n_part * mlp_part_bytes() / sizeof(double)));
+  HIP_TRY(B.alloc(&dloss, (size_t)n_steps));
   if (!h->mlp_initialized) {
     // He initialisation of a fresh network (a zero network has dead ReLUs):
     // W1 ~ N(0, 2/n_env) on the used inputs, b1 = 0.1, W2 ~ N(0, 1/64), b2 = 0
@@ -2866,30 +2859,21 @@ clexmc_status clexmc_mlp_train(clexmc_handle *h, int n_per_chain, int n_steps, f
   }
   clexmc_status st = collect_device(h, n_per_chain, seed, include_chem, dX, dy, dt);
   if (st != CLEXMC_OK) return st;
-  std::vector<float> l(n);
   for (int it = 0; it < n_steps; ++it) {
-    HIP_TRY(launch_mlp_train_step(train_args(h, (int)n, dX, dy, dt, dH, ddl, dloss, dg), h->stream));
     h->adam_t += 1;
     AdamArgs ad;
-    ad.n_params = kNParams;
     ad.p = h->d_mlp_params;
     ad.m = h->d_adam_m;
     ad.v = h->d_adam_v;
-    ad.grad = dg;
     ad.lr = lr;
     ad.b1m = 0.9f;
     ad.b2m = 0.999f;
     ad.b1t = (float)std::pow(0.9, (double)h->adam_t);
     ad.b2t = (float)std::pow(0.999, (double)h->adam_t);
-    HIP_TRY(launch_mlp_adam(ad, h->stream));
-    if (loss_out) {
-      HIP_TRY(hipMemcpyAsync(l.data(), dloss, sizeof(float) * n, hipMemcpyDeviceToHost, h->stream));
-      HIP_TRY(hipStreamSynchronize(h->stream));
-      double acc = 0.0;
-      for (float v : l) acc += v;
-      loss_out[it] = (float)(acc / n);
-    }
+    HIP_TRY(launch_mlp_train_step(train_args(h, (int)n, dX, dy, dt, n_part, dpart, nullptr, dloss + it), ad, h->stream));
   }
+  if (loss_out)
+    HIP_TRY(hipMemcpyAsync(loss_out, dloss, sizeof(float) * n_steps, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(launch_mlp_publish(h->d_mlp_params, h->d_mlp, h->n_env, h->mlp_eps, h->stream));
   HIP_TRY(hipStreamSynchronize(h->stream));
   return CLEXMC_OK;

@@ -110,16 +110,15 @@ struct TrainArgs {
   const float *y;          // [n]
   const float *t;          // [n] logit scale of each sample (nullptr: 1)
   const float *W1, *b1, *W2, *b2;   // views into the FP32 parameter vector
-  float *H;                // [kHidden][n] pre-activations
-  float *dl;               // [n]
-  float *loss;             // [n]
-  float *grad;             // [n_params]
+  int n_part;              // blocks of the step, each leaving its sums in part
+  double *part;            // [n_part][n_params + 1] gradient sums and the loss sum
+  float *grad;             // [n_params] mean gradient (nullptr: not wanted)
+  float *loss;             // mean loss (nullptr: not wanted)
 };
 
+// Adam update applied by the step's reduction (p == nullptr: none)
 struct AdamArgs {
-  int n_params;
   float *p, *m, *v;
-  const float *grad;
   float lr, b1m, b2m, b1t, b2t;  // b1t = b1m^t, b2t = b2m^t
 };
 
@@ -166,8 +165,9 @@ hipError_t launch_lds_probe(int mode, int iters, int blocks, unsigned *sink, hip
 hipError_t launch_wave_pick(int n_rows, const float *v, const float *u, float *scan_out, int *pick_out,
                             hipStream_t st);
 hipError_t launch_mlp_collect(const CollectArgs &a, int n_chains, hipStream_t st);
-hipError_t launch_mlp_train_step(const TrainArgs &a, hipStream_t st);
-hipError_t launch_mlp_adam(const AdamArgs &a, hipStream_t st);
+int mlp_train_parts(int n, int n_cu);
+size_t mlp_part_bytes();
+hipError_t launch_mlp_train_step(const TrainArgs &a, const AdamArgs &ad, hipStream_t st);
 hipError_t launch_mlp_publish(const float *p, MlpDev *m, int n_env, float eps, hipStream_t st);
 
 hipError_t launch_metropolis(const RunArgs &args, bool binary, int kind, bool packed, int n_chains, int threads,
