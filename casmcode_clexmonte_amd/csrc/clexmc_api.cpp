@@ -65,6 +65,9 @@ struct clexmc_handle {
   std::vector<int> entry_home;  // home sublattice of each entry
   std::vector<double> eci;
   int halo = 0;
+  // correlations: elements of the largest orbit, largest site offset of an
+  // element, decorations of an orbit (largest) and of all orbits
+  int max_elem = 1, elem_reach = 0, max_ntau = 1, n_bins = 0;
   DevSystem dsys{};
   DevSystem *d_sys = nullptr;
   std::vector<void *> sys_allocs;
@@ -345,9 +348,28 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
     HIP_TRY(hipStreamSynchronize(h->stream));
   }
   // correlations
-  std::vector<int> func_orbit(s->n_corr, 0);
-  for (int a = 0; a < s->n_orbits; ++a)
-    for (int f = 0; f < s->orbit_nfunc[a]; ++f) func_orbit[s->orbit_func_begin[a] + f] = a;
+  std::vector<int> ntau(s->n_orbits, 1), bin0(s->n_orbits, 0);
+  long long n_bins = 0;
+  for (int a = 0; a < s->n_orbits; ++a) {
+    const int k = s->orbit_k[a], ne = s->corr_orbit_begin[a + 1] - s->corr_orbit_begin[a];
+    h->max_elem = std::max(h->max_elem, ne);
+    for (int e = 0; e < ne; ++e) {
+      long long n = 1;
+      for (int q = 0; q < k; ++q) {
+        const int *es = s->corr_elem_sites + 4 * (size_t)(s->corr_elem_begin[a] + e * k + q);
+        ARG_CHECK(es[0] >= 0 && es[0] < s->n_sublat, "orbit element sublattice out of range");
+        n *= s->n_occ[es[0]];
+        for (int c = 1; c < 4; ++c) h->elem_reach = std::max(h->elem_reach, std::abs(es[c]));
+        ARG_CHECK(n < (1ll << 28), "orbit with too many decorations");
+      }
+      ntau[a] = std::max(ntau[a], (int)n);
+    }
+    bin0[a] = (int)n_bins;
+    n_bins += ntau[a];
+    ARG_CHECK(n_bins < (1ll << 30), "too many cluster decorations");
+    h->max_ntau = std::max(h->max_ntau, ntau[a]);
+  }
+  h->n_bins = (int)n_bins;
   HIP_TRY(upload(h, A, s->orbit_k, (size_t)s->n_orbits, (int **)&d.orbit_k_all));
   HIP_TRY(upload(h, A, s->orbit_mult, (size_t)s->n_orbits, (int **)&d.orbit_mult));
   HIP_TRY(upload(h, A, s->orbit_nfunc, (size_t)s->n_orbits, (int **)&d.orbit_nfunc));
@@ -357,7 +379,8 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
   HIP_TRY(upload(h, A, (const int4 *)s->corr_elem_sites, (size_t)s->n_corr_elem_sites, (int4 **)&d.corr_elem_sites));
   HIP_TRY(upload(h, A, s->orbit_table_offset, (size_t)s->n_orbits, (int **)&d.orbit_table_offset));
   HIP_TRY(upload(h, A, s->orbit_tables, (size_t)s->n_orbit_tables, (double **)&d.orbit_tables));
-  HIP_TRY(upload(h, A, func_orbit.data(), func_orbit.size(), (int **)&d.func_orbit));
+  HIP_TRY(upload(h, A, ntau.data(), ntau.size(), (int **)&d.orbit_ntau));
+  HIP_TRY(upload(h, A, bin0.data(), bin0.size(), (int **)&d.orbit_bin0));
   HIP_TRY(upload(h, A, &h->dsys, 1, &h->d_sys));
   return CLEXMC_OK;
 }
@@ -1191,8 +1214,9 @@ clexmc_status clexmc_load_chains(clexmc_handle *h, int n_chains, const int *supe
 }
 
 static clexmc_status run_corr(clexmc_handle *h, int chain0, int n, double *out_host) {
-  double *d_out = nullptr;
-  HIP_TRY(hipMalloc(&d_out, sizeof(double) * h->n_corr * (size_t)n));
+  long long max_cells = 1;
+  for (int c = chain0; c < chain0 + n; ++c)
+    max_cells = std::max<long long>(max_cells, h->scs[h->chain_sc[c]].dev.n_cells);
   CorrArgs a;
   a.sys = h->d_sys;
   a.scs = h->d_scs;
@@ -1200,12 +1224,23 @@ static clexmc_status run_corr(clexmc_handle *h, int chain0, int n, double *out_h
   a.occ = h->d_occ;
   a.chain0 = chain0;
   a.n_corr = h->n_corr;
-  a.out = d_out;
-  hipError_t e = launch_corr(a, h->n_corr, n, h->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(out_host, d_out, sizeof(double) * h->n_corr * (size_t)n, hipMemcpyDeviceToHost, h->stream);
+  a.n_bins = h->n_bins;
+  a.elem_reach = h->elem_reach;
+  a.direct = corr_direct(max_cells, h->max_elem, h->max_ntau) ? 1 : 0;
+  a.cells_per_block = a.direct ? (int)max_cells
+                               : corr_cells_per_block(max_cells, h->max_elem, h->n_orbits, n, h->n_cu);
+  DevBufs B;
+  const size_t out_bytes = sizeof(double) * h->n_corr * (size_t)n;
+  const size_t hist_bytes = a.direct ? 0 : sizeof(unsigned long long) * h->n_bins * (size_t)n;
+  unsigned char *buf;
+  HIP_TRY(B.alloc(&buf, out_bytes + hist_bytes));
+  a.out = (double *)buf;
+  a.hist = a.direct ? nullptr : (unsigned long long *)(buf + out_bytes);
+  // (also the correlations: functions of an orbit without clusters stay 0)
+  hipError_t e = hipMemsetAsync(buf, 0, out_bytes + hist_bytes, h->stream);
+  if (e == hipSuccess) e = launch_corr(a, max_cells, h->n_orbits, n, h->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(out_host, a.out, out_bytes, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  hipFree(d_out);
   if (e != hipSuccess) {
     h->err = std::string("correlations: ") + hipGetErrorString(e);
     return CLEXMC_ERR_HIP;

@@ -108,7 +108,8 @@ struct DevSystem {
   const int4 *corr_elem_sites;
   const int *orbit_table_offset;
   const double *orbit_tables;
-  const int *func_orbit;        // [n_corr] orbit of each function
+  const int *orbit_ntau;        // [n_orbits] decorations of an orbit's cluster
+  const int *orbit_bin0;        // [n_orbits] first decoration counter of each orbit
 };
 
 // Binary site program of one sublattice (per supercell).

@@ -78,9 +78,14 @@ struct CorrArgs {
   const DevSupercell *scs;
   const ChainParams *params;
   const int8_t *occ;
-  int chain0;            // first chain; blockIdx.y selects chain0 + y
+  int chain0;            // first chain of the launch
   int n_corr;
   double *out;           // [n_chains][n_corr]
+  int n_bins;            // decoration counters per chain, all orbits
+  unsigned long long *hist;  // [n_chains][n_bins], zero before the launch (direct: not used)
+  int cells_per_block;
+  int direct;            // every chain's cells in one block per orbit
+  int elem_reach;        // largest cell offset of an orbit element's site
 };
 
 struct LearnArgs {
@@ -174,7 +179,9 @@ hipError_t launch_metropolis(const RunArgs &args, bool binary, int kind, bool pa
                              size_t lds, hipStream_t st, bool launch);
 hipError_t launch_slab_post(const RunArgs &a, int n_chains, hipStream_t st);
 hipError_t launch_delta_batch(const DeltaArgs &a, hipStream_t st);
-hipError_t launch_corr(const CorrArgs &a, int n_corr, int n_chains, hipStream_t st);
+bool corr_direct(long long max_cells, int max_elem, int max_ntau);
+int corr_cells_per_block(long long max_cells, int max_elem, int n_orbits, int n_chains, int n_cu);
+hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int n_chains, hipStream_t st);
 hipError_t launch_philox(int n, const uint4 *ctr, const uint2 *key, uint4 *out, hipStream_t st);
 size_t metropolis_lds_bytes(int pad_sites, int n_tab, bool binary, int n_func_max, int max_class, bool packed);
 hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st);

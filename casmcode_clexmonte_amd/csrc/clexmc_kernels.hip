@@ -15,11 +15,13 @@
 //                      uniforms; lane accumulators are reduced per wavefront
 //                      with cross-lane shuffles.
 //  delta_batch_kernel  per-proposal dE (BaseMontePotential::occ_delta_per_supercell)
-//  corr_kernel         full per-supercell correlations in FP64
+//  corr_count_kernel   decoration counts per orbit and
+//  corr_finish_kernel  full per-supercell correlations in FP64 from them
 //  philox_kernel       device Philox for known-answer checks
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -98,49 +100,143 @@ __global__ void delta_batch_kernel(DeltaArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Full correlations: one block per (function, chain), FP64 deterministic
-// reduction
+// Full correlations.  An orbit's functions depend on its clusters only through
+// how often each decoration tau occurs: corr_f = sum_tau count[tau] T[tau][f]
+// / mult.  So the lattice is walked once per orbit, not once per function,
+// with exact integer counts, and the FP64 sum runs over decorations.
+//
+// corr_count_kernel: a block counts the decorations of one orbit over a range
+// of cells of one chain (grid: cell ranges x orbits x chains) in LDS, with up
+// to 16 copies of every counter (by lane) so that the few decorations of a
+// pair do not serialise the lanes.  `direct` (a chain's cells in one block):
+// it forms the correlations at once.  Else the counts go to a.hist and
+// corr_finish_kernel forms them.  Orbits with more than kCorrLdsBins
+// decorations count in global memory.  Bound by the address arithmetic of the
+// cluster sites (about 10 VALU operations per site).
+// BCC quaternary 32^3, 8 chains loaded and every correlation read one chain
+// at a time: 1.29 ms (counting 23 us per chain); one FP64 walk of the lattice
+// per function took 17.2 ms.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void corr_kernel(CorrArgs a) {
-  __shared__ double red[256];
-  const int f = blockIdx.x;
-  const int chain = a.chain0 + blockIdx.y;
-  const DevSystem *__restrict__ sys = a.sys;
+constexpr int kCorrThreads = 512;
+constexpr int kCorrLdsBins = 8192;  // counters in LDS (32 KB)
+
+// decoration counts of one orbit over the cells [c0, c1); K: sites per
+// cluster (-1: any), NEAR: every site offset is at most one period
+template <int K, bool NEAR, class ADD>
+__device__ __forceinline__ void corr_count(cptr<DevSystem> sys, const DevSupercell &sc, const int8_t *__restrict__ occ,
+                                           const int4 *elem_sites, int ne, int k_rt, int c0, int c1, ADD add) {
+  const int k = K >= 0 ? K : k_rt;
+  const int L1 = sc.L1, L2 = sc.L2, L3 = sc.L3, n_cells = sc.n_cells;
+  cptr<int4> es = cst(elem_sites);
+  for (int c = c0 + (int)threadIdx.x; c < c1; c += kCorrThreads) {
+    const int i0 = c % L1, j0 = (c / L1) % L2, k0 = c / (L1 * L2);
+#pragma unroll 2
+    for (int e = 0; e < ne; ++e) {
+      int tau = 0, mul = 1;
+#pragma unroll
+      for (int q = 0; q < k; ++q) {
+        const int bq = es[e * k + q].x, dy = es[e * k + q].y, dz = es[e * k + q].z, dw = es[e * k + q].w;
+        int ii = i0 + dy, jj = j0 + dz, kk = k0 + dw;
+        if (NEAR) {
+          ii += ii < 0 ? L1 : 0;
+          jj += jj < 0 ? L2 : 0;
+          kk += kk < 0 ? L3 : 0;
+          ii -= ii >= L1 ? L1 : 0;
+          jj -= jj >= L2 ? L2 : 0;
+          kk -= kk >= L3 ? L3 : 0;
+        } else {
+          ii %= L1;
+          jj %= L2;
+          kk %= L3;
+          ii += ii < 0 ? L1 : 0;
+          jj += jj < 0 ? L2 : 0;
+          kk += kk < 0 ? L3 : 0;
+        }
+        tau += occ[bq * n_cells + ii + L1 * (jj + L2 * kk)] * mul;
+        mul *= sys->n_occ[bq];
+      }
+      add(tau);
+    }
+  }
+}
+
+__global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
+  __shared__ unsigned bins[kCorrLdsBins];
+  const int tid = threadIdx.x;
+  const int orb = blockIdx.y;
+  const int chain = a.chain0 + blockIdx.z;
+  cptr<DevSystem> sys = cst(a.sys);
   const ChainParams &cp = a.params[chain];
   const DevSupercell &sc = a.scs[cp.sc];
   const int8_t *__restrict__ occ = a.occ + cp.occ_offset;
-  const int orb = sys->func_orbit[f];
-  const int k = sys->orbit_k_all[orb];
   const int nf = sys->orbit_nfunc[orb];
-  const int fl = f - sys->orbit_func_begin[orb];
-  const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
+  const int c0 = (int)blockIdx.x * a.cells_per_block;
+  if (nf <= 0 || c0 >= sc.n_cells) return;
+  const int c1 = min(c0 + a.cells_per_block, sc.n_cells);
+  const int k = sys->orbit_k_all[orb];
   const int ne = sys->corr_orbit_begin[orb + 1] - sys->corr_orbit_begin[orb];
   const int4 *es = sys->corr_elem_sites + sys->corr_elem_begin[orb];
-  const long long total = (long long)ne * sc.n_cells;
-  double acc = 0.0;
-  for (long long w = threadIdx.x; w < total; w += blockDim.x) {
-    const int e = (int)(w / sc.n_cells);
-    const int c = (int)(w - (long long)e * sc.n_cells);
-    const int i0 = c % sc.L1, j0 = (c / sc.L1) % sc.L2, k0 = c / (sc.L1 * sc.L2);
-    int tau = 0, mul = 1;
-    for (int q = 0; q < k; ++q) {
-      const int4 d = es[e * k + q];
-      int ii = (i0 + d.y) % sc.L1, jj = (j0 + d.z) % sc.L2, kk = (k0 + d.w) % sc.L3;
-      if (ii < 0) ii += sc.L1;
-      if (jj < 0) jj += sc.L2;
-      if (kk < 0) kk += sc.L3;
-      tau += occ[d.x * sc.n_cells + ii + sc.L1 * (jj + sc.L2 * kk)] * mul;
-      mul *= sys->n_occ[d.x];
-    }
-    acc += T[tau * nf + fl];
-  }
-  red[threadIdx.x] = acc;
+  const int ntau = sys->orbit_ntau[orb];
+  const bool in_lds = ntau <= kCorrLdsBins;
+  int copies = 1;
+  while (copies < 16 && ntau * copies * 2 <= kCorrLdsBins) copies *= 2;
+  unsigned long long *hist = a.hist ? a.hist + (long long)blockIdx.z * a.n_bins + sys->orbit_bin0[orb] : nullptr;
+  if (in_lds)
+    for (int t = tid; t < ntau * copies; t += kCorrThreads) bins[t] = 0u;
   __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-    __syncthreads();
+  const bool near = a.elem_reach <= sc.L1 && a.elem_reach <= sc.L2 && a.elem_reach <= sc.L3;
+  if (in_lds) {
+    unsigned *mine = bins + (tid & (copies - 1));
+    auto add = [&](int tau) { atomicAdd(&mine[tau * copies], 1u); };
+    if (!near) corr_count<-1, false>(sys, sc, occ, es, ne, k, c0, c1, add);
+    else if (k == 1) corr_count<1, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+    else if (k == 2) corr_count<2, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+    else if (k == 3) corr_count<3, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+    else if (k == 4) corr_count<4, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+    else corr_count<-1, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+  } else {
+    auto add = [&](int tau) { atomicAdd(&hist[tau], 1ull); };
+    corr_count<-1, false>(sys, sc, occ, es, ne, k, c0, c1, add);
   }
-  if (threadIdx.x == 0) a.out[(long long)blockIdx.y * a.n_corr + f] = red[0] / (double)sys->orbit_mult[orb];
+  __syncthreads();
+  if (!in_lds) return;
+  if (a.direct) {
+    const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
+    const int f0 = sys->orbit_func_begin[orb];
+    for (int f = tid >> 6; f < nf; f += kCorrThreads / 64) {
+      double acc = 0.0;
+      for (int t = tid & 63; t < ntau; t += 64) {
+        unsigned v = 0u;
+        for (int q = 0; q < copies; ++q) v += bins[t * copies + q];
+        if (v) acc += (double)v * T[t * nf + f];
+      }
+      acc = wave_sum(acc);
+      if ((tid & 63) == 0) a.out[(long long)blockIdx.z * a.n_corr + f0 + f] = acc / (double)sys->orbit_mult[orb];
+    }
+    return;
+  }
+  for (int t = tid; t < ntau; t += kCorrThreads) {
+    unsigned v = 0u;
+    for (int q = 0; q < copies; ++q) v += bins[t * copies + q];
+    if (v) atomicAdd(&hist[t], (unsigned long long)v);
+  }
+}
+
+// correlations from the decoration counts: one block per (orbit, chain), one
+// wavefront per function
+__global__ __launch_bounds__(1024) void corr_finish_kernel(CorrArgs a) {
+  const int orb = blockIdx.x, lane = threadIdx.x & 63;
+  cptr<DevSystem> sys = cst(a.sys);
+  const int nf = sys->orbit_nfunc[orb], f0 = sys->orbit_func_begin[orb], ntau = sys->orbit_ntau[orb];
+  const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
+  const unsigned long long *hist = a.hist + (long long)blockIdx.y * a.n_bins + sys->orbit_bin0[orb];
+  for (int f = threadIdx.x >> 6; f < nf; f += 16) {
+    double acc = 0.0;
+    for (int t = lane; t < ntau; t += 64)
+      if (hist[t]) acc += (double)hist[t] * T[t * nf + f];
+    acc = wave_sum(acc);
+    if (lane == 0) a.out[(long long)blockIdx.y * a.n_corr + f0 + f] = acc / (double)sys->orbit_mult[orb];
+  }
 }
 
 __global__ void philox_kernel(int n, const uint4 *ctr, const uint2 *key, uint4 *out) {
@@ -357,9 +453,38 @@ hipError_t launch_delta_batch(const DeltaArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_corr(const CorrArgs &a, int n_corr, int n_chains, hipStream_t st) {
-  hipLaunchKernelGGL(corr_kernel, dim3(n_corr, n_chains), dim3(256), 0, st, a);
-  return hipGetLastError();
+bool corr_direct(long long max_cells, int max_elem, int max_ntau) {
+  // one block per (orbit, chain) up to 32,768 clusters: the two further
+  // launches of the split form (about 10 us) cost more than the longer loop
+  return max_cells * max_elem <= 32768 && max_ntau <= kCorrLdsBins;
+}
+
+// cells per block of the split form: about 64K clusters of the largest orbit,
+// fewer while that leaves the device short of blocks, at least one per thread
+int corr_cells_per_block(long long max_cells, int max_elem, int n_orbits, int n_chains, int n_cu) {
+  long long cells = std::max(1, 65536 / std::max(1, max_elem));
+  while (cells > kCorrThreads && (max_cells + cells - 1) / cells * n_orbits * n_chains < 4ll * n_cu) cells /= 2;
+  return (int)((cells + kCorrThreads - 1) / kCorrThreads * kCorrThreads);
+}
+
+hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int n_chains, hipStream_t st) {
+  // the grid's z extent is bounded: chains in slices
+  for (int z0 = 0; z0 < n_chains; z0 += 32768) {
+    CorrArgs s = a;
+    const int nz = std::min(32768, n_chains - z0);
+    s.chain0 = a.chain0 + z0;
+    s.out = a.out + (long long)z0 * a.n_corr;
+    if (a.hist) s.hist = a.hist + (long long)z0 * a.n_bins;
+    const unsigned gx = a.direct ? 1u : (unsigned)((max_cells + a.cells_per_block - 1) / a.cells_per_block);
+    hipLaunchKernelGGL(corr_count_kernel, dim3(gx, n_orbits, nz), dim3(kCorrThreads), 0, st, s);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && !a.direct) {
+      hipLaunchKernelGGL(corr_finish_kernel, dim3(n_orbits, nz), dim3(1024), 0, st, s);
+      e = hipGetLastError();
+    }
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_philox(int n, const uint4 *ctr, const uint2 *key, uint4 *out, hipStream_t st) {
