@@ -2829,7 +2829,9 @@ static clexmc_status collect_device(clexmc_handle *h, int n_per_chain, uint32_t 
   c.X = dX;
   c.y = dy;
   c.t = dt;
-  HIP_TRY(launch_mlp_collect(c, h->n_chains, h->stream));
+  int max_sites = 1;
+  for (int q = 0; q < h->n_chains; ++q) max_sites = std::max(max_sites, h->scs[h->chain_sc[q]].dev.n_sites);
+  HIP_TRY(launch_mlp_collect(c, h->n_chains, max_sites, h->stream));
   return CLEXMC_OK;
 }
 

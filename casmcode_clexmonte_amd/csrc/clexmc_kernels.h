@@ -169,7 +169,7 @@ hipError_t launch_metropolis_split(const RunArgs &args, int kind, bool packed, i
 hipError_t launch_lds_probe(int mode, int iters, int blocks, unsigned *sink, hipStream_t st);
 hipError_t launch_wave_pick(int n_rows, const float *v, const float *u, float *scan_out, int *pick_out,
                             hipStream_t st);
-hipError_t launch_mlp_collect(const CollectArgs &a, int n_chains, hipStream_t st);
+hipError_t launch_mlp_collect(const CollectArgs &a, int n_chains, int max_sites, hipStream_t st);
 int mlp_train_parts(int n, int n_cu);
 size_t mlp_part_bytes();
 hipError_t launch_mlp_train_step(const TrainArgs &a, const AdamArgs &ad, hipStream_t st);

@@ -715,33 +715,55 @@ hipError_t launch_wave_pick(int n_rows, const float *v, const float *u, float *s
 // and the chain's logit scale t = beta * kMlpEnergyUnit.
 // ---------------------------------------------------------------------------
 // Flip energy of variable site l (binary: to the other occupant) from the
-// flower tables, including the chemical term when include_chem.
-__device__ float collect_flip_energy(const CollectArgs &a, const ChainParams &cp, const DevSupercell &sc,
-                                     const int8_t *__restrict__ occ, int l) {
-  const DevSystem *__restrict__ sys = a.sys;
-  const int b = l / sc.n_cells;
-  const int c = l - b * sc.n_cells;
-  const int i0 = c % sc.L1, j0 = (c / sc.L1) % sc.L2, k0 = c / (sc.L1 * sc.L2);
-  const int o = occ[l];
+// flower tables, including the chemical term when include_chem.  The
+// clusters of a sublattice are walked with uniform addresses (scalar loads);
+// NEAR: no cluster reaches further than one period, so a coordinate wraps by
+// two selects.
+template <bool NEAR, class OCC>
+__device__ __forceinline__ float collect_flip_energy(const CollectArgs &a, const ChainParams &cp,
+                                                     const DevSupercell &sc, OCC occ, int l) {
+  cptr<DevSystem> sys = cst(a.sys);
+  const int L1 = sc.L1, L2 = sc.L2, L3 = sc.L3, n_cells = sc.n_cells;
+  const int bl = l / n_cells;
+  const int c = l - bl * n_cells;
+  const int i0 = c % L1, j0 = (c / L1) % L2, k0 = c / (L1 * L2);
+  const int o = occ(l);
   const int nw = 1 - o;
-  float G[kMaxFunc] = {0.f, 0.f, 0.f};
-  const int nf = sys->n_func[b];
-  for (int e = sys->flower_begin[b]; e < sys->flower_begin[b + 1]; ++e) {
-    int idx = 0;
-    for (int q = sys->entry_site_begin[e]; q < sys->entry_site_begin[e + 1]; ++q) {
-      const int4 d = sys->entry_sites[q];
-      int ii = (i0 + d.y) % sc.L1, jj = (j0 + d.z) % sc.L2, kk = (k0 + d.w) % sc.L3;
-      if (ii < 0) ii += sc.L1;
-      if (jj < 0) jj += sc.L2;
-      if (kk < 0) kk += sc.L3;
-      idx += occ[d.x * sc.n_cells + ii + sc.L1 * (jj + sc.L2 * kk)] * sys->entry_mul[q];
+  float G = 0.0f;  // binary: one site function
+  cptr<int4> es = cst(sys->entry_sites);
+  cptr<int> esb = cst(sys->entry_site_begin), mul = cst(sys->entry_mul), tb = cst(sys->entry_table),
+            fb = cst(sys->flower_begin);
+  for (int b = 0; b < sys->n_sublat; ++b) {
+    if (b != bl) continue;  // lanes of other sublattices wait
+    const int e1 = fb[b + 1];
+    int q = esb[fb[b]];
+#pragma unroll 4
+    for (int e = fb[b]; e < e1; ++e) {
+      const int q1 = esb[e + 1];
+      int idx = 0;
+      for (; q < q1; ++q) {
+        const int dx = es[q].x, dy = es[q].y, dz = es[q].z, dw = es[q].w;
+        int ii = i0 + dy, jj = j0 + dz, kk = k0 + dw;
+        if (!NEAR) {
+          ii %= L1;
+          jj %= L2;
+          kk %= L3;
+        }
+        ii += ii < 0 ? L1 : 0;
+        jj += jj < 0 ? L2 : 0;
+        kk += kk < 0 ? L3 : 0;
+        if (NEAR) {
+          ii -= ii >= L1 ? L1 : 0;
+          jj -= jj >= L2 ? L2 : 0;
+          kk -= kk >= L3 ? L3 : 0;
+        }
+        idx += occ(dx * n_cells + ii + L1 * (jj + L2 * kk)) * mul[q];
+      }
+      G += sys->flower_tables[tb[e] + idx];
     }
-    const float *V = sys->flower_tables + sys->entry_table[e] + idx * nf;
-    for (int f = 0; f < nf; ++f) G[f] += V[f];
   }
-  float dE = 0.0f;
-  for (int f = 0; f < nf; ++f) dE += (sys->site_func[b][f][nw] - sys->site_func[b][f][o]) * G[f];
-  if (a.include_chem) dE -= cp.chem[b * kMaxOcc + nw] - cp.chem[b * kMaxOcc + o];
+  float dE = (sys->site_func[bl][0][nw] - sys->site_func[bl][0][o]) * G;
+  if (a.include_chem) dE -= cp.chem[bl * kMaxOcc + nw] - cp.chem[bl * kMaxOcc + o];
   return dE;
 }
 
@@ -749,49 +771,82 @@ __device__ float collect_flip_energy(const CollectArgs &a, const ChainParams &cp
 // first, odd t the one with the largest flip probability.  Rare mobile
 // environments (the sites a weighted proposal should find) thus make up
 // about half of the training set even in well-ordered configurations.
-__global__ void mlp_collect_kernel(CollectArgs a) {
-  const int chain = blockIdx.y;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.n_per_chain) return;
-  const DevSystem *__restrict__ sys = a.sys;
+//
+// A block takes kCollectSamples samples of one chain with the chain's
+// occupation in LDS (where it fits; lds_occ): first one thread per candidate
+// (1 and 8 alternate, so a thread per sample would leave half the lanes
+// waiting), then one per sample picks, then the feature rows are written, one
+// thread per byte.  Bound by the occupation gathers.
+constexpr int kCollectThreads = 512;
+constexpr int kCollectSamples = 222;  // 9 candidates per two samples: 999 of 2 x 512 turns used
+constexpr int kCollectLdsSites = 49152;
+
+template <bool LDS>
+__global__ __launch_bounds__(kCollectThreads) void mlp_collect_kernel(CollectArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ float yc[kCollectSamples / 2 * 9];
+  __shared__ int lc[kCollectSamples / 2 * 9];
+  __shared__ int lbest[kCollectSamples];
+  const int chain = blockIdx.y, tid = threadIdx.x;
+  const int t0 = blockIdx.x * kCollectSamples;
+  const int nt = min(kCollectSamples, a.n_per_chain - t0);
+  cptr<DevSystem> sys = cst(a.sys);
   const ChainParams &cp = a.params[chain];
   const DevSupercell &sc = a.scs[cp.sc];
-  const int8_t *__restrict__ occ = a.occ + cp.occ_offset;
-  const uint4 r0 = philox4x32_10(make_uint4((uint32_t)t, a.seed, 0xC011EC7u, (uint32_t)chain), cp.key0, cp.key1);
-  const uint4 r1 = philox4x32_10(make_uint4((uint32_t)t, a.seed, 0xC011EC8u, (uint32_t)chain), cp.key0, cp.key1);
-  const uint32_t rr[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-  const int n_cand = (t & 1) ? 8 : 1;
-  int l = -1;
-  float best_y = -1.0f;
-  for (int m = 0; m < n_cand; ++m) {
-    int lc = (int)(rr[m] % (uint32_t)sc.n_sites);
-    for (int tries = 0; tries < sc.n_sites && sys->n_occ[lc / sc.n_cells] < 2; ++tries) lc = (lc + 1) % sc.n_sites;
-    const float dE = collect_flip_energy(a, cp, sc, occ, lc);
-    const float y = 1.0f / (1.0f + __expf(cp.beta * dE));
-    if (y > best_y) {
-      best_y = y;
-      l = lc;
-    }
+  const int8_t *__restrict__ occG = a.occ + cp.occ_offset;
+  const int n_sites = sc.n_sites, n_cells = sc.n_cells;
+  if (LDS) {
+    for (int l = tid; l < n_sites; l += kCollectThreads) smem[l] = (unsigned char)occG[l];
+    __syncthreads();
   }
-  const int b = l / sc.n_cells;
-  const int c = l - b * sc.n_cells;
-  const int i0 = c % sc.L1, j0 = (c / sc.L1) % sc.L2, k0 = c / (sc.L1 * sc.L2);
-  const int o = occ[l];
-  const long long out = (long long)chain * a.n_per_chain + t;
-  for (int k = 0; k < kEnvMax; ++k) {
+  auto occ = [&](int l) -> int { return LDS ? (int)smem[l] : (int)occG[l]; };
+  const bool near = sc.h <= sc.L1 && sc.h <= sc.L2 && sc.h <= sc.L3;
+  // t0 is even: candidates 9 p (sample t0 + 2 p) and 9 p + 1 .. 9 p + 8 (t0 + 2 p + 1)
+  const int n_cand = nt / 2 * 9 + (nt & 1);
+  for (int q = tid; q < n_cand; q += kCollectThreads) {
+    const int pr = q / 9, r = q - 9 * pr;
+    const int t = t0 + 2 * pr + (r > 0 ? 1 : 0), m = r > 0 ? r - 1 : 0;
+    const uint4 w = philox4x32_10(make_uint4((uint32_t)t, a.seed, m < 4 ? 0xC011EC7u : 0xC011EC8u, (uint32_t)chain),
+                                  cp.key0, cp.key1);
+    const uint32_t x = (m & 3) == 0 ? w.x : ((m & 3) == 1 ? w.y : ((m & 3) == 2 ? w.z : w.w));
+    int l = (int)(x % (uint32_t)n_sites);
+    for (int tries = 0; tries < n_sites && sys->n_occ[l / n_cells] < 2; ++tries) l = l + 1 < n_sites ? l + 1 : 0;
+    const float dE = near ? collect_flip_energy<true>(a, cp, sc, occ, l) : collect_flip_energy<false>(a, cp, sc, occ, l);
+    yc[q] = 1.0f / (1.0f + __expf(cp.beta * dE));
+    lc[q] = l;
+  }
+  __syncthreads();
+  for (int s = tid; s < nt; s += kCollectThreads) {
+    const int q0 = s / 2 * 9 + (s & 1), nc = (s & 1) ? 8 : 1;
+    int l = lc[q0];
+    float best = -1.0f;
+    for (int m = 0; m < nc; ++m)
+      if (yc[q0 + m] > best) {
+        best = yc[q0 + m];
+        l = lc[q0 + m];
+      }
+    lbest[s] = l;
+    const long long out = (long long)chain * a.n_per_chain + t0 + s;
+    a.y[out] = best;
+    a.t[out] = cp.beta * kMlpEnergyUnit;
+  }
+  __syncthreads();
+  int8_t *X = a.X + ((long long)chain * a.n_per_chain + t0) * kEnvMax;
+  for (int p = tid; p < nt * kEnvMax; p += kCollectThreads) {
+    const int s = p / kEnvMax, k = p - s * kEnvMax;
     int8_t f = 0;
     if (k < a.n_env) {
+      const int l = lbest[s], b = l / n_cells, c = l - b * n_cells;
       const int4 d = a.env_sites[b * kEnvMax + k];
-      int ii = (i0 + d.y) % sc.L1, jj = (j0 + d.z) % sc.L2, kk = (k0 + d.w) % sc.L3;
+      int ii = (c % sc.L1 + d.y) % sc.L1, jj = ((c / sc.L1) % sc.L2 + d.z) % sc.L2,
+          kk = (c / (sc.L1 * sc.L2) + d.w) % sc.L3;
       if (ii < 0) ii += sc.L1;
       if (jj < 0) jj += sc.L2;
       if (kk < 0) kk += sc.L3;
-      f = occ[d.x * sc.n_cells + ii + sc.L1 * (jj + sc.L2 * kk)] == o ? 1 : -1;
+      f = occ(d.x * n_cells + ii + sc.L1 * (jj + sc.L2 * kk)) == occ(l) ? 1 : -1;
     }
-    a.X[out * kEnvMax + k] = f;
+    X[p] = f;
   }
-  a.y[out] = best_y;
-  a.t[out] = cp.beta * kMlpEnergyUnit;
 }
 
 // ---------------------------------------------------------------------------
@@ -1032,8 +1087,14 @@ hipError_t launch_mlp_infer(const MlpDev *mlp, int n, const int8_t *X, float *ou
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_collect(const CollectArgs &a, int n_chains, hipStream_t st) {
-  hipLaunchKernelGGL(mlp_collect_kernel, dim3((a.n_per_chain + 127) / 128, n_chains), dim3(128), 0, st, a);
+hipError_t launch_mlp_collect(const CollectArgs &a, int n_chains, int max_sites, hipStream_t st) {
+  // the occupation in LDS up to 49,152 sites (with the candidates within 64 KB:
+  // two blocks per compute unit); larger chains gather from global memory
+  const dim3 blocks((a.n_per_chain + kCollectSamples - 1) / kCollectSamples, n_chains);
+  if (max_sites <= kCollectLdsSites)
+    hipLaunchKernelGGL(mlp_collect_kernel<true>, blocks, dim3(kCollectThreads), (max_sites + 15) & ~15, st, a);
+  else
+    hipLaunchKernelGGL(mlp_collect_kernel<false>, blocks, dim3(kCollectThreads), 0, st, a);
   return hipGetLastError();
 }
 
