@@ -98,6 +98,8 @@ struct clexmc_handle {
   int *d_sampN = nullptr;
   int *d_sample_count = nullptr;
   int sample_cap = 0;
+  unsigned char *d_pack = nullptr;  // clexmc_read_samples: samples of several chains side by side (<= 32 MiB)
+  size_t pack_bytes = 0;
   // upper bound of the samples any chain holds since the last load or clear
   // (kept on the host so that planning a run needs no device read)
   long long samples_bound = 0;
@@ -1096,6 +1098,9 @@ static void free_chains(clexmc_handle *h) {
   hipFree(h->d_sampN);
   hipFree(h->d_sample_count);
   hipFree(h->d_slab_rec);
+  hipFree(h->d_pack);
+  h->d_pack = nullptr;
+  h->pack_bytes = 0;
   h->d_slab_rec = nullptr;
   h->slab_rec_chains = 0;
   h->d_params = nullptr;
@@ -2605,12 +2610,46 @@ clexmc_status clexmc_read_samples(clexmc_handle *h, int *n_samples, double *E, i
   if (!E && !counts) return CLEXMC_OK;
   ARG_CHECK(want >= ns, "output arrays too small for the recorded samples");
   if (ns == 0) return CLEXMC_OK;
-  if (E)
-    HIP_TRY(hipMemcpy2D(E, sizeof(double) * ns, h->d_sampE, sizeof(double) * h->sample_cap, sizeof(double) * ns,
-                        h->n_chains, hipMemcpyDeviceToHost));
-  if (counts)
-    HIP_TRY(hipMemcpy2D(counts, sizeof(int) * kMaxOcc * ns, h->d_sampN, sizeof(int) * kMaxOcc * h->sample_cap,
-                        sizeof(int) * kMaxOcc * ns, h->n_chains, hipMemcpyDeviceToHost));
+  // chains share a contiguous copy per kPackBytes of samples; a chain with
+  // more than half of that (700,000 samples) is copied from its own row
+  static constexpr size_t kPackBytes = 32u << 20;
+  const size_t per_chain = (sizeof(double) + kMaxOcc * sizeof(int)) * (size_t)ns;
+  const int group = (int)std::min<size_t>((size_t)h->n_chains, kPackBytes / per_chain);
+  if (group <= 1) {
+    for (int c = 0; c < h->n_chains; ++c) {
+      if (E)
+        HIP_TRY(hipMemcpyAsync(E + (size_t)c * ns, h->d_sampE + (size_t)c * h->sample_cap, sizeof(double) * ns,
+                               hipMemcpyDeviceToHost, h->stream));
+      if (counts)
+        HIP_TRY(hipMemcpyAsync(counts + (size_t)c * ns * kMaxOcc, h->d_sampN + (size_t)c * h->sample_cap * kMaxOcc,
+                               sizeof(int) * kMaxOcc * ns, hipMemcpyDeviceToHost, h->stream));
+    }
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return CLEXMC_OK;
+  }
+  if (h->pack_bytes < per_chain * group) {
+    hipFree(h->d_pack);
+    h->d_pack = nullptr;
+    h->pack_bytes = 0;
+    HIP_TRY(hipMalloc(&h->d_pack, per_chain * group));
+    h->pack_bytes = per_chain * group;
+  }
+  for (int c0 = 0; c0 < h->n_chains; c0 += group) {
+    const int nc = std::min(group, h->n_chains - c0);
+    // counts first: 16-byte aligned
+    int *pN = (int *)h->d_pack;
+    double *pE = (double *)(h->d_pack + sizeof(int) * kMaxOcc * (size_t)ns * nc);
+    HIP_TRY(launch_pack_samples(h->d_sampE + (size_t)c0 * h->sample_cap,
+                                h->d_sampN + (size_t)c0 * h->sample_cap * kMaxOcc, h->sample_cap, ns, nc, pE, pN,
+                                h->stream));
+    if (E)
+      HIP_TRY(hipMemcpyAsync(E + (size_t)c0 * ns, pE, sizeof(double) * (size_t)ns * nc, hipMemcpyDeviceToHost,
+                             h->stream));
+    if (counts)
+      HIP_TRY(hipMemcpyAsync(counts + (size_t)c0 * ns * kMaxOcc, pN, sizeof(int) * kMaxOcc * (size_t)ns * nc,
+                             hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+  }
   return CLEXMC_OK;
 }
 

@@ -182,6 +182,8 @@ hipError_t launch_delta_batch(const DeltaArgs &a, hipStream_t st);
 bool corr_direct(long long max_cells, int max_elem, int max_ntau);
 int corr_cells_per_block(long long max_cells, int max_elem, int n_orbits, int n_chains, int n_cu);
 hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int n_chains, hipStream_t st);
+hipError_t launch_pack_samples(const double *E, const int *N, int cap, int n_samples, int n_chains, double *outE,
+                               int *outN, hipStream_t st);
 hipError_t launch_philox(int n, const uint4 *ctr, const uint2 *key, uint4 *out, hipStream_t st);
 size_t metropolis_lds_bytes(int pad_sites, int n_tab, bool binary, int n_func_max, int max_class, bool packed);
 hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st);

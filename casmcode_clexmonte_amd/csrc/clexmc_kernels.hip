@@ -239,6 +239,19 @@ __global__ __launch_bounds__(1024) void corr_finish_kernel(CorrArgs a) {
   }
 }
 
+// The first n samples of every chain's row of `cap` samples, rows put next to
+// each other (E, and the occupant counts as one int4 per sample; one block row
+// per chain), so that a read is one contiguous copy: the row-by-row copy it
+// replaces took 3.3 ms for 256 chains of 20 samples.  Bound by its launch.
+__global__ __launch_bounds__(256) void pack_samples_kernel(const double *E, const int4 *N, int cap, int n, double *outE,
+                                                           int4 *outN) {
+  const int s = blockIdx.x * 256 + threadIdx.x;
+  if (s >= n) return;
+  const long long src = (long long)blockIdx.y * cap + s, dst = (long long)blockIdx.y * n + s;
+  outE[dst] = E[src];
+  outN[dst] = N[src];
+}
+
 __global__ void philox_kernel(int n, const uint4 *ctr, const uint2 *key, uint4 *out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = philox4x32_10(ctr[i], key[i].x, key[i].y);
@@ -482,6 +495,20 @@ hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int
       hipLaunchKernelGGL(corr_finish_kernel, dim3(n_orbits, nz), dim3(1024), 0, st, s);
       e = hipGetLastError();
     }
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_pack_samples(const double *E, const int *N, int cap, int n_samples, int n_chains, double *outE,
+                               int *outN, hipStream_t st) {
+  static_assert(kMaxOcc == 4, "occupant counts of a sample are one int4");
+  for (int c0 = 0; c0 < n_chains; c0 += 32768) {
+    const int nc = std::min(32768, n_chains - c0);
+    hipLaunchKernelGGL(pack_samples_kernel, dim3((n_samples + 255) / 256, nc), dim3(256), 0, st, E + (size_t)c0 * cap,
+                       (const int4 *)N + (size_t)c0 * cap, cap, n_samples, outE + (size_t)c0 * n_samples,
+                       (int4 *)outN + (size_t)c0 * n_samples);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
