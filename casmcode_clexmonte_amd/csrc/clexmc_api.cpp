@@ -104,6 +104,8 @@ struct clexmc_handle {
   // (kept on the host so that planning a run needs no device read)
   long long samples_bound = 0;
   int max_lds = 0, n_cu = 0;        // device attributes, read at creation
+  unsigned char *h_stage = nullptr, *d_stage = nullptr;  // delta-energy staging (pinned host, device)
+  size_t stage_bytes = 0;
   unsigned char *noalloc = nullptr; // the device's staging array (clexmc_delta_energy_batch_noalloc)
   int block_size = 0;
   int nfold_threads = 0;  // N-fold kernel block size (0: automatic)
@@ -1280,6 +1282,23 @@ static clexmc_status check_proposals(clexmc_handle *h, int n_prop, const int32_t
   return CLEXMC_OK;
 }
 
+static DeltaArgs delta_args(clexmc_handle *h, int n_prop, int sites_per_prop, int include_chem, const int *chain,
+                            const int *sites, const int *new_occ, float *dE) {
+  DeltaArgs a;
+  a.sys = h->d_sys;
+  a.scs = h->d_scs;
+  a.params = h->d_params;
+  a.occ = h->d_occ;
+  a.n_prop = n_prop;
+  a.sites_per_prop = sites_per_prop;
+  a.include_chem = include_chem;
+  a.chain = chain;
+  a.sites = sites;
+  a.new_occ = new_occ;
+  a.dE = dE;
+  return a;
+}
+
 // Copies the proposals into the device buffers given, evaluates them and
 // copies dE back (the handle's stream, synchronised before returning).
 static hipError_t delta_batch_staged(clexmc_handle *h, int n_prop, const int32_t *chain, const int32_t *sites,
@@ -1289,23 +1308,57 @@ static hipError_t delta_batch_staged(clexmc_handle *h, int n_prop, const int32_t
   hipError_t e = hipMemcpyAsync(d_chain, chain, sizeof(int) * n_prop, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(d_sites, sites, sizeof(int) * ns, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(d_new, new_occ, sizeof(int) * ns, hipMemcpyHostToDevice, h->stream);
-  if (e == hipSuccess) {
-    DeltaArgs a;
-    a.sys = h->d_sys;
-    a.scs = h->d_scs;
-    a.params = h->d_params;
-    a.occ = h->d_occ;
-    a.n_prop = n_prop;
-    a.sites_per_prop = sites_per_prop;
-    a.include_chem = include_chem;
-    a.chain = d_chain;
-    a.sites = d_sites;
-    a.new_occ = d_new;
-    a.dE = d_dE;
-    e = launch_delta_batch(a, h->stream);
-  }
+  if (e == hipSuccess)
+    e = launch_delta_batch(delta_args(h, n_prop, sites_per_prop, include_chem, d_chain, d_sites, d_new, d_dE), h->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(dE_out, d_dE, sizeof(float) * n_prop, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  return e;
+}
+
+// Staging of the delta-energy calls: pinned host memory and a device buffer of
+// the same size, grown in powers of two to at most kDeltaSlice proposals'
+// bytes (2.5 MiB each), kept until the handle goes.
+static constexpr int kDeltaSlice = 65536;
+// proposals up to which the kernel reads and writes the pinned memory itself:
+// the two copies' launches (about 10 us) cost more than its reads over the bus.
+// One proposed swap, the whole call: 226 us with four allocations, three
+// copies in and one out; 26 us so.
+static constexpr int kDeltaDirect = 256;
+static hipError_t delta_stage(clexmc_handle *h, size_t bytes) {
+  if (h->stage_bytes >= bytes) return hipSuccess;
+  size_t cap = 4096;
+  while (cap < bytes) cap *= 2;
+  (void)hipHostFree(h->h_stage);
+  (void)hipFree(h->d_stage);
+  h->h_stage = h->d_stage = nullptr;
+  h->stage_bytes = 0;
+  hipError_t e = hipHostMalloc((void **)&h->h_stage, cap, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipMalloc((void **)&h->d_stage, cap);
+  if (e == hipSuccess) h->stage_bytes = cap;
+  return e;
+}
+
+// One slice of at most kDeltaSlice proposals: packed into the pinned memory as
+// dE | chain | sites | new occupants, one copy in, one out.
+static hipError_t delta_slice(clexmc_handle *h, int n, const int32_t *chain, const int32_t *sites,
+                              const int32_t *new_occ, int m, int include_chem, float *dE_out) {
+  const size_t nb = sizeof(int) * (size_t)n, in_bytes = nb + 2 * nb * m;
+  hipError_t e = delta_stage(h, nb + in_bytes);
+  if (e != hipSuccess) return e;
+  unsigned char *hs = h->h_stage;
+  memcpy(hs + nb, chain, nb);
+  memcpy(hs + 2 * nb, sites, nb * m);
+  memcpy(hs + 2 * nb + nb * m, new_occ, nb * m);
+  const bool direct = n <= kDeltaDirect;
+  unsigned char *ds = direct ? hs : h->d_stage;
+  if (!direct) e = hipMemcpyAsync(ds + nb, hs + nb, in_bytes, hipMemcpyHostToDevice, h->stream);
+  if (e == hipSuccess)
+    e = launch_delta_batch(delta_args(h, n, m, include_chem, (int *)(ds + nb), (int *)(ds + 2 * nb),
+                                      (int *)(ds + 2 * nb + nb * m), (float *)ds),
+                           h->stream);
+  if (e == hipSuccess && !direct) e = hipMemcpyAsync(hs, ds, nb, hipMemcpyDeviceToHost, h->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) memcpy(dE_out, hs, nb);
   return e;
 }
 
@@ -1318,19 +1371,12 @@ clexmc_status clexmc_delta_energy_batch(clexmc_handle *h, int n_prop, const int3
   const clexmc_status st = check_proposals(h, n_prop, chain, sites, new_occ, sites_per_prop);
   if (st != CLEXMC_OK) return st;
   HIP_TRY(hipSetDevice(h->device));
-  const size_t ns = (size_t)n_prop * sites_per_prop;
-  int *d_chain = nullptr, *d_sites = nullptr, *d_new = nullptr;
-  float *d_dE = nullptr;
-  HIP_TRY(hipMalloc(&d_chain, sizeof(int) * n_prop));
-  HIP_TRY(hipMalloc(&d_sites, sizeof(int) * ns));
-  HIP_TRY(hipMalloc(&d_new, sizeof(int) * ns));
-  HIP_TRY(hipMalloc(&d_dE, sizeof(float) * n_prop));
-  const hipError_t e = delta_batch_staged(h, n_prop, chain, sites, new_occ, sites_per_prop, include_chem, dE_out,
-                                          d_chain, d_sites, d_new, d_dE);
-  hipFree(d_chain);
-  hipFree(d_sites);
-  hipFree(d_new);
-  hipFree(d_dE);
+  hipError_t e = hipSuccess;
+  for (int p = 0; p < n_prop && e == hipSuccess; p += std::min(kDeltaSlice, n_prop - p)) {
+    const size_t o = (size_t)p * sites_per_prop;
+    e = delta_slice(h, std::min(kDeltaSlice, n_prop - p), chain + p, sites + o, new_occ + o, sites_per_prop,
+                    include_chem, dE_out + p);
+  }
   if (e != hipSuccess) {
     h->err = std::string("delta_energy_batch: ") + hipGetErrorString(e);
     return CLEXMC_ERR_HIP;
@@ -2967,6 +3013,8 @@ void clexmc_destroy(clexmc_handle *h) {
   for (auto m : h->fused_mods) hipModuleUnload(m);
   free_all(h->sys_allocs);
   free_mswaps(h);
+  hipHostFree(h->h_stage);
+  hipFree(h->d_stage);
   if (h->d_scs) hipFree(h->d_scs);
   if (h->ev0) hipEventDestroy(h->ev0);
   if (h->ev1) hipEventDestroy(h->ev1);

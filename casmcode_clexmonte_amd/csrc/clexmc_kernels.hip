@@ -47,56 +47,81 @@ __global__ __launch_bounds__(1024) void metropolis_split_kernel(RunArgs args) {
 }
 
 // ---------------------------------------------------------------------------
-// Per-proposal dE in FP32 on unpadded occupation (periodic wrap)
+// Per-proposal dE on the unpadded occupation (periodic wrap): one wavefront
+// per proposal, one cluster of the site per lane and turn, the FP32 table
+// values times the FP32 site-function differences summed in FP64.  A proposal
+// is bound by three dependent loads (cluster, occupants, table), so clusters
+// run side by side: one swap on FCC 12^3 took @D1@, 65,536 swaps on
+// BCC 32^3 @D2@.
 // ---------------------------------------------------------------------------
-__global__ void delta_batch_kernel(DeltaArgs a) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void delta_batch_kernel(DeltaArgs a) {
+  const int p = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int lane = threadIdx.x & 63;
   if (p >= a.n_prop) return;
-  const DevSystem *__restrict__ sys = a.sys;
-  const int chain = a.chain[p];
-  const ChainParams &cp = a.params[chain];
-  const DevSupercell &sc = a.scs[cp.sc];
-  const int8_t *__restrict__ occ = a.occ + cp.occ_offset;
+  cptr<DevSystem> sys = cst(a.sys);
+  const int chain = __builtin_amdgcn_readfirstlane(a.chain[p]);
+  cptr<ChainParams> cp = cst(a.params + chain);
+  cptr<DevSupercell> sc = cst(a.scs + cp->sc);
+  const int8_t *__restrict__ occ = a.occ + cp->occ_offset;
+  const int L1 = sc->L1, L2 = sc->L2, L3 = sc->L3, n_cells = sc->n_cells;
+  const bool near = sc->h <= L1 && sc->h <= L2 && sc->h <= L3;  // a coordinate wraps by one period at most
   const int m = a.sites_per_prop;
-  const int *sites = a.sites + p * m;
-  const int *nocc = a.new_occ + p * m;
-  float dE = 0.0f;
-  for (int i = 0; i < m; ++i) {
-    const int l = sites[i];
-    const int b = l / sc.n_cells;
-    const int c = l - b * sc.n_cells;
-    const int i0 = c % sc.L1, j0 = (c / sc.L1) % sc.L2, k0 = c / (sc.L1 * sc.L2);
-    // current occupant of l (with earlier changes of this proposal applied)
-    int o = occ[l];
-    for (int j = 0; j < i; ++j)
-      if (sites[j] == l) o = nocc[j];
+  int site[kMaxSitesPerProp], nocc[kMaxSitesPerProp];
+#pragma unroll
+  for (int i = 0; i < kMaxSitesPerProp; ++i) {
+    site[i] = i < m ? __builtin_amdgcn_readfirstlane(a.sites[(long long)p * m + i]) : -1;
+    nocc[i] = i < m ? __builtin_amdgcn_readfirstlane(a.new_occ[(long long)p * m + i]) : 0;
+  }
+  double dE = 0.0;  // this lane's share
+#pragma unroll
+  for (int i = 0; i < kMaxSitesPerProp; ++i) {
+    if (i >= m) break;
+    const int l = site[i];
+    const int b = l / n_cells;
+    const int c = l - b * n_cells;
+    const int i0 = c % L1, j0 = (c / L1) % L2, k0 = c / (L1 * L2);
+    // occupant of site x with the earlier changes of this proposal applied
+    auto occ_of = [&](int x) -> int {
+      int o = occ[x];
+#pragma unroll
+      for (int j = 0; j < i; ++j) o = site[j] == x ? nocc[j] : o;
+      return o;
+    };
+    const int o = __builtin_amdgcn_readfirstlane(occ_of(l));
     const int nw = nocc[i];
     if (nw == o) continue;
-    float G[kMaxFunc] = {0.f, 0.f, 0.f};
     const int nf = sys->n_func[b];
-    for (int e = sys->flower_begin[b]; e < sys->flower_begin[b + 1]; ++e) {
+    double ds[kMaxFunc];
+#pragma unroll
+    for (int f = 0; f < kMaxFunc; ++f) ds[f] = f < nf ? (double)(sys->site_func[b][f][nw] - sys->site_func[b][f][o]) : 0.0;
+    const int e1 = sys->flower_begin[b + 1];
+    for (int e = sys->flower_begin[b] + lane; e < e1; e += 64) {
       int idx = 0;
       for (int q = sys->entry_site_begin[e]; q < sys->entry_site_begin[e + 1]; ++q) {
         const int4 d = sys->entry_sites[q];
-        int ii = (i0 + d.y) % sc.L1, jj = (j0 + d.z) % sc.L2, kk = (k0 + d.w) % sc.L3;
-        if (ii < 0) ii += sc.L1;
-        if (jj < 0) jj += sc.L2;
-        if (kk < 0) kk += sc.L3;
-        const int lq = d.x * sc.n_cells + ii + sc.L1 * (jj + sc.L2 * kk);
-        int ov = occ[lq];
-        for (int j = 0; j < i; ++j)
-          if (sites[j] == lq) ov = nocc[j];
-        idx += ov * sys->entry_mul[q];
+        int ii = i0 + d.y, jj = j0 + d.z, kk = k0 + d.w;
+        if (!near) {
+          ii %= L1;
+          jj %= L2;
+          kk %= L3;
+        }
+        ii += ii < 0 ? L1 : 0;
+        jj += jj < 0 ? L2 : 0;
+        kk += kk < 0 ? L3 : 0;
+        ii -= ii >= L1 ? L1 : 0;
+        jj -= jj >= L2 ? L2 : 0;
+        kk -= kk >= L3 ? L3 : 0;
+        idx += occ_of(d.x * n_cells + ii + L1 * (jj + L2 * kk)) * sys->entry_mul[q];
       }
       const float *V = sys->flower_tables + sys->entry_table[e] + idx * nf;
-      for (int f = 0; f < nf; ++f) G[f] += V[f];
+      dE += ds[0] * (double)V[0];
+      if (nf > 1) dE += ds[1] * (double)V[1];
+      if (nf > 2) dE += ds[2] * (double)V[2];
     }
-    float d = 0.0f;
-    for (int f = 0; f < nf; ++f) d += (sys->site_func[b][f][nw] - sys->site_func[b][f][o]) * G[f];
-    if (a.include_chem) d -= cp.chem[b * kMaxOcc + nw] - cp.chem[b * kMaxOcc + o];
-    dE += d;
+    if (a.include_chem && lane == 0) dE -= (double)(cp->chem[b * kMaxOcc + nw] - cp->chem[b * kMaxOcc + o]);
   }
-  a.dE[p] = dE;
+  dE = wave_sum(dE);
+  if (lane == 0) a.dE[p] = (float)dE;
 }
 
 // ---------------------------------------------------------------------------
@@ -460,9 +485,7 @@ hipError_t noalloc_scratch(int device, unsigned char **ptr) {
 }
 
 hipError_t launch_delta_batch(const DeltaArgs &a, hipStream_t st) {
-  const int threads = 128;
-  const int blocks = (a.n_prop + threads - 1) / threads;
-  hipLaunchKernelGGL(delta_batch_kernel, dim3(blocks), dim3(threads), 0, st, a);
+  hipLaunchKernelGGL(delta_batch_kernel, dim3((unsigned)(((long long)a.n_prop + 3) / 4)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
