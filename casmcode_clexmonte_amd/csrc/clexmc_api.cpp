@@ -1893,6 +1893,12 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
     h->err = "chain image does not fit in LDS (" + std::to_string(lds) + " > " + std::to_string(max_lds) + " bytes)";
     return CLEXMC_ERR_UNSUPPORTED;
   }
+  // canonical sweeps (plain, multiswap) keep a class's occupants side by side
+  // during its matchings where the LDS still holds them; images at the limit
+  // go on reading them through the site addresses
+  const bool sweep = !P.learned && (kind == 0 || h->n_mswaps > 0);
+  const bool class_occ = sweep && (long long)(lds + class_occ_bytes(max_class)) <= (long long)max_lds - 64;
+  if (class_occ) lds += class_occ_bytes(max_class);
   clexmc_status st = grow_samples(h, (long long)total_passes / sample_period);
   if (st != CLEXMC_OK) return st;
   // semi-grand canonical runs with multiswaps: the fixed-composition
@@ -1928,6 +1934,7 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
   a.n_orbits = h->n_orbits;
   a.n_tab = n_tab;
   a.global_swaps = h->global_swaps;
+  a.class_occ = class_occ ? 1 : 0;
   a.chain_map = nullptr;
   a.slabs = 1;
   a.slab_rec = h->d_slab_rec;
@@ -2182,6 +2189,7 @@ static bool run_fused(clexmc_handle *h, int kind, int n_passes, int sample_perio
   a.slab_rec = h->d_slab_rec;
   a.chain_map = nullptr;
   a.slabs = 1;
+  for (const RunPlan &P : plans) a.class_occ = a.class_occ && P.a.class_occ;
   std::vector<int> lens;
   if (max_slabs > 1)
     lens = slab_epochs(n_passes);

@@ -26,6 +26,7 @@ struct RunArgs {
   int n_orbits;
   int n_tab;           // general path: flower table floats staged in LDS
   int global_swaps;    // canonical: serial swaps of uniformly random site pairs per pass
+  int class_occ;       // canonical: the launch's LDS holds the class's occupants (class_occ_bytes)
   const int *chain_map; // workgroup -> chain (nullptr: workgroup i runs chain i)
   // slabs > 1: workgroup w runs slab w % slabs of chain w / slabs; it updates
   // only the sites of its slab's planes (minus a frozen band of kreach
@@ -185,6 +186,8 @@ hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int
 hipError_t launch_pack_samples(const double *E, const int *N, int cap, int n_samples, int n_chains, double *outE,
                                int *outN, hipStream_t st);
 hipError_t launch_philox(int n, const uint4 *ctr, const uint2 *key, uint4 *out, hipStream_t st);
+// further LDS of a canonical launch that keeps the occupants of a class side by side
+inline size_t class_occ_bytes(int max_class) { return (size_t)((max_class + 15) & ~15); }
 size_t metropolis_lds_bytes(int pad_sites, int n_tab, bool binary, int n_func_max, int max_class, bool packed);
 hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st);
 // nb_total: neighbour-list entries of the supercell, all sublattices

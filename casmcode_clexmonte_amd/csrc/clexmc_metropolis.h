@@ -434,6 +434,8 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
   const int nfs = BIN ? 1 : sys->n_func_max;              // field values kept per class site
   float *cF = (float *)(smem + off_b);                   // [nfs][max_class]
   int8_t *cK = (int8_t *)(cF + nfs * max_class);         // [kMaxSlots][max_class] (binary)
+  // occupants of the class in canonical matchings (args.class_occ)
+  uint8_t *cO = (uint8_t *)(cK + (BIN ? kMaxSlots * max_class : 0));  // [max_class]
 
   // ---- load the padded image (and general tables) ----
   const int8_t *__restrict__ occG = args.occ + cp->occ_offset;
@@ -626,29 +628,38 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
     }
   }
 
-  // n^2 - sum_o n_o^2 over the occupants of one independent set (block-uniform)
-  auto class_mixed = [&](const Ranges &R) -> long long {
-    const int n = R.n();
-    int cnt[kMaxOcc] = {0, 0, 0, 0};
-    for (int t = tid; t < n; t += nthr) {
-      const int o = img.get(sc->class_addr[R.at(t)]);
-#pragma unroll
-      for (int q = 0; q < kMaxOcc; ++q) cnt[q] += (o == q) ? 1 : 0;
+  // n^2 - sum_o n_o^2 over the occupants of the independent sets c0 .. c0 + 63
+  // (lane l receives set c0 + l's), and `total` their sum: one wavefront per
+  // set, 16 sets between two barriers (their values pass through redI)
+  auto class_mixed64 = [&](int c0, long long &total) -> long long {
+    long long mine = 0;
+    long long *ex = (long long *)redI;
+    for (int sub = 0; sub < 4 && c0 + 16 * sub < n_classes; ++sub) {
+      for (int i = wave; i < 16 && c0 + 16 * sub + i < n_classes; i += n_waves) {
+        const Ranges R = ranges(c0 + 16 * sub + i);
+        const int n = R.n();
+        int b0 = 0, b1 = 0, b3 = 0;  // sites whose occupant has bit 0, bit 1, both
+#pragma unroll 4
+        for (int t = lane; t < n; t += 64) {
+          const int o = img.get(sc->class_addr[R.at(t)]);
+          b0 += o & 1;
+          b1 += o >> 1;
+          b3 += o & (o >> 1);
+        }
+        const long long n3 = wave_sum(b3), n1 = wave_sum(b0) - n3, n2 = wave_sum(b1) - n3, n0 = n - n1 - n2 - n3;
+        if (lane == 0) ex[i] = (long long)n * n - (n0 * n0 + n1 * n1 + n2 * n2 + n3 * n3);
+      }
+      __syncthreads();
+      const int m = min(16, n_classes - (c0 + 16 * sub));
+      if ((lane >> 4) == sub && (lane & 15) < m) mine = ex[lane & 15];
+      for (int i = 0; i < m; ++i) total += ex[i];
+      __syncthreads();  // every lane has read redI before it is written again
     }
-#pragma unroll
-    for (int q = 0; q < kMaxOcc; ++q) {
-      const int v = wave_sum(cnt[q]);
-      if (lane == 0) redI[q * n_waves + wave] = v;
-    }
-    __syncthreads();
-    long long sq = 0;
-    for (int q = 0; q < kMaxOcc; ++q) {
-      long long m = 0;
-      for (int w = 0; w < n_waves; ++w) m += redI[q * n_waves + w];
-      sq += m * m;
-    }
-    __syncthreads();  // every lane has read redI before it is written again
-    return (long long)n * n - sq;
+    return mine;
+  };
+  auto lane_ll = [](long long x, int l) -> long long {
+    return (long long)(((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32) |
+                       (uint32_t)__builtin_amdgcn_readlane((int)x, l));
   };
 
   for (int pass = 0; pass < args.n_passes; ++pass) {
@@ -659,8 +670,26 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
       n_mut = 0;
       for (int c = 0; c < n_classes; ++c) n_mut += ranges(c).n();
     }
+    // swaps inside a set keep its occupant counts, and only the pair phases
+    // after the sweep move occupants between sets: the values taken at the
+    // start of the pass hold for its sweep (recounted past 64 sets, where a
+    // lane keeps the current 64's)
+    long long mixed = 0;
     if (KIND != 1 && auto_rounds)
-      for (int c = 0; c < n_classes; ++c) m_total += class_mixed(ranges(c));
+      for (int c = 0; c < n_classes; c += 64) {
+        const long long m = class_mixed64(c, m_total);
+        if (c == 0) mixed = m;
+      }
+    // matching offsets (block-uniform random integers; a Philox block and a
+    // 64-bit remainder, about 180 instructions), drawn one per lane for 64
+    // matchings at a time instead of one after the other in every lane.  With
+    // the set compositions above and the occupants in cO (no site addresses
+    // from global memory inside a matching), 10 passes of 128 chains of FCC
+    // 32^3, automatic rounds, took 3.9 ms before and take 2.8 ms.
+    // Lane l of rvec holds matching rbase + l, counted from the first set's
+    // first matching (fixed rounds) or within the set (automatic)
+    uint32_t rvec = 0u;
+    int rbase = -64;
     if constexpr (kCubePath) {
       if (use_cube) {
         // register-cube sweep (one sublattice, 27 residue classes, lane =
@@ -771,29 +800,40 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
       } else {
         // ---- canonical: fields of all class sites, then random matchings
         const int n = nR;
-        const int n_rounds = auto_rounds ? auto_canonical_rounds(n, class_mixed(R), n_mut, m_total) : rounds;
+        if (auto_rounds && c > 0 && (c & 63) == 0) {
+          long long unused = 0;
+          mixed = class_mixed64(c, unused);
+        }
+        const int n_rounds = auto_rounds ? auto_canonical_rounds(n, lane_ll(mixed, c & 63), n_mut, m_total) : rounds;
+        if (auto_rounds) rbase = -64;
+        const bool local = args.class_occ != 0;  // occupants of the class in cO during the matchings
+        const int pa_own = tid < n ? sc->class_addr[R.at(tid)] : 0;
         if (n_rounds > 0) {
         if constexpr (BIN && SPLIT == 2) {
           const int part = tid & 1;
           for (int t = tid >> 1; t < n; t += (nthr >> 1)) {
             const int pa = sc->class_addr[R.at(t)];
+            const int o = img.get(pa);
             int X[kMaxSlots], K[kMaxSlots];
-            FIELD::bin_x(fctx, img, b, pa, img.get(pa), part, X);
+            FIELD::bin_x(fctx, img, b, pa, o, part, X);
 #pragma unroll
             for (int a = 0; a < kMaxSlots; ++a) X[a] += pair_swap(X[a]);
             const float F = FIELD::bin_finish(fctx, b, X, K);
             if (part == 0) {
               cF[t] = F;
+              if (local) cO[t] = (uint8_t)o;
 #pragma unroll
               for (int a = 0; a < kMaxSlots; ++a) cK[a * max_class + t] = (int8_t)K[a];
             }
           }
         } else
         for (int t = tid; t < n; t += nthr) {
-          const int pa = sc->class_addr[R.at(t)];
+          const int pa = t == tid ? pa_own : sc->class_addr[R.at(t)];
+          const int o = img.get(pa);
+          if (local) cO[t] = (uint8_t)o;
           if (BIN) {
             int K[kMaxSlots];
-            cF[t] = FIELD::bin(fctx, img, b, pa, img.get(pa), K);
+            cF[t] = FIELD::bin(fctx, img, b, pa, o, K);
 #pragma unroll
             for (int a = 0; a < kMaxSlots; ++a) cK[a * max_class + t] = (int8_t)K[a];
           } else {
@@ -806,14 +846,32 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         }
         __syncthreads();
         for (int rd = 0; rd < n_rounds; ++rd) {
-          const uint32_t r = uniform_int((uint32_t)n, gpass, ((uint32_t)c << 12) | (uint32_t)rd, rchain,
-                                         cp->key0, cp->key1);
+          const int qr = auto_rounds ? rd : c * rounds + rd;
+          if (qr >= rbase + 64) {
+            rbase = qr;
+            int cl = c, rl = rd + lane, nl = n;
+            if (!auto_rounds) {
+              cl = (qr + lane) / rounds;
+              rl = qr + lane - cl * rounds;
+              nl = cl < n_classes ? ranges(cl).n() : 1;
+            }
+            rvec = uniform_int((uint32_t)nl, gpass, ((uint32_t)cl << 12) | (uint32_t)rl, rchain, cp->key0, cp->key1);
+          }
+          const int r = __builtin_amdgcn_readlane((int)rvec, qr - rbase);
           for (int p = tid; p < n; p += nthr) {
-            int q = (int)r - p;
+            int q = r - p;
             if (q < 0) q += n;
             if (p >= q) continue;  // q == p: unpaired; p > q: the partner leads
-            const int pa = sc->class_addr[R.at(p)], qa = sc->class_addr[R.at(q)];
-            const int op = img.get(pa), oq = img.get(qa);
+            int pa = 0, qa = 0, op, oq;
+            if (local) {
+              op = cO[p];
+              oq = cO[q];
+            } else {
+              pa = sc->class_addr[R.at(p)];
+              qa = sc->class_addr[R.at(q)];
+              op = img.get(pa);
+              oq = img.get(qa);
+            }
             if (op == oq) continue;
             const uint32_t u = rng.next_u32();
             float dE;
@@ -828,8 +886,13 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             const bool acc = metropolis_accept(dE, beta, u, rng);
             accAtt += 1;
             if (acc) {
-              img.set(pa, op, oq);
-              img.set(qa, oq, op);
+              if (local) {
+                cO[p] = (uint8_t)oq;
+                cO[q] = (uint8_t)op;
+              } else {
+                img.set(pa, op, oq);
+                img.set(qa, oq, op);
+              }
               accAcc += 1;
               if (BIN) {
                 const int sp = op ? -2 : 2;
@@ -839,6 +902,18 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               } else {
                 accE += (double)dE;
               }
+            }
+          }
+          __syncthreads();
+        }
+        if (local) {
+          for (int t = tid; t < n; t += nthr) {
+            const int pa = t == tid ? pa_own : sc->class_addr[R.at(t)];
+            if constexpr (PACK) {
+              const int o = img.get(pa), nw = cO[t];
+              if (o != nw) img.set(pa, o, nw);
+            } else {
+              img.set(pa, 0, cO[t]);
             }
           }
           __syncthreads();
@@ -871,9 +946,14 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         (KIND != 1 && auto_rounds && sc->n_pair_phases > 0)
             ? auto_pair_rounds(sc->class_begin[n_classes], sc->pair_begin[sc->n_pair_phases], sc->n_pair_phases)
             : 1;
+    // the phase of every round, one per lane (at most kMaxPairRounds = 64)
+    static_assert(kMaxPairRounds <= 64, "one lane per pair round");
+    uint32_t phvec = 0u;
+    if (KIND != 1 && sc->n_pair_phases > 0)
+      phvec = uniform_int((uint32_t)sc->n_pair_phases, gpass, 0xFFFFFFF0u - (uint32_t)lane, (uint32_t)chain, cp->key0,
+                          cp->key1);
     for (int pr = 0; KIND != 1 && sc->n_pair_phases > 0 && pr < n_pair_rounds; ++pr) {
-      const uint32_t ph = uniform_int((uint32_t)sc->n_pair_phases, gpass, 0xFFFFFFF0u - (uint32_t)pr,
-                                      (uint32_t)chain, cp->key0, cp->key1);
+      const uint32_t ph = (uint32_t)__builtin_amdgcn_readlane((int)phvec, pr);
       const int pb = sc->pair_begin[ph], pe = sc->pair_begin[ph + 1];
       for (int t = pb + tid; t < pe; t += nthr) {
         const int2 pq = sc->pair_addr[t];
