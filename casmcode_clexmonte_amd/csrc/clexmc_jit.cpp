@@ -1,6 +1,8 @@
 // Run-time specialisation of the binary Metropolis kernel (see clexmc_jit.h).
 #include "clexmc_jit.h"
 
+#include "clexmc_kernels.h"
+
 #include <hip/hiprtc.h>
 
 #include <algorithm>
@@ -438,7 +440,7 @@ std::string jit_source(int n_sublat, const std::vector<int> &variable, bool bina
       << kJitCubeName << "(clexmc::RunArgs a) { clexmc::metropolis_body<true, 1, false, clexmc::JitField, 1, true>"
       << "(a, clexmc::BlockRole{(int)blockIdx.x, a.chain_map, a.slabs}); }\n";
   if (with_nfold)
-    o << "extern \"C\" __global__ __launch_bounds__(256) void " << kJitNfoldName
+    o << "extern \"C\" __global__ __launch_bounds__(" << kNfoldMaxThreads << ") void " << kJitNfoldName
       << "(clexmc::NfoldArgs na) { clexmc::nfold_body<" << (binary ? "true" : "false")
       << ", clexmc::JitField>(na); }\n";
   return o.str();

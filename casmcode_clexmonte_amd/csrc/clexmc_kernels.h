@@ -137,6 +137,11 @@ struct AdamArgs {
 constexpr int kNfoldBlockSums = 21;
 // LDS bytes of the N-fold kernel's neighbour-list starts ([kMaxSublat + 1] ints)
 constexpr int kNfoldNbBeginBytes = ((kMaxSublat + 1) * 4 + 15) & ~15;
+// threads of the largest N-fold block: 256 that make the events and a
+// wavefront that keeps the books
+constexpr int kNfoldMaxThreads = 256 + 64;
+// LDS bytes of the current event's record (16 words and the total rate)
+constexpr int kNfoldSelBytes = 16 * 4 + 16;
 struct NfoldArgs {
   RunArgs a;               // system, supercells, chain params / state, occupations, exact counts
   int n_events;            // events per chain in this launch
@@ -191,7 +196,7 @@ inline size_t class_occ_bytes(int max_class) { return (size_t)((max_class + 15) 
 size_t metropolis_lds_bytes(int pad_sites, int n_tab, bool binary, int n_func_max, int max_class, bool packed);
 hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st);
 // nb_total: neighbour-list entries of the supercell, all sublattices
-size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total);
+size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total, int n_sublat);
 
 #endif  // __HIPCC_RTC__
 

@@ -17,15 +17,17 @@
 //    finds the group by a scan over per-lane chunks of group sums, then the
 //    site by a scan of the group's 64 rates (FP64 wavefront scans), so a rate
 //    is drawn in proportion to its value however small it is next to R;
-//  * the current state is weighted by its expected residence time
-//    w = n_mutable / R in Metropolis steps (the jump chain visits states in
-//    proportion to pi(x) R(x); weights 1/R recover pi);
-//  * one lane applies the change (the new occupant drawn in proportion to
-//    its rate; binary: exact integer cluster counts, general: FP64 energy;
-//    every periodic copy of the site), then the lanes recompute the rates of
-//    the site and of its interaction neighbours (each neighbour once), and
-//    the sum of every group holding one of them is formed again from its 64
-//    rates.  Group sums are never updated by differences, so they carry no
+//  * wavefront 0 applies the change (the new occupant drawn in proportion to
+//    its rate; every periodic copy of the site, one per lane), then the lanes
+//    recompute the rates of the site and of its interaction neighbours (each
+//    neighbour once), and the sum of every group holding one of them is
+//    formed again from its 64 rates, four lanes per group;
+//  * meanwhile one lane of the last wavefront weights the state the event
+//    leaves by its expected residence time w = n_mutable / R in Metropolis
+//    steps (the jump chain visits states in proportion to pi(x) R(x); weights
+//    1/R recover pi) and keeps the counts (binary: exact integer cluster
+//    counts, general: FP64 energy).
+//    Group sums are never updated by differences, so they carry no
 //    cancellation error when rates of very different size come and go;
 //  * if R falls below 1e-30 (every rate of the chain within a few decades of
 //    FP32 underflow, beta dE > ~69 for all changes) the chain stops and
@@ -87,22 +89,33 @@ __device__ __forceinline__ double u01_53(uint32_t a, uint32_t b) {
   return ((double)(a >> 5) * 67108864.0 + (double)(b >> 6)) * (1.0 / 9007199254740992.0);
 }
 
-// sum of the 64 FP32 rates of a group in FP64, in a fixed order (four
-// interleaved partial sums of 16), so every lane that forms it gets the same
-// value
-__device__ __forceinline__ double group_rate_sum(const float *rate, int g) {
-  const float4 *r4 = (const float4 *)(rate + (size_t)g * 64);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const float4 v = r4[q];
-    a0 += (double)v.x;
-    a1 += (double)v.y;
-    a2 += (double)v.z;
-    a3 += (double)v.w;
-  }
-  return (a0 + a1) + (a2 + a3);
+// Place of site l's rate: its group's 64 rates stay together, but the 16
+// blocks of four are permuted by the group number, so that lanes that walk
+// different groups in step read different LDS banks (with plain rows every
+// group's block q lies in the same four banks: 860 conflict cycles per event)
+__device__ __forceinline__ int rate_at(int l) {
+  return (l & ~63) | ((((l >> 2) ^ (l >> 6)) & 15) << 2) | (l & 3);
 }
+
+// Sum of the 64 FP32 rates of group g in FP64: lane q of a quad adds the rates
+// 4 p + q, p = 0..15, then (q0 + q1) + (q2 + q3) over the quad (DPP), so the
+// order is fixed and every lane of the quad has the sum.  All four lanes must
+// be active.
+__device__ __forceinline__ double group_rate_sum(const float *rate, int g, int q) {
+  const float *r = rate + g * 64 + q;
+  double a = 0.0;
+#pragma unroll
+  for (int p = 0; p < 16; ++p) a += (double)r[(p ^ (g & 15)) << 2];
+  a += dpp_d<0xB1, 0xf>(a);
+  return a + dpp_d<0x4E, 0xf>(a);
+}
+
+// x / d for 0 <= x < 2^18 and 1 <= d < 2^14 or d > x, by one high product (on
+// the scalar unit for a uniform x): m = floor(2^32 / d) + 1 exceeds 2^32 / d
+// by at most 1, so x m / 2^32 exceeds x / d by less than 2^-14 < 1 / d (and
+// by less than 2^-14 below 1 for d > x); d = 1 has m = 0
+__device__ __forceinline__ uint32_t div_magic(int d) { return d > 1 ? (uint32_t)(4294967296ull / (uint32_t)d) + 1u : 0u; }
+__device__ __forceinline__ int div_small(int x, uint32_t m) { return m ? (int)__umulhi((uint32_t)x, m) : x; }
 
 // smallest total rate a chain may reach before it stops with an error
 constexpr double kNfoldMinTotalRate = 1e-30;
@@ -115,7 +128,7 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_waves = nthr >> 6;
   cptr<DevSystem> sys = cst(args.sys);
   cptr<ChainParams> cp = cst(args.params + chain);
@@ -139,18 +152,24 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   off += nfold_align16((size_t)sc->nb_max * 4);
   int *affp = (int *)(smem + off);   // their padded addresses
   off += nfold_align16((size_t)sc->nb_max * 4);
+  // the event: [0] site (-2: stopped), [1], [2] random words, [3] time
+  // sampling complete, [4], [5] old and new occupant, [6] energy change (FP32,
+  // general), [8..] cluster sums of the flipped site, and the total rate
   int *sel = (int *)(smem + off);
-  off += 16;
+  double *selR = (double *)(sel + 16);
+  off += kNfoldSelBytes;
   // the interaction-neighbour offsets of every sublattice, staged once: an
   // event reads them right after its flip
   int *nbB = (int *)(smem + off);     // [n_sublat + 1] list starts
   off += kNfoldNbBeginBytes;
-  int4 *nbL = (int4 *)(smem + off);   // (sublattice, di, dj, dk) per neighbour
-  off += nfold_align16((size_t)(sc->nb_begin[sys->n_sublat]) * 16);
+  // sublattice, di, dj, dk of a neighbour, a byte each (an image that fits in
+  // LDS has a halo of at most 26 cells)
+  int *nbL = (int *)(smem + off);
+  off += nfold_align16((size_t)(sc->nb_begin[sys->n_sublat]) * 4);
   // occupant counts and chemical potentials per sublattice: the rate of a
   // neighbour reads them for its sublattice (a per-lane index)
-  int *noccL = (int *)(smem + off);           // [kMaxSublat]
-  float *chemL = (float *)(noccL + kMaxSublat);  // [kMaxSublat][kMaxOcc]
+  int *noccL = (int *)(smem + off);                 // [n_sublat]
+  float *chemL = (float *)(noccL + sys->n_sublat);  // [n_sublat][kMaxOcc]
 
   // ---- padded image, neighbour lists
   const int8_t *__restrict__ occG = args.occ + cp->occ_offset;
@@ -164,13 +183,20 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   {
     const int n_sub = sys->n_sublat;
     const int nb_tot = sc->nb_begin[n_sub];
-    for (int t = tid; t < nb_tot; t += nthr) nbL[t] = sc->nb_cell[t];
+    for (int t = tid; t < nb_tot; t += nthr) {
+      const int4 o = sc->nb_cell[t];
+      nbL[t] = (o.x & 0xff) | (o.y & 0xff) << 8 | (o.z & 0xff) << 16 | (o.w & 0xff) << 24;
+    }
     if (tid <= n_sub) nbB[tid] = sc->nb_begin[tid];
     if (tid < n_sub) noccL[tid] = sys->n_occ[tid];
     if (tid < n_sub * kMaxOcc) chemL[tid] = cp->chem[tid];
   }
   __syncthreads();
   const int P3 = S / P12;
+  auto neighbour = [&](int t) {
+    const int v = nbL[t];
+    return make_int4(v & 0xff, (int)(int8_t)(v >> 8), (int)(int8_t)(v >> 16), v >> 24);
+  };
 
   const float beta = cp->beta;
   cptr<int> bin_off = cst(sc->bin_off);
@@ -211,84 +237,68 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
     int K[kMaxSlots];
     return site_rate_at(l / n_cells, main_addr(l), K);
   };
-  for (int l = tid; l < n_groups * 64; l += nthr) rate[l] = l < n_sites ? site_rate(l) : 0.0f;
+  for (int l = tid; l < n_groups * 64; l += nthr) rate[rate_at(l)] = l < n_sites ? site_rate(l) : 0.0f;
   __syncthreads();
-  for (int g = tid; g < n_groups; g += nthr) G[g] = group_rate_sum(rate, g);
+  for (int w = tid; w < 4 * n_groups; w += nthr) {
+    const double s = group_rate_sum(rate, w >> 2, w & 3);
+    if ((w & 3) == 0) G[w >> 2] = s;
+  }
   __syncthreads();
 
-  // per-chain running quantities (lane 0 of the workgroup)
-  long long C[kMaxSlots] = {0, 0, 0, 0, 0, 0, 0, 0};  // binary: cluster-count changes per slot
-  long long cnt[kMaxOcc];
-  for (int q = 0; q < kMaxOcc; ++q) cnt[q] = cs->counts[q];
-  double E_run = cs->E;  // general: running energy
-  // residence-weighted moments of the current block (kNfoldBlockSums layout)
-  double mom[kNfoldBlockSums];
-#pragma unroll
-  for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
-  long long n_done = 0;
-  double n_mutable = 0.0;
-  for (int b = 0; b < sys->n_sublat; ++b)
-    if (sys->n_occ[b] >= 2) n_mutable += (double)n_cells;
-  // binary: the weight of each slot's orbit, read once (the energy of a
-  // state is formed at every event)
-  double wslot[kMaxSlots];
-#pragma unroll
-  for (int j = 0; j < kMaxSlots; ++j) wslot[j] = (BIN && j < n_slots) ? sys->bin_w64[sys->slot_orbit[j]] : 0.0;
-  double E0 = 0.0;  // binary: energy of the exact counts at launch
-  if (BIN) {
-    const long long *C0 = args.binC + (long long)chain * args.n_orbits;
-    for (int a = 0; a < args.n_orbits; ++a) E0 += sys->bin_w64[a] * (double)C0[a];
-  }
+  const uint32_t m1_ = div_magic(L1), m2_ = div_magic(L2), mc_ = div_magic(n_cells);
   const unsigned long long ev0 = cs->pass_base;
   // sampling by N-fold time (na.n_time_samples > 0): samples at times
   // 0, dt, 2 dt, ... (passes since the launch) of the state occupied then
   const int n_tsamp = na.n_time_samples;
-  // (the sample storage is only passed in for time sampling)
-  const int s_base = n_tsamp > 0 ? args.sample_count[chain] : 0;
-  double T_now = 0.0;
-  int n_rec = 0;
+  const bool distinct = sc->nb_distinct != 0;  // no duplicate sites: no list in LDS, no search
   if (tid == 0) sel[3] = 0;
 
-  for (int ev = 0; ev < na.n_events; ++ev) {
-    // ---- select an event (wavefront 0)
-    if (wave == 0) {
-      const int chunk = (n_groups + 63) / 64;
-      const int g0 = min(lane * chunk, n_groups), g1 = min(g0 + chunk, n_groups);
-      double ls = 0.0;
-      for (int g = g0; g < g1; ++g) ls += G[g];
-      const double incl = wave_scan_incl_d(ls);
-      const double R = lane_d(incl, 63);
-      const unsigned long long gev = ev0 + (unsigned long long)ev;
-      const uint4 r = philox4x32_10(make_uint4(0x4E464C44u, (uint32_t)gev, (uint32_t)(gev >> 32), (uint32_t)chain),
-                                    cp->key0, cp->key1);
-      const double t = u01_53(r.x, r.y) * R;
-      int site = -1;
-      const bool live = R >= kNfoldMinTotalRate;
-      const int L = live ? pick_lane(incl, ls, t) : -1;
-      if (L >= 0) {
-        const double before = lane_d(incl, L) - lane_d(ls, L);
-        const int gl0 = __builtin_amdgcn_readlane(g0, L), gl1 = __builtin_amdgcn_readlane(g1, L);
-        const double gv = (gl0 + lane < gl1) ? G[gl0 + lane] : 0.0;
-        const double gi = wave_scan_incl_d(gv);
-        const double t2 = t - before;
-        const int lg = pick_lane(gi, gv, t2);
-        if (lg >= 0) {
-          const int g = gl0 + lg;
-          const double before2 = lane_d(gi, lg) - lane_d(gv, lg);
-          const double rv = (double)rate[g * 64 + lane];
-          const double ri = wave_scan_incl_d(rv);
-          const int ls2 = pick_lane(ri, rv, t2 - before2);
-          if (ls2 >= 0) site = g * 64 + ls2;
-        }
-      }
-      if (lane == 0) {
-        // a chain whose total rate vanished (or a group sum without a
-        // positive rate, which exact group sums rule out) stops: -2
-        sel[0] = site >= 0 ? site : -2;
-        sel[1] = (int)r.z;  // the new occupant (general sites): 53-bit uniform
-        sel[2] = (int)r.w;
-        if (site >= 0) {
-          // weight of the current state: expected Metropolis steps spent in it
+  // The last wavefront keeps the books; the others make the events.  Both
+  // loops pass the same barriers per event:
+  //  A  the event is chosen (sel, selR)
+  // [T  time sampling: the state's samples are taken; sel[3] ends the run]
+  // [B  the flip and the neighbour list; not where the first wavefront, which
+  //     makes the flip, takes all rates itself: at most 64 distinct sites]
+  //  C  the rates
+  //  D  the group sums
+  // The event's record (sel[4..15]) stands until the next flip, after the next
+  // A, so the books take it in while the next event is being chosen.
+  auto list_in_first_wave = [&](int sb) { return distinct && nbB[sb + 1] - nbB[sb] <= 64; };
+  if (wave == n_waves - 1) {
+    long long C[kMaxSlots] = {0, 0, 0, 0, 0, 0, 0, 0};  // binary: cluster-count changes per slot
+    long long cnt[kMaxOcc];
+    for (int q = 0; q < kMaxOcc; ++q) cnt[q] = cs->counts[q];
+    double E_run = cs->E;  // general: running energy
+    // residence-weighted moments of the current block (kNfoldBlockSums layout)
+    double mom[kNfoldBlockSums];
+#pragma unroll
+    for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
+    long long n_done = 0;
+    double n_mutable = 0.0;
+    for (int b = 0; b < sys->n_sublat; ++b)
+      if (sys->n_occ[b] >= 2) n_mutable += (double)n_cells;
+    // binary: the weight of each slot's orbit, read once (the energy of a
+    // state is formed at every event)
+    double wslot[kMaxSlots];
+#pragma unroll
+    for (int j = 0; j < kMaxSlots; ++j) wslot[j] = (BIN && j < n_slots) ? sys->bin_w64[sys->slot_orbit[j]] : 0.0;
+    double E0 = 0.0;  // binary: energy of the exact counts at launch
+    if (BIN) {
+      const long long *C0 = args.binC + (long long)chain * args.n_orbits;
+      for (int a = 0; a < args.n_orbits; ++a) E0 += sys->bin_w64[a] * (double)C0[a];
+    }
+    // (the sample storage is only passed in for time sampling)
+    const int s_base = n_tsamp > 0 ? args.sample_count[chain] : 0;
+    double T_now = 0.0;
+    int n_rec = 0;
+    for (int ev = 0; ev < na.n_events; ++ev) {
+      __syncthreads();  // A
+      const int site = __builtin_amdgcn_readfirstlane(sel[0]);
+      if (site < 0) break;
+      // the state the event leaves, weighted by its expected Metropolis steps;
+      // in time sampling before the event is applied
+      for (int turn = 0; turn < 2; ++turn) {
+        if (lane == 0 && turn == (n_tsamp > 0 ? 0 : 1)) {
           double E = E0;
           if (BIN) {
 #pragma unroll
@@ -297,9 +307,9 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
           } else {
             E = E_run;
           }
-          const double w = n_mutable / (double)R;
-          // sampling by N-fold time: every sample time in this state's
-          // residence interval [T, T + w / n_mutable) (in passes) samples it
+          const double w = n_mutable / *selR;
+          // every sample time in this state's residence interval
+          // [T, T + w / n_mutable) (in passes) samples it
           if (n_tsamp > 0) {
             const double t1 = T_now + w / n_mutable;
             while (n_rec < n_tsamp && (double)n_rec * na.sample_dt < t1) {
@@ -325,169 +335,278 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
             for (int q = o; q < kMaxOcc; ++q, ++t) mom[7 + t] += wn * (double)cnt[q];
           }
         }
-      }
-    }
-    __syncthreads();
-    const int site = __builtin_amdgcn_readfirstlane(sel[0]);  // the same in every lane
-    if (site < 0) {
-      // uniform across the workgroup: record the stall for the host
-      if (tid == 0) cs->flags |= kChainFlagNfoldStalled;
-      break;
-    }
-    if (sel[3]) break;  // time sampling complete (uniform across the workgroup)
-
-    // ---- apply the change (one lane); binary: its cluster sums K come with
-    // its new rate below; general: the new occupant in proportion to its rate
-    int o_flip = 0;
-    if (tid == 0) {
-      const int b = site / n_cells;
-      const int pa = main_addr(site);
-      const int o = img.get(pa);
-      o_flip = o;
-      int nw = 1 - o;
-      if (!BIN) {
-        const int no = noccL[b];
-        float G[kMaxFunc];
-        FIELD::gen(fctx, img, b, pa, tab, G);
-        double rq[kMaxOcc] = {0.0, 0.0, 0.0, 0.0}, tot = 0.0;
-        for (int q = 0; q < no; ++q)
-          if (q != o) {
-            rq[q] = (double)change_rate(b, o, q, G);
-            tot += rq[q];
-          }
-        const double t = u01_53((uint32_t)sel[1], (uint32_t)sel[2]) * tot;
-        double acc = 0.0;
-        nw = -1;
-        for (int q = 0; q < no; ++q) {
-          if (q == o) continue;
-          acc += rq[q];
-          if (nw < 0 && t < acc) nw = q;
+        if (turn == 0) {
+          if (n_tsamp > 0) __syncthreads();  // T
+          if (n_tsamp > 0 && __builtin_amdgcn_readfirstlane(sel[3])) break;
+          if (!list_in_first_wave(div_small(site, mc_))) __syncthreads();  // B
         }
-        if (nw < 0) nw = (o + 1 < no) ? no - 1 : no - 2;  // rounding: the last other occupant
-        E_run += (double)general_dE(sys, b, o, nw, G);
       }
-      cnt[o] -= 1;
-      cnt[nw] += 1;
-      // the site and every periodic copy of it in the padded image: padded
-      // coordinate (i + h) + d L for every d that stays inside [0, L + 2h)
-      {
-        const int c = site - b * n_cells;
-        const int ci = c % L1, cj = (c / L1) % L2, ck = c / (L1 * L2);
-        if (h <= L1 && h <= L2 && h <= L3) {
-          // d in {0, +1 (i < h), -1 (i >= L - h)}: at most three per axis
-          const int qi[3] = {ci + h, ci + h + L1, ci + h - L1}, qj[3] = {cj + h, cj + h + L2, cj + h - L2},
-                    qk[3] = {ck + h, ck + h + L3, ck + h - L3};
-          const bool vi[3] = {true, ci < h, ci >= L1 - h}, vj[3] = {true, cj < h, cj >= L2 - h},
-                     vk[3] = {true, ck < h, ck >= L3 - h};
+      if (n_tsamp > 0 && __builtin_amdgcn_readfirstlane(sel[3])) break;  // (uniform across the workgroup)
+      __syncthreads();  // C
+      __syncthreads();  // D
+      if (lane == 0) {
+        const int o = sel[4], nw = sel[5];
+        if (BIN) {
+          const int sk = o ? -2 : 2;
 #pragma unroll
-          for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int e = 0; e < 3; ++e)
-#pragma unroll
-              for (int f = 0; f < 3; ++f)
-                if (vk[a] && vj[e] && vi[f]) img.p[b * S + qk[a] * P12 + qj[e] * P1 + qi[f]] = (uint8_t)nw;
+          for (int a = 0; a < kMaxSlots; ++a) C[a] += (long long)sk * sel[8 + a];
         } else {
-        const int m1 = (h + L1 - 1) / L1, m2 = (h + L2 - 1) / L2, m3 = (h + L3 - 1) / L3;
-        for (int dk = -m3; dk <= m3; ++dk) {
-          const int qk = ck + h + dk * L3;
-          if (qk < 0 || qk >= P3) continue;
-          for (int dj = -m2; dj <= m2; ++dj) {
-            const int qj = cj + h + dj * L2;
-            if (qj < 0 || qj >= P12 / P1) continue;
-            for (int di = -m1; di <= m1; ++di) {
-              const int qi = ci + h + di * L1;
-              if (qi < 0 || qi >= P1) continue;
-              img.p[b * S + qk * P12 + qj * P1 + qi] = (uint8_t)nw;
+          E_run += (double)__int_as_float(sel[6]);
+        }
+#pragma unroll
+        for (int q = 0; q < kMaxOcc; ++q) cnt[q] += (q == nw ? 1 : 0) - (q == o ? 1 : 0);
+        ++n_done;
+        if ((ev + 1) % na.events_per_block == 0) {
+          const int blk = (ev + 1) / na.events_per_block - 1;
+          if (blk < na.n_blocks) {
+            double *out = na.blocks + ((long long)chain * na.n_blocks + blk) * kNfoldBlockSums;
+#pragma unroll
+            for (int q = 0; q < kNfoldBlockSums; ++q) out[q] = mom[q];
+          }
+#pragma unroll
+          for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
+        }
+      }
+    }
+    if (lane == 0) {
+      if (BIN) {
+        long long *Cg = args.binC + (long long)chain * args.n_orbits;
+        for (int j = 0; j < n_slots; ++j) Cg[sys->slot_orbit[j]] += C[j];
+        double E = 0.0;
+        for (int a = 0; a < args.n_orbits; ++a) E += sys->bin_w64[a] * (double)Cg[a];
+        cs->E = E;
+      } else {
+        cs->E = E_run;
+      }
+      for (int q = 0; q < kMaxOcc; ++q) cs->counts[q] = cnt[q];
+      if (n_tsamp > 0) args.sample_count[chain] = s_base + n_rec;
+      cs->n_attempt += n_done;
+      cs->n_accept += n_done;
+      cs->pass_base = ev0 + (unsigned long long)na.n_events;
+    }
+  } else {
+    const int n_work = nthr - 64;  // threads that make the events
+    // this lane's periodic copy in a flip: shift 0, +1 or -1 period per axis
+    const int cpk = lane / 9, cpj = (lane / 3) % 3, cpi = lane % 3;
+    const bool near = h <= L1 && h <= L2 && h <= L3;  // a coordinate wraps by one period at most
+    uint4 rv = make_uint4(0u, 0u, 0u, 0u);  // wavefront 0: the random words of events ev0 + 64 m + lane
+    for (int ev = 0; ev < na.n_events; ++ev) {
+      // ---- select an event (wavefront 0)
+      int site = -1;
+      if (wave == 0) {
+        const int chunk = (n_groups + 63) / 64;
+        const int g0 = min(lane * chunk, n_groups), g1 = min(g0 + chunk, n_groups);
+        // (four group sums on their way at a time; adding 0 leaves a sum as it is)
+        double ls = 0.0, v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
+        for (int g = g0; g < g0 + chunk; g += 4) {
+          v0 = g < g1 ? G[g] : 0.0;
+          v1 = g + 1 < g1 ? G[g + 1] : 0.0;
+          v2 = g + 2 < g1 ? G[g + 2] : 0.0;
+          v3 = g + 3 < g1 ? G[g + 3] : 0.0;
+          ls += v0;
+          ls += v1;
+          ls += v2;
+          ls += v3;
+        }
+        const double incl = wave_scan_incl_d(ls);
+        const double R = lane_d(incl, 63);
+        if ((ev & 63) == 0) {
+          const unsigned long long gev = ev0 + (unsigned long long)(ev + lane);
+          rv = philox4x32_10(make_uint4(0x4E464C44u, (uint32_t)gev, (uint32_t)(gev >> 32), (uint32_t)chain), cp->key0,
+                             cp->key1);
+        }
+        const uint32_t rx = (uint32_t)__builtin_amdgcn_readlane((int)rv.x, ev & 63),
+                       ry = (uint32_t)__builtin_amdgcn_readlane((int)rv.y, ev & 63);
+        const double t = u01_53(rx, ry) * R;
+        const bool live = R >= kNfoldMinTotalRate;
+        const int L = live ? pick_lane(incl, ls, t) : -1;
+        if (L >= 0) {
+          const double before = lane_d(incl, L) - lane_d(ls, L);
+          const int gl0 = __builtin_amdgcn_readlane(g0, L), gl1 = __builtin_amdgcn_readlane(g1, L);
+          // the chunk's groups: at most four come from the registers of lane L
+          // and need the scan's first two steps only (the others add 0)
+          double gv, gi;
+          if (chunk <= 4) {
+            const double c0 = lane_d(v0, L), c1 = lane_d(v1, L), c2 = lane_d(v2, L), c3 = lane_d(v3, L);
+            gv = lane == 0 ? c0 : (lane == 1 ? c1 : (lane == 2 ? c2 : (lane == 3 ? c3 : 0.0)));
+            gi = gv + dpp_d<0x111, 0xf>(gv);
+            gi += dpp_d<0x112, 0xf>(gi);
+          } else {
+            gv = (gl0 + lane < gl1) ? G[gl0 + lane] : 0.0;
+            gi = wave_scan_incl_d(gv);
+          }
+          const double t2 = t - before;
+          const int lg = pick_lane(gi, gv, t2);
+          if (lg >= 0) {
+            const int g = gl0 + lg;
+            const double before2 = lane_d(gi, lg) - lane_d(gv, lg);
+            const double rg = (double)rate[rate_at(g * 64 + lane)];
+            const double ri = wave_scan_incl_d(rg);
+            const int ls2 = pick_lane(ri, rg, t2 - before2);
+            if (ls2 >= 0) site = g * 64 + ls2;
+          }
+        }
+        if (lane == 0) {
+          // a chain whose total rate vanished (or a group sum without a
+          // positive rate, which exact group sums rule out) stops: -2
+          sel[0] = site >= 0 ? site : -2;
+          *selR = R;
+        }
+        // the new occupant (general sites): 53-bit uniform
+        const int rz = __builtin_amdgcn_readlane((int)rv.z, ev & 63), rw = __builtin_amdgcn_readlane((int)rv.w, ev & 63);
+        if (lane == 1) sel[1] = rz;
+        if (lane == 2) sel[2] = rw;
+      }
+      __syncthreads();  // A
+      // the same in every lane (the first wavefront has it in a register)
+      if (wave != 0) site = sel[0];
+      site = __builtin_amdgcn_readfirstlane(site);
+      if (site < 0) {
+        // uniform across the workgroup: record the stall for the host
+        if (tid == 0) cs->flags |= kChainFlagNfoldStalled;
+        break;
+      }
+      if (n_tsamp > 0) {
+        __syncthreads();  // T
+        if (__builtin_amdgcn_readfirstlane(sel[3])) break;  // time sampling complete (uniform across the workgroup)
+      }
+      // ---- apply the change (first wavefront); binary: its cluster sums K come
+      // with its new rate below; general: the new occupant in proportion to its
+      // rate
+      const int sb = div_small(site, mc_), scell = site - sb * n_cells;
+      const int srow = div_small(scell, m1_);
+      const int ci = scell - srow * L1, ck = div_small(srow, m2_), cj = srow - ck * L2;
+      if (wave == 0) {
+        const int b = sb;
+        const int pa = b * S + (ck + h) * P12 + (cj + h) * P1 + (ci + h);
+        const int o = img.get(pa);
+        int nw = 1 - o;
+        if (!BIN) {
+          const int no = noccL[b];
+          float Gf[kMaxFunc];
+          FIELD::gen(fctx, img, b, pa, tab, Gf);
+          double rq[kMaxOcc] = {0.0, 0.0, 0.0, 0.0}, tot = 0.0;
+          for (int q = 0; q < no; ++q)
+            if (q != o) {
+              rq[q] = (double)change_rate(b, o, q, Gf);
+              tot += rq[q];
+            }
+          const double t = u01_53((uint32_t)sel[1], (uint32_t)sel[2]) * tot;
+          double acc = 0.0;
+          nw = -1;
+          for (int q = 0; q < no; ++q) {
+            if (q == o) continue;
+            acc += rq[q];
+            if (nw < 0 && t < acc) nw = q;
+          }
+          if (nw < 0) nw = (o + 1 < no) ? no - 1 : no - 2;  // rounding: the last other occupant
+          if (lane == 0) sel[6] = __float_as_int(general_dE(sys, b, o, nw, Gf));
+        }
+        // every lane has read the site before a copy of it is written
+        __builtin_amdgcn_wave_barrier();
+        if (lane == 0) {
+          sel[4] = o;
+          sel[5] = nw;
+        }
+        // the site and every periodic copy of it in the padded image: padded
+        // coordinate (i + h) + d L for every d that stays inside [0, L + 2h)
+        if (near) {
+          // d in {0, +1 (i < h), -1 (i >= L - h)}: at most three per axis, one
+          // combination per lane
+          const int qi = ci + h + (cpi == 1 ? L1 : (cpi == 2 ? -L1 : 0)), qj = cj + h + (cpj == 1 ? L2 : (cpj == 2 ? -L2 : 0)),
+                    qk = ck + h + (cpk == 1 ? L3 : (cpk == 2 ? -L3 : 0));
+          const bool vi = cpi == 0 || (cpi == 1 ? ci < h : ci >= L1 - h), vj = cpj == 0 || (cpj == 1 ? cj < h : cj >= L2 - h),
+                     vk = cpk == 0 || (cpk == 1 ? ck < h : ck >= L3 - h);
+          if (lane < 27 && vi && vj && vk) img.p[b * S + qk * P12 + qj * P1 + qi] = (uint8_t)nw;
+        } else if (lane == 0) {
+          const int m1 = (h + L1 - 1) / L1, m2 = (h + L2 - 1) / L2, m3 = (h + L3 - 1) / L3;
+          for (int dk = -m3; dk <= m3; ++dk) {
+            const int qk = ck + h + dk * L3;
+            if (qk < 0 || qk >= P3) continue;
+            for (int dj = -m2; dj <= m2; ++dj) {
+              const int qj = cj + h + dj * L2;
+              if (qj < 0 || qj >= P12 / P1) continue;
+              for (int di = -m1; di <= m1; ++di) {
+                const int qi = ci + h + di * L1;
+                if (qi < 0 || qi >= P1) continue;
+                img.p[b * S + qk * P12 + qj * P1 + qi] = (uint8_t)nw;
+              }
             }
           }
         }
-        }
       }
-      ++n_done;
-    }
-    // ---- rates of the site and its interaction neighbours
-    {
-      const int b = site / n_cells;
-      const int c = site - b * n_cells;
-      const int i = c % L1, j = (c / L1) % L2, k = c / (L1 * L2);
-      const int nb0 = nbB[b], nb1 = nbB[b + 1];
-      const bool distinct = sc->nb_distinct != 0;  // no duplicate sites: no list in LDS, no search
-      if (!distinct)
-        for (int t = tid; t < nb1 - nb0; t += nthr) {
-          const int4 o = nbL[nb0 + t];
-          // (neighbour offsets are within the halo width h)
-          const int it = pad_wrap(i + o.y + h, h, L1), jt = pad_wrap(j + o.z + h, h, L2), kt = pad_wrap(k + o.w + h, h, L3);
-          aff[t] = o.x * n_cells + it + L1 * (jt + L2 * kt);
-          affp[t] = o.x * S + (kt + h) * P12 + (jt + h) * P1 + (it + h);
-        }
-      __syncthreads();  // the flip (thread 0) and the list before any rate is read
-      for (int t = tid; t < nb1 - nb0; t += nthr) {
-        int lt, pt;
-        if (distinct) {
-          const int4 o = nbL[nb0 + t];
-          // (neighbour offsets are within the halo width h)
-          const int it = pad_wrap(i + o.y + h, h, L1), jt = pad_wrap(j + o.z + h, h, L2), kt = pad_wrap(k + o.w + h, h, L3);
+      // ---- rates of the site and its interaction neighbours
+      {
+        const int i = ci, j = cj, k = ck;
+        const int nb0 = nbB[sb], nb1 = nbB[sb + 1];
+        // the neighbour o of the site: linear index and padded address
+        // (neighbour offsets are within the halo width h)
+        auto place = [&](const int4 &o, int &lt, int &pt) {
+          int it = i + o.y, jt = j + o.z, kt = k + o.w;
+          if (near) {
+            it += it < 0 ? L1 : 0;
+            jt += jt < 0 ? L2 : 0;
+            kt += kt < 0 ? L3 : 0;
+            it -= it >= L1 ? L1 : 0;
+            jt -= jt >= L2 ? L2 : 0;
+            kt -= kt >= L3 ? L3 : 0;
+          } else {
+            it = pad_wrap(it + h, h, L1);
+            jt = pad_wrap(jt + h, h, L2);
+            kt = pad_wrap(kt + h, h, L3);
+          }
           lt = o.x * n_cells + it + L1 * (jt + L2 * kt);
           pt = o.x * S + (kt + h) * P12 + (jt + h) * P1 + (it + h);
-        } else {
-          lt = aff[t];
-          pt = affp[t];
-        }
-        bool dup = false;
+        };
         if (!distinct)
-          for (int q = 0; q < t; ++q) dup = dup || (aff[q] == lt);
-        if (distinct) aff[t] = lt;  // the groups to sum again below
-        if (!dup) {
-          int K[kMaxSlots];
-          rate[lt] = site_rate_at(nbL[nb0 + t].x, pt, K);
-          if (BIN && t == 0) {
-            // the flipped site itself (first in the list, lane 0): exact cluster-count change
-            const int sk = o_flip ? -2 : 2;
+          for (int t = tid; t < nb1 - nb0; t += n_work) {
+            int lt, pt;
+            place(neighbour(nb0 + t), lt, pt);
+            aff[t] = lt;
+            affp[t] = pt;
+          }
+        // the flip and the list before any rate is read (a list of at most 64
+        // distinct sites stays in the first wavefront, which made the flip)
+        if (!list_in_first_wave(sb)) __syncthreads();  // B
+        for (int t = tid; t < nb1 - nb0; t += n_work) {
+          int lt, pt;
+          if (distinct) {
+            place(neighbour(nb0 + t), lt, pt);
+          } else {
+            lt = aff[t];
+            pt = affp[t];
+          }
+          bool dup = false;
+          if (!distinct)
+            for (int q = 0; q < t; ++q) dup = dup || (aff[q] == lt);
+          if (distinct) aff[t] = lt;  // the groups to sum again below
+          if (!dup) {
+            int K[kMaxSlots];
+            rate[rate_at(lt)] = site_rate_at(nbL[nb0 + t] & 0xff, pt, K);
+            if (BIN && t == 0) {
+              // the flipped site itself (first in the list): its cluster sums
 #pragma unroll
-            for (int a = 0; a < kMaxSlots; ++a) C[a] += (long long)sk * K[a];
+              for (int a = 0; a < kMaxSlots; ++a) sel[8 + a] = K[a];
+            }
           }
         }
+        __syncthreads();  // C
+        // the groups of the changed rates, summed again from their 64 rates by
+        // four lanes each (several quads may form one group's sum: they write
+        // the same value)
+        for (int w = tid; w < 4 * (nb1 - nb0); w += n_work) {
+          const int g = aff[w >> 2] >> 6;
+          const double s = group_rate_sum(rate, g, w & 3);
+          if ((w & 3) == 0) G[g] = s;
+        }
+        __syncthreads();  // D
       }
-      __syncthreads();
-      // the groups of the changed rates, summed again from their 64 rates
-      // (several lanes may form one group's sum: they write the same value)
-      for (int t = tid; t < nb1 - nb0; t += nthr) {
-        const int g = aff[t] >> 6;
-        G[g] = group_rate_sum(rate, g);
-      }
-      __syncthreads();
-    }
-    if (tid == 0 && ((ev + 1) % na.events_per_block) == 0) {
-      const int blk = (ev + 1) / na.events_per_block - 1;
-      if (blk < na.n_blocks) {
-        double *out = na.blocks + ((long long)chain * na.n_blocks + blk) * kNfoldBlockSums;
-#pragma unroll
-        for (int q = 0; q < kNfoldBlockSums; ++q) out[q] = mom[q];
-      }
-#pragma unroll
-      for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
     }
   }
 
   // ---- write back: occupation, exact counts, energy, counters
   int8_t *occW = args.occ + cp->occ_offset;
   for (int l = tid; l < n_sites; l += nthr) occW[l] = (int8_t)img.get(main_addr(l));
-  if (tid == 0) {
-    if (BIN) {
-      long long *Cg = args.binC + (long long)chain * args.n_orbits;
-      for (int j = 0; j < n_slots; ++j) Cg[sys->slot_orbit[j]] += C[j];
-      double E = 0.0;
-      for (int a = 0; a < args.n_orbits; ++a) E += sys->bin_w64[a] * (double)Cg[a];
-      cs->E = E;
-    } else {
-      cs->E = E_run;
-    }
-    for (int q = 0; q < kMaxOcc; ++q) cs->counts[q] = cnt[q];
-    if (n_tsamp > 0) args.sample_count[chain] = s_base + n_rec;
-    cs->n_attempt += n_done;
-    cs->n_accept += n_done;
-    cs->pass_base = ev0 + (unsigned long long)na.n_events;
-  }
 }
 
 }  // namespace clexmc

@@ -7,15 +7,15 @@
 
 namespace clexmc {
 
-size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total) {
+size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total, int n_sublat) {
   const int n_groups = (n_sites + 63) / 64;
   return nfold_align16((size_t)image_bytes(pad_sites, false)) + nfold_align16((size_t)n_groups * 64 * 4) +
-         nfold_align16((size_t)n_groups * 8) + 2 * nfold_align16((size_t)nb_max * 4) + 16 + kNfoldNbBeginBytes +
-         nfold_align16((size_t)nb_total * 16) + (size_t)kMaxSublat * (1 + kMaxOcc) * 4;
+         nfold_align16((size_t)n_groups * 8) + 2 * nfold_align16((size_t)nb_max * 4) + kNfoldSelBytes +
+         kNfoldNbBeginBytes + nfold_align16((size_t)nb_total * 4) + (size_t)n_sublat * (1 + kMaxOcc) * 4;
 }
 
 template <bool BIN>
-__global__ __launch_bounds__(256) void nfold_kernel(NfoldArgs na) {
+__global__ __launch_bounds__(kNfoldMaxThreads) void nfold_kernel(NfoldArgs na) {
   nfold_body<BIN, GenericField>(na);
 }
 

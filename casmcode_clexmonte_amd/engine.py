@@ -365,8 +365,8 @@ class Engine:
         self._check(lib().clexmc_set_block_size(self.h, C.c_int(threads)), "clexmc_set_block_size")
 
     def set_nfold_block_size(self, threads: int):
-        """Threads per chain of the N-fold kernel: 64, 128, 256, or 0 (default)
-        for the smallest multiple of 64 covering the neighbour list."""
+        """Threads per chain that make the N-fold kernel's events: 64, 128,
+        256, or 0 (default) for 256."""
         self._check(lib().clexmc_set_nfold_block_size(self.h, C.c_int(threads)), "clexmc_set_nfold_block_size")
 
     def read_samples(self):

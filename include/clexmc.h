@@ -242,12 +242,11 @@ clexmc_status clexmc_last_run_ms(clexmc_handle *h, double *ms);
  * library caps the block at 512). */
 clexmc_status clexmc_set_block_size(clexmc_handle *h, int threads);
 
-/* Block size of the N-fold kernel (clexmc_nfold_run*): 64, 128 or 256
- * threads per chain, or 0 (default) for the smallest multiple of 64 that
- * covers a site's interaction-neighbour list, at most 256.  An event's
- * select and flip run in the first wavefront, its neighbours' rates one per
- * thread; more wavefronts share only the launch's image load and initial
- * rates.  Results do not depend on it.  No counterpart in the reference
+/* Threads per chain that make the N-fold kernel's events (clexmc_nfold_run*):
+ * 64, 128 or 256, or 0 (default) for 256; one more wavefront keeps the
+ * chain's books.  An event's select and flip run in the first wavefront, its
+ * neighbours' rates one per thread, the sums of the changed groups of rates
+ * four threads each.  Results do not depend on it.  No counterpart in the reference
  * (its nfold loop, include/casm/clexmonte/nfold/nfold_impl.hh:18-98, runs
  * on one CPU thread). */
 clexmc_status clexmc_set_nfold_block_size(clexmc_handle *h, int threads);
