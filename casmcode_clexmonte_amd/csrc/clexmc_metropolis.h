@@ -19,27 +19,37 @@ namespace clexmc {
 // Counter = (lane, draw_lo, draw_hi, chain); key = chain seed.
 // ---------------------------------------------------------------------------
 struct LaneRng {
-  uint4 buf;
+  uint4 buf, nxt;  // the open block and, with `ahead`, the one after it
   int left;
-  unsigned long long draw;
+  bool ahead;
+  unsigned long long draw;  // blocks opened
   uint32_t lane, chain, k0, k1;
 
-  __device__ __forceinline__ float next() {
-    if (left == 0) {
-      buf = philox4x32_10(make_uint4(lane, (uint32_t)draw, (uint32_t)(draw >> 32), chain), k0, k1);
-      ++draw;
-      left = 4;
-    }
-    --left;
-    return u01(word(left));
+  __device__ __forceinline__ uint4 block() const {
+    return philox4x32_10(make_uint4(lane, (uint32_t)draw, (uint32_t)(draw >> 32), chain), k0, k1);
   }
+  // At least `need` (<= 4) words at hand in every lane of the wavefront.
+  // Lanes that draw at different times (canonical moves draw for pairs of
+  // different occupants only) would otherwise run a Philox block for a few of
+  // them at almost every draw; here all lanes without a next block get it at
+  // once, when one of them is about to run dry.
+  __device__ __forceinline__ void prepare(int need) {
+    if (__any(left + (ahead ? 4 : 0) < need) && !ahead) {
+      nxt = block();
+      ahead = true;
+    }
+  }
+  __device__ __forceinline__ void open() {
+    if (ahead) buf = nxt;
+    else buf = block();
+    ahead = false;
+    ++draw;
+    left = 4;
+  }
+  __device__ __forceinline__ float next() { return u01(next_u32()); }
   // one 32-bit word of the stream (acceptance tests)
   __device__ __forceinline__ uint32_t next_u32() {
-    if (left == 0) {
-      buf = philox4x32_10(make_uint4(lane, (uint32_t)draw, (uint32_t)(draw >> 32), chain), k0, k1);
-      ++draw;
-      left = 4;
-    }
+    if (left == 0) open();
     --left;
     return word(left);
   }
@@ -59,6 +69,16 @@ __device__ __forceinline__ uint32_t uniform_int(uint32_t n, unsigned long long p
   uint4 r = philox4x32_10(make_uint4(0xFFFFFFFFu, (uint32_t)pass, phase, chain ^ 0x9E3779B9u), k0, k1);
   unsigned long long x = ((unsigned long long)r.x << 32) | r.y;
   return n ? (uint32_t)(x % n) : 0u;
+}
+
+// Workgroup barrier for LDS data only.  __syncthreads() also waits for every
+// global load in flight, which would end the loads of the next class's site
+// and halo copy at the first barrier of the current class; the sweep passes
+// data between lanes through LDS alone.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Sum over the 64 lanes of a full wave, returned to every lane.  Four DPP
@@ -432,10 +452,18 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
   ChainLds *cl = (ChainLds *)(smem + off_b);
   off_b += kChainLdsBytes;
   const int nfs = BIN ? 1 : sys->n_func_max;              // field values kept per class site
-  float *cF = (float *)(smem + off_b);                   // [nfs][max_class]
-  int8_t *cK = (int8_t *)(cF + nfs * max_class);         // [kMaxSlots][max_class] (binary)
+  // binary: the cluster sums of a class site, a byte per slot (one 8-byte word)
+  uint2 *cK = (uint2 *)(smem + off_b);                   // [max_class]
+  float *cF = (float *)(cK + (BIN ? max_class : 0));     // [nfs][max_class]
   // occupants of the class in canonical matchings (args.class_occ)
-  uint8_t *cO = (uint8_t *)(cK + (BIN ? kMaxSlots * max_class : 0));  // [max_class]
+  uint8_t *cO = (uint8_t *)(cF + nfs * max_class);       // [max_class]
+  static_assert(kMaxSlots == 8, "cluster sums of a site are 8 bytes");
+  auto pack_K = [](const int (&K)[kMaxSlots]) -> uint2 {
+    return make_uint2(((uint32_t)K[0] & 255u) | ((uint32_t)K[1] & 255u) << 8 | ((uint32_t)K[2] & 255u) << 16 |
+                          (uint32_t)K[3] << 24,
+                      ((uint32_t)K[4] & 255u) | ((uint32_t)K[5] & 255u) << 8 | ((uint32_t)K[6] & 255u) << 16 |
+                          (uint32_t)K[7] << 24);
+  };
 
   // ---- load the padded image (and general tables) ----
   const int8_t *__restrict__ occG = args.occ + cp->occ_offset;
@@ -521,6 +549,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
   const float beta = cp->beta;
   LaneRng rng;
   rng.left = 0;
+  rng.ahead = false;
   rng.draw = cs->draw_base;
   rng.lane = (uint32_t)tid | ((uint32_t)slab << 16);
   rng.chain = (uint32_t)chain;
@@ -570,6 +599,45 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
     const int kb = ka + U;
     if (kb <= L3) return Ranges{cb + kx[ka], kx[kb] - kx[ka], ce, 0};
     return Ranges{cb + kx[ka], kx[L3] - kx[ka], cb, kx[kb - L3]};
+  };
+  // What the sweep needs of a class, fetched ahead: its numbers (sublattice,
+  // site ranges, halo copies; scalar loads) two classes before it runs, this
+  // lane's first site and halo copy (vector loads by those numbers) one class
+  // before, so that a class starts without waiting for global memory.  After
+  // the last class comes the next pass's first.
+  // (halo copies: list positions a0 + t for t < na, then b0 + t - na; nh in all.
+  // Slabs copy their own sites only: the others are unchanged in this image.)
+  struct ClassNums {
+    int b;
+    Ranges R;
+    int a0, na, b0, nh;
+  };
+  struct ClassFirst {
+    int pa;
+    int2 hc;
+  };
+  auto class_nums = [&](int c) -> ClassNums {
+    ClassNums q;
+    q.b = sc->class_sublat[c];
+    q.R = ranges(c);
+    if (n_slabs == 1) {
+      q.a0 = sc->halo_begin[c];
+      q.na = q.nh = sc->halo_begin[c + 1] - q.a0;
+      q.b0 = 0;
+    } else {
+      q.a0 = sc->halo_site[q.R.r0];
+      q.na = sc->halo_site[q.R.r0 + q.R.n0] - q.a0;
+      q.b0 = sc->halo_site[q.R.r1];
+      q.nh = q.na + sc->halo_site[q.R.r1 + q.R.n1] - q.b0;
+    }
+    return q;
+  };
+  auto halo_at = [](const ClassNums &q, int t) -> int { return t < q.na ? q.a0 + t : q.b0 + (t - q.na); };
+  auto class_first = [&](const ClassNums &q) -> ClassFirst {
+    ClassFirst f{0, make_int2(0, 0)};
+    if (tid < q.R.n()) f.pa = sc->class_addr[q.R.at(tid)];
+    if (tid < q.nh) f.hc = sc->halo[halo_at(q, tid)];
+    return f;
   };
   // whether the site at padded main address a lies on an updated plane
   auto updated = [&](int a) -> bool {
@@ -649,11 +717,11 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         const long long n3 = wave_sum(b3), n1 = wave_sum(b0) - n3, n2 = wave_sum(b1) - n3, n0 = n - n1 - n2 - n3;
         if (lane == 0) ex[i] = (long long)n * n - (n0 * n0 + n1 * n1 + n2 * n2 + n3 * n3);
       }
-      __syncthreads();
+      lds_barrier();
       const int m = min(16, n_classes - (c0 + 16 * sub));
       if ((lane >> 4) == sub && (lane & 15) < m) mine = ex[lane & 15];
       for (int i = 0; i < m; ++i) total += ex[i];
-      __syncthreads();  // every lane has read redI before it is written again
+      lds_barrier();  // every lane has read redI before it is written again
     }
     return mine;
   };
@@ -662,6 +730,13 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
                        (uint32_t)__builtin_amdgcn_readlane((int)x, l));
   };
 
+  ClassNums nums1{}, nums2{};
+  ClassFirst first1{0, make_int2(0, 0)};
+  if (!use_cube) {
+    nums1 = class_nums(0);
+    nums2 = class_nums(n_classes > 1 ? 1 : 0);
+    first1 = class_first(nums1);
+  }
   for (int pass = 0; pass < args.n_passes; ++pass) {
     const unsigned long long gpass = pass0 + (unsigned long long)pass;
     long long m_total = 0;
@@ -719,13 +794,18 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
       }
     }
     for (int c = 0; c < n_classes && !use_cube; ++c) {
-      const int b = sc->class_sublat[c];
-      const Ranges R = ranges(c);
+      const ClassNums nums = nums1;
+      const ClassFirst first = first1;
+      nums1 = nums2;
+      first1 = class_first(nums1);
+      {
+        int c2 = c + 2;
+        while (c2 >= n_classes) c2 -= n_classes;
+        nums2 = class_nums(c2);
+      }
+      const int b = nums.b;
+      const Ranges R = nums.R;
       const int nR = R.n();
-      // this lane's first halo copy of the class, loaded before the sweep so
-      // that its global-memory latency overlaps the sweep
-      const int hb0 = sc->halo_begin[c] + tid, hb1 = n_slabs == 1 ? sc->halo_begin[c + 1] : 0;
-      const int2 hc0 = hb0 < hb1 ? sc->halo[hb0] : make_int2(0, 0);
       cptr<BinSub> bs = cst(sc->bin_sub + b);
       cptr<GenSub> gs = cst(sc->gen_sub + b);
       const float chem0 = cp->chem[b * kMaxOcc + 0], chem1 = cp->chem[b * kMaxOcc + 1];
@@ -758,7 +838,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
           }
         } else
         for (int v = tid; v < nR; v += nthr) {
-          const int pa = sc->class_addr[R.at(v)];
+          const int pa = v == tid ? first.pa : sc->class_addr[R.at(v)];
           const int o = img.get(pa);
           const uint32_t u = rng.next_u32();
           if (BIN) {
@@ -796,7 +876,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             }
           }
         }
-        __syncthreads();
+        lds_barrier();
       } else {
         // ---- canonical: fields of all class sites, then random matchings
         const int n = nR;
@@ -807,7 +887,6 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         const int n_rounds = auto_rounds ? auto_canonical_rounds(n, lane_ll(mixed, c & 63), n_mut, m_total) : rounds;
         if (auto_rounds) rbase = -64;
         const bool local = args.class_occ != 0;  // occupants of the class in cO during the matchings
-        const int pa_own = tid < n ? sc->class_addr[R.at(tid)] : 0;
         if (n_rounds > 0) {
         if constexpr (BIN && SPLIT == 2) {
           const int part = tid & 1;
@@ -822,20 +901,18 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             if (part == 0) {
               cF[t] = F;
               if (local) cO[t] = (uint8_t)o;
-#pragma unroll
-              for (int a = 0; a < kMaxSlots; ++a) cK[a * max_class + t] = (int8_t)K[a];
+              cK[t] = pack_K(K);
             }
           }
         } else
         for (int t = tid; t < n; t += nthr) {
-          const int pa = t == tid ? pa_own : sc->class_addr[R.at(t)];
+          const int pa = t == tid ? first.pa : sc->class_addr[R.at(t)];
           const int o = img.get(pa);
           if (local) cO[t] = (uint8_t)o;
           if (BIN) {
             int K[kMaxSlots];
             cF[t] = FIELD::bin(fctx, img, b, pa, o, K);
-#pragma unroll
-            for (int a = 0; a < kMaxSlots; ++a) cK[a * max_class + t] = (int8_t)K[a];
+            cK[t] = pack_K(K);
           } else {
             float G[kMaxFunc];
             FIELD::gen(fctx, img, b, pa, tabL, G);
@@ -844,7 +921,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             if (nfs > 2) cF[2 * max_class + t] = G[2];
           }
         }
-        __syncthreads();
+        lds_barrier();
         for (int rd = 0; rd < n_rounds; ++rd) {
           const int qr = auto_rounds ? rd : c * rounds + rd;
           if (qr >= rbase + 64) {
@@ -858,11 +935,16 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             rvec = uniform_int((uint32_t)nl, gpass, ((uint32_t)cl << 12) | (uint32_t)rl, rchain, cp->key0, cp->key1);
           }
           const int r = __builtin_amdgcn_readlane((int)rvec, qr - rbase);
-          for (int p = tid; p < n; p += nthr) {
+          for (int p = tid, turn = 0; p < n; p += nthr, ++turn) {
+            if ((turn & 1) == 0) rng.prepare(2);  // this turn's draw and the next one's
             int q = r - p;
             if (q < 0) q += n;
             if (p >= q) continue;  // q == p: unpaired; p > q: the partner leads
             int pa = 0, qa = 0, op, oq;
+            // everything the swap may need in one LDS round trip (with the
+            // words drawn ahead: FCC 12^3, one chain, 100 passes 8.33 ms -> 7.58 ms)
+            const float Fp0 = cF[p], Fq0 = cF[q];
+            const uint2 kp = BIN ? cK[p] : make_uint2(0u, 0u), kq = BIN ? cK[q] : make_uint2(0u, 0u);
             if (local) {
               op = cO[p];
               oq = cO[q];
@@ -877,10 +959,10 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             float dE;
             if (BIN) {
               const float dp = op ? -2.0f : 2.0f;
-              dE = dp * cF[p] - dp * cF[q];
+              dE = dp * Fp0 - dp * Fq0;
             } else {
-              float Gp[kMaxFunc] = {cF[p], nfs > 1 ? cF[max_class + p] : 0.f, nfs > 2 ? cF[2 * max_class + p] : 0.f};
-              float Gq[kMaxFunc] = {cF[q], nfs > 1 ? cF[max_class + q] : 0.f, nfs > 2 ? cF[2 * max_class + q] : 0.f};
+              float Gp[kMaxFunc] = {Fp0, nfs > 1 ? cF[max_class + p] : 0.f, nfs > 2 ? cF[2 * max_class + p] : 0.f};
+              float Gq[kMaxFunc] = {Fq0, nfs > 1 ? cF[max_class + q] : 0.f, nfs > 2 ? cF[2 * max_class + q] : 0.f};
               dE = general_dE(sys, b, op, oq, Gp) + general_dE(sys, b, oq, op, Gq);
             }
             const bool acc = metropolis_accept(dE, beta, u, rng);
@@ -897,18 +979,21 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               if (BIN) {
                 const int sp = op ? -2 : 2;
 #pragma unroll
-                for (int a = 0; a < kMaxSlots; ++a)
-                  accC[a] += __mul24(sp, (int)cK[a * max_class + p] - (int)cK[a * max_class + q]);
+                for (int a = 0; a < kMaxSlots; ++a) {
+                  const int sh = 8 * (a & 3);
+                  accC[a] += __mul24(sp, (int)(int8_t)((a < 4 ? kp.x : kp.y) >> sh) -
+                                             (int)(int8_t)((a < 4 ? kq.x : kq.y) >> sh));
+                }
               } else {
                 accE += (double)dE;
               }
             }
           }
-          __syncthreads();
+          lds_barrier();
         }
         if (local) {
           for (int t = tid; t < n; t += nthr) {
-            const int pa = t == tid ? pa_own : sc->class_addr[R.at(t)];
+            const int pa = t == tid ? first.pa : sc->class_addr[R.at(t)];
             if constexpr (PACK) {
               const int o = img.get(pa), nw = cO[t];
               if (o != nw) img.set(pa, o, nw);
@@ -916,28 +1001,17 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               img.set(pa, 0, cO[t]);
             }
           }
-          __syncthreads();
+          lds_barrier();
         }
         }  // n_rounds > 0
       }
-      // ---- halo copies of this class (slabs: of this workgroup's sites only;
-      // the other sites are unchanged in this image)
-      if (n_slabs == 1) {
-        if (hb0 < hb1) img.copy(hc0.y, hc0.x);
-        for (int t = hb0 + nthr; t < hb1; t += nthr) {
-          const int2 hc = sc->halo[t];
-          img.copy(hc.y, hc.x);
-        }
-      } else {
-        const int a0 = sc->halo_site[R.r0], a1 = sc->halo_site[R.r0 + R.n0];
-        const int b0 = sc->halo_site[R.r1], b1 = sc->halo_site[R.r1 + R.n1];
-        const int na = a1 - a0, nh = na + (b1 - b0);
-        for (int t = tid; t < nh; t += nthr) {
-          const int2 hc = sc->halo[t < na ? a0 + t : b0 + (t - na)];
-          img.copy(hc.y, hc.x);
-        }
+      // ---- halo copies of this class
+      if (tid < nums.nh) img.copy(first.hc.y, first.hc.x);
+      for (int t = tid + nthr; t < nums.nh; t += nthr) {
+        const int2 hc = sc->halo[halo_at(nums, t)];
+        img.copy(hc.y, hc.x);
       }
-      __syncthreads();
+      lds_barrier();
     }
 
     // ---- canonical cross-class mixing: randomly chosen pair phases (one per
@@ -991,12 +1065,12 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
           }
         }
       }
-      __syncthreads();
+      lds_barrier();
       for (int t = sc->pair_halo_begin[ph] + tid; t < sc->pair_halo_begin[ph + 1]; t += nthr) {
         const int2 hc = sc->pair_halo[t];
         img.copy(hc.y, hc.x);
       }
-      __syncthreads();
+      lds_barrier();
     }
 
     // ---- canonical global swaps: uniformly random site pairs anywhere in the
@@ -1053,7 +1127,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
           }
         }
       }
-      __syncthreads();
+      lds_barrier();
     }
 
     // ---- semi-grand canonical multiswaps (SemiGrandCanonicalCalculator.cc:
@@ -1168,7 +1242,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             msw[5] = n_pick;
             for (int q = 0; q < n_pick; ++q) msw[8 + q] = pick_a[q];
           }
-          __syncthreads();
+          lds_barrier();
           const int state = msw[0];
           if (state != 1) break;
           // workgroup-wide search: the k-th site (in unit order) of unit u
@@ -1194,7 +1268,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               if (lane >= o) incl += y;
             }
             if (lane == 63) redI[wave] = incl;
-            __syncthreads();
+            lds_barrier();
             int before = incl - cnt;
             for (int w = 0; w < wave; ++w) before += redI[w];
             if (kk >= before && kk < before + cnt) {
@@ -1210,7 +1284,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
                 }
               }
             }
-            __syncthreads();
+            lds_barrier();
           }
           if (tid == 0) {
             if (msw[4] < 0) {
@@ -1292,7 +1366,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             }
           }
         }
-        __syncthreads();
+        lds_barrier();
       }
     }
 
@@ -1338,7 +1412,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         if (lane == 0) redD[wave] = v;
         accE = 0.0;
       }
-      __syncthreads();
+      lds_barrier();
       if (wave == 0) {
         // lane q adds up slot q over the waves; thread 0 reads the totals
         int part = 0;
@@ -1410,7 +1484,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         }  // n_slabs == 1
       }  // lane 0
       }  // wave 0
-      __syncthreads();
+      lds_barrier();
     }
   }
 
