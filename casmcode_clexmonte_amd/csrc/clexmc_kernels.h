@@ -92,6 +92,7 @@ struct CorrArgs {
 struct LearnArgs {
   const MlpDev *mlp;
   int rounds_per_group;
+  int stream_threads;  // threads whose random streams the chain uses (set by launch_learned)
 };
 
 struct CollectArgs {

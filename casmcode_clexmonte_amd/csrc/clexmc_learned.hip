@@ -39,6 +39,7 @@
 
 #include "clexmc_device.h"
 #include "clexmc_kernels.h"
+#include "clexmc_metropolis.h"
 
 namespace clexmc {
 
@@ -49,8 +50,29 @@ __device__ __forceinline__ short bf16_of_sign(int v) {
   return v > 0 ? (short)0x3F80 : (v < 0 ? (short)0xBF80 : (short)0);
 }
 
+// Sum over a row of 16 lanes, in every lane: DPP row rotations by 8, 4, 2, 1.
+// After a rotation by 2^k every lane agrees with the one 2^k away, so the
+// sums are those of a butterfly (lane ^ 8, ^ 4, ^ 2, ^ 1), bit for bit.
+__device__ __forceinline__ float row_all_sum(float x) {
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xF, 0xF, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xF, 0xF, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xF, 0xF, false));
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xF, 0xF, false));
+  return x;
+}
+
+// lane N's value of the row of 16, in every lane of the row
+template <int N>
+__device__ __forceinline__ int row_bcast(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x150 + N, 0xF, 0xF, false);
+}
+
+// the next lane's value within the row of 16 (lane 15: lane 0's)
+__device__ __forceinline__ int row_next(int x) { return __builtin_amdgcn_update_dpp(0, x, 0x12F, 0xF, 0xF, false); }
+
 struct MlpFrags {
   short4_t B[3][4];  // B operand: lane l holds W1[16 tn + l%16][16 tk + 4 (l/16) + 0..3]
+  uint32_t one[3][2];  // halves of the lane's A operands that are inputs (k < n_env): all ones, else 0
   float b1[4], W2[4];
   float b2, eps;
   int n_env;
@@ -79,6 +101,13 @@ __device__ __forceinline__ void load_frags(cptr<MlpDev> m, int lane, MlpFrags &F
   F.b2 = m->b2;
   F.eps = m->eps;
   F.n_env = m->n_env;
+#pragma unroll
+  for (int tk = 0; tk < 3; ++tk)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int k = 16 * tk + 4 * g + 2 * q;
+      F.one[tk][q] = (k < F.n_env ? 0xFFFFu : 0u) | (k + 1 < F.n_env ? 0xFFFF0000u : 0u);
+    }
 }
 
 // Network outputs of the 64 sites of a wavefront for their current
@@ -97,14 +126,15 @@ __device__ __forceinline__ void mlp_wave(const MlpFrags &F, uint32_t fm_lo, uint
     short4_t A[3];
 #pragma unroll
     for (int tk = 0; tk < 3; ++tk) {
-      short4_t v;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = 16 * tk + 4 * g + q;
-        const uint32_t bit = k < 32 ? (lo >> k) & 1u : (hi >> (k - 32)) & 1u;
-        v[q] = k < F.n_env ? (bit ? (short)0x3F80 : (short)0xBF80) : (short)0;
-      }
-      A[tk] = v;
+      // inputs 16 tk + 4 g + 0..3: 1.0 with the sign of a clear bit, 0 past n_env
+      const uint32_t d = ~(tk < 2 ? lo >> ((16 * tk + 4 * g) & 31) : hi >> (4 * g));
+      union {
+        uint32_t u[2];
+        short4_t v;
+      } w;
+      w.u[0] = F.one[tk][0] & (0x3F803F80u | (d << 15 & 0x8000u) | (d << 30 & 0x80000000u));
+      w.u[1] = F.one[tk][1] & (0x3F803F80u | (d << 13 & 0x8000u) | (d << 28 & 0x80000000u));
+      A[tk] = w.v;
     }
     float pc[4] = {0.f, 0.f, 0.f, 0.f}, pn[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -122,11 +152,8 @@ __device__ __forceinline__ void mlp_wave(const MlpFrags &F, uint32_t fm_lo, uint
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-#pragma unroll
-      for (int o = 8; o > 0; o >>= 1) {
-        pc[r] += __shfl_xor(pc[r], o, 64);
-        pn[r] += __shfl_xor(pn[r], o, 64);
-      }
+      pc[r] = row_all_sum(pc[r]);
+      pn[r] = row_all_sum(pn[r]);
     }
     if (c == 0) {
 #pragma unroll
@@ -199,12 +226,8 @@ __device__ __forceinline__ float row_scan_incl(float x) {
   return x;
 }
 
-// The row's total (the inclusive sum of its last lane) in every lane of the
-// row; rb is the row's first lane.
-__device__ __forceinline__ float row_total(float scan, int rb) {
-  const float z0 = lane_f(scan, 15), z1 = lane_f(scan, 31), z2 = lane_f(scan, 47), z3 = lane_f(scan, 63);
-  return rb == 0 ? z0 : (rb == 16 ? z1 : (rb == 32 ? z2 : z3));
-}
+// The row's total (the inclusive sum of its last lane) in every lane of the row.
+__device__ __forceinline__ float row_total(float scan) { return __int_as_float(row_bcast<15>(__float_as_int(scan))); }
 
 // Weighted choice within a row (lanes rb .. rb + 15): v >= 0 per lane, scan
 // = row_scan_incl(v), t = u * the row's total.  The first lane of the row
@@ -234,11 +257,13 @@ __device__ __forceinline__ float binary_field_l(const uint8_t *img, int pa, int 
         const int len = bs->slot_len[j];
         int X = 0;
         if (ko == 1) {
+#pragma unroll 3
           for (int e = 0; e < len; e += 4) {
             const int q = q0 + e;
             X += (img[pa + off[q]] + img[pa + off[q + 1]]) + (img[pa + off[q + 2]] + img[pa + off[q + 3]]);
           }
         } else if (ko == 2) {
+#pragma unroll 3
           for (int e = 0; e < len; e += 4) {
             const int q = q0 + 2 * e;
             X += ((img[pa + off[q]] ^ img[pa + off[q + 1]]) + (img[pa + off[q + 2]] ^ img[pa + off[q + 3]])) +
@@ -265,8 +290,16 @@ __device__ __forceinline__ float binary_field_l(const uint8_t *img, int pa, int 
 // Grouped-proposal Metropolis kernel (binary path).  KIND 0 canonical, 1 SGC;
 // WEIGHTS 0 uniform, 1 learned network, 2 informed (exact Barker weights).
 // ---------------------------------------------------------------------------
+// The launch has twice the threads of the chain's random streams
+// (la.stream_threads: the block size asked for): wavefront w draws from stream
+// w mod (stream_threads / 64), whose groups are the same ones with either
+// count, so the results do not depend on it.  A group is a chain of dependent
+// shuffles, scans and ballots (half of all wave cycles waited with 8
+// wavefronts per chain).  128 chains of FCC 32^3, 16 rounds, 4 passes: 7.5 ms;
+// 5.5 ms with twice the wavefronts and DPP in place of most shuffles, 4.5 ms
+// with both halves in the pair phases and the inputs built two to a word.
 template <int KIND, int WEIGHTS>
-__global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la) {
+__global__ __launch_bounds__(1024) void learned_kernel(RunArgs args, LearnArgs la) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int chain = blockIdx.x;
   const int tid = threadIdx.x;
@@ -296,17 +329,20 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
   float *logitN = logitC + 16 * 64;         // [n_waves][64]
 
   const int8_t *__restrict__ occG = args.occ + cp->occ_offset;
-  for (int p = tid; p < pad_bytes; p += nthr) {
-    int b = p / S;
-    int r = p - b * S;
-    int pk = r / P12;
-    int r2 = r - pk * P12;
-    int pj = r2 / P1;
-    int pi = r2 - pj * P1;
-    int i = ((pi - h) % L1 + L1) % L1;
-    int j = ((pj - h) % L2 + L2) % L2;
-    int k = ((pk - h) % L3 + L3) % L3;
-    img[p] = (uint8_t)occG[b * n_cells + i + L1 * (j + L2 * k)];
+  {
+    constexpr int kBatch = 8;  // loads in flight per lane
+    PadWalk w(tid, nthr, P1, P12 / P1, S / P12);
+    for (int p0 = tid; p0 < pad_bytes; p0 += kBatch * nthr) {
+      int v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u, w.step())
+        v[u] = p0 + u * nthr < pad_bytes ? occG[w.b * n_cells + pad_wrap(w.pi, h, L1) +
+                                                L1 * (pad_wrap(w.pj, h, L2) + L2 * pad_wrap(w.pk, h, L3))]
+                                         : 0;
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (p0 + u * nthr < pad_bytes) img[p0 + u * nthr] = (uint8_t)v[u];
+    }
   }
   if (tid == 0) *maxDraw = 0ull;
   __syncthreads();
@@ -323,6 +359,10 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
   draw = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(draw >> 32)) << 32) |
          (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)draw);
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  // `draw` is the counter of this wavefront's stream
+  const int n_str = la.stream_threads >> 6;  // streams; two wavefronts each
+  const int str = wave_u % n_str;
+  const int stream_tid = tid < la.stream_threads ? tid : tid - la.stream_threads;
 
   int accC[kMaxSlots];
 #pragma unroll
@@ -349,7 +389,10 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
       uint4 rr = philox4x32_10(make_uint4(0xFFFFFFFDu, (uint32_t)gpass, (uint32_t)c, (uint32_t)chain), k0, k1);
       const int rot = n ? (int)(rr.x % (uint32_t)n) : 0;
       const int n_groups = (n + 63) / 64;
+      const unsigned long long draw0 = draw;
+      const unsigned long long per_group = 64ull * (unsigned long long)((R + 15) / 16);  // blocks a group draws
       for (int grp = wave_u; grp < n_groups; grp += n_waves) {
+        draw = draw0 + (unsigned long long)(grp / n_str) * per_group;
         const int p = grp * 64 + lane;
         const bool valid = p < n;
         int q = p + rot;
@@ -364,6 +407,7 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
         float w = 1.0f, wn = 1.0f;
         if (USE_MLP) {
           uint32_t fm_lo = 0u, fm_hi = 0u;
+#pragma unroll 7
           for (int kk = 0; kk < F.n_env; ++kk) {
             const uint32_t same = (int)img[pa + env[kk]] == o ? 1u : 0u;
             if (kk < 32) fm_lo |= same << kk;
@@ -394,23 +438,27 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
           const int slot = rd & 15;
           if (slot == 0) {
             const unsigned long long dl = draw + (unsigned long long)lane;
-            ul = philox4x32_10(make_uint4(0xFFFF0000u | (uint32_t)wave_u, (uint32_t)dl, (uint32_t)(dl >> 32),
+            ul = philox4x32_10(make_uint4(0xFFFF0000u | (uint32_t)str, (uint32_t)dl, (uint32_t)(dl >> 32),
                                           (uint32_t)chain), k0, k1);
             draw += 64ull;
           }
-          const int src = rb | slot;
-          const uint32_t x1 = (uint32_t)__shfl((int)ul.x, src, 64);
-          const uint32_t x2 = (uint32_t)__shfl((int)ul.y, src, 64);
-          const uint32_t x3 = (uint32_t)__shfl((int)ul.z, src, 64);
+          // lane 0 of the row holds this round's words, then the row moves on
+          // (DPP: a shuffle would cost an LDS round trip)
+          const uint32_t x1 = (uint32_t)row_bcast<0>((int)ul.x), x2 = (uint32_t)row_bcast<0>((int)ul.y),
+                         x3 = (uint32_t)row_bcast<0>((int)ul.z);
           // the fourth word refines an acceptance test whose 32-bit word ties
-          const uint32_t x4 = (uint32_t)__shfl((int)ul.w, src, 64);
+          const uint32_t x4 = (uint32_t)row_bcast<0>((int)ul.w);
+          ul.x = (uint32_t)row_next((int)ul.x);
+          ul.y = (uint32_t)row_next((int)ul.y);
+          ul.z = (uint32_t)row_next((int)ul.z);
+          ul.w = (uint32_t)row_next((int)ul.w);
           auto more = [&]() { return x4; };
           const float u1 = u01(x1);
           if (KIND == 0) {
             const float vA = (o == 0) ? w : 0.0f;
             const float vB = (o == 1) ? w : 0.0f;
             const float sA = row_scan_incl(vA), sB = row_scan_incl(vB);
-            const float ZA = row_total(sA, rb), ZB = row_total(sB, rb);
+            const float ZA = row_total(sA), ZB = row_total(sB);
             const bool live = ZA > 0.0f && ZB > 0.0f;
             const int la_ = row_pick(vA, sA, u1 * ZA, rb), lb_ = row_pick(vB, sB, u01(x2) * ZB, rb);
             const bool prop = live && la_ >= 0 && lb_ >= 0;
@@ -437,7 +485,7 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
             }
           } else {
             const float sv = row_scan_incl(w);
-            const float Z = row_total(sv, rb);
+            const float Z = row_total(sv);
             const int ls = row_pick(w, sv, u1 * Z, rb);
             const bool prop = Z > 0.0f && ls >= 0;
             const int ps = prop ? ls : lane;
@@ -469,6 +517,8 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
           if (KIND == 1) accN1 += o0 ? -1 : 1;
         }
       }
+      // the stream's groups of this class: str, str + n_str, ...
+      draw = draw0 + (unsigned long long)((n_groups - str + n_str - 1) / n_str) * per_group;
       __syncthreads();
       for (int t = sc->halo_begin[c] + tid; t < sc->halo_begin[c + 1]; t += nthr) {
         const int2 hc = sc->halo[t];
@@ -491,12 +541,14 @@ __global__ __launch_bounds__(512) void learned_kernel(RunArgs args, LearnArgs la
                               .x %
                           (uint32_t)sc->n_pair_phases;
       const int pb = sc->pair_begin[ph], pe = sc->pair_begin[ph + 1];
+      // (the pairs of a phase share no cluster: the threads of both halves
+      // take one each, with the words of thread tid mod stream_threads)
       for (int t = pb + tid; t < pe; t += nthr) {
         const int2 pq = sc->pair_addr[t];
         const int bpq = sc->pair_sublat[t];
         const int op = img[pq.x], oq = img[pq.y];
         if (op == oq) continue;
-        const uint4 ur = philox4x32_10(make_uint4((uint32_t)tid, (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
+        const uint4 ur = philox4x32_10(make_uint4((uint32_t)stream_tid, (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
                                                  (uint32_t)chain), k0, k1);
         int Kp[kMaxSlots], Kq[kMaxSlots];
         const float Fp = binary_field_l(img, pq.x, op, cst(sc->bin_sub + (bpq & 0xFF)), bin_off, n_slots, Kp);
@@ -873,15 +925,6 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kTrainParams = kHidden * kEnvMax + 2 * kHidden + 1;
 
-// sum over a row of 16 lanes, in every lane (DPP row rotations)
-__device__ __forceinline__ float row_all_sum(float x) {
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xF, 0xF, false));
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xF, 0xF, false));
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xF, 0xF, false));
-  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xF, 0xF, false));
-  return x;
-}
-
 __global__ __launch_bounds__(256) void mlp_step_kernel(TrainArgs a) {
   __shared__ double red[kTrainParams + 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1061,7 +1104,9 @@ static hipError_t launch_l(const RunArgs &args, const LearnArgs &la, int n_chain
                            hipStream_t st, bool launch) {
   auto kern = learned_kernel<KIND, WEIGHTS>;
   if (!launch) return hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  hipLaunchKernelGGL(kern, dim3(n_chains), dim3(threads), lds, st, args, la);
+  LearnArgs l2 = la;
+  l2.stream_threads = threads;
+  hipLaunchKernelGGL(kern, dim3(n_chains), dim3(2 * threads), lds, st, args, l2);
   return hipGetLastError();
 }
 
