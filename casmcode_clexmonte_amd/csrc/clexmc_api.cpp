@@ -40,6 +40,9 @@ struct HostSupercell {
   size_t jit_lds_fail = 0;  // smallest dynamic LDS size at which a specialised launch was refused
   std::vector<hipModule_t> jit_mods;
   hipFunction_t jit_fn[3][2][2][2] = {};  // [kind][packed][lanes][block above 512]
+  // the same for sets of a few sites (spread fields) [kind 0, 1]
+  int jit_spread_state[2] = {};
+  hipFunction_t jit_spread[2] = {};
   hipFunction_t jit_nfold = nullptr;  // N-fold kernel of the SGC (unpacked, one-lane) module
   hipFunction_t jit_cube[2] = {nullptr, nullptr};  // register-cube kernel of that module [block above 512]
   // register-cube sweep (binary, one sublattice, classes = the residues of
@@ -1559,7 +1562,8 @@ clexmc_status clexmc_set_lds_row_pitch(clexmc_handle *h, int extra) {
   return CLEXMC_OK;
 }
 
-static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads);
+static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads,
+                                bool spread = false);
 
 // Chains whose N-fold run stopped because their total rate vanished: the
 // flags are cleared and the run reported as failed (its blocks past the stop
@@ -1777,6 +1781,8 @@ struct RunPlan {
   int slabs = 1;                // workgroups per chain (slab decomposition along k)
   bool threads_auto = false;    // block size chosen by the planner (not requested)
   bool cube = false;            // jit is the register-cube kernel
+  bool spread = false;          // jit spreads a site's clusters over the lanes
+  size_t lds_spread = 0;        // LDS that takes
   unsigned long long pass_start = 0;  // the chains' pass counter before the run
   RunArgs a;
   LearnArgs la;
@@ -1785,19 +1791,20 @@ struct RunPlan {
 // The specialised kernel for (supercell, kind, packing, lanes per site, block
 // size above 512 or not), compiled on first use; nullptr when specialisation
 // is off or unavailable.
-static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads) {
+static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads,
+                                bool spread) {
   HostSupercell &hs = h->scs[sc_id];
   const int k = kind < 0 ? 0 : (kind > 2 ? 2 : kind), p = packed ? 1 : 0, l = lanes == 2 ? 1 : 0,
             w = lanes * threads > kAotMaxThreads;
-  int &state = hs.jit_state[k][p][l][w];
-  hipFunction_t &fn = hs.jit_fn[k][p][l][w];
+  int &state = spread ? hs.jit_spread_state[k] : hs.jit_state[k][p][l][w];  // spread: kinds 0 and 1
+  hipFunction_t &fn = spread ? hs.jit_spread[k] : hs.jit_fn[k][p][l][w];
   if (state == 0) {
     state = -1;
     std::vector<int> variable(h->n_sublat);
     for (int b = 0; b < h->n_sublat; ++b) variable[b] = h->n_occ[b] >= 2;
     const std::string src = jit_source(h->n_sublat, variable, h->binary != 0, hs.bin_sub, hs.bin_off, h->n_slots,
                                        hs.gen_sub, hs.gen_prog, kind, packed, lanes, w ? kMaxJitThreads : kAotMaxThreads,
-                                       hs.cube_ok ? &hs.cube : nullptr);
+                                       hs.cube_ok ? &hs.cube : nullptr, spread);
     hipModule_t mod = nullptr;
     const hipError_t je = jit_compile_load(src, &mod, &h->jit_log);
     if (je != hipSuccess) h->jit_log += std::string("\n[compile/load: ") + hipGetErrorString(je) + "]";
@@ -1805,9 +1812,9 @@ static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool pack
       if (hipModuleGetFunction(&fn, mod, jit_kernel_name(kind, packed, lanes)) == hipSuccess) {
         hs.jit_mods.push_back(mod);
         state = 1;
-        if (k == 1 && p == 0 && l == 0 && hipModuleGetFunction(&hs.jit_nfold, mod, kJitNfoldName) != hipSuccess)
+        if (!spread && k == 1 && p == 0 && l == 0 && hipModuleGetFunction(&hs.jit_nfold, mod, kJitNfoldName) != hipSuccess)
           hs.jit_nfold = nullptr;
-        if (k == 1 && p == 0 && l == 0 && hs.cube_ok &&
+        if (!spread && k == 1 && p == 0 && l == 0 && hs.cube_ok &&
             hipModuleGetFunction(&hs.jit_cube[w], mod, kJitCubeName) != hipSuccess)
           hs.jit_cube[w] = nullptr;
       } else {
@@ -1848,6 +1855,33 @@ static clexmc_status grow_samples(clexmc_handle *h, long long n_new_samples) {
     h->sample_cap = cap;
   }
   return CLEXMC_OK;
+}
+
+static constexpr int kMinSlabSites = 8192;  // sites per workgroup of a slab, at least
+
+// LDS of the spread kernel's rows for a launch of 64 threads per chain on
+// supercell hs, 0: the launch keeps lane = site.  A set then costs the same
+// whatever it holds (4.0 us: ternary HCP, 406 clusters), while spread fields
+// cost 1.8 us and 0.2 us per site: 5 passes of 64 chains, lane = site -> spread,
+//   HCP   8 x 7 x 7  (2 sites per set)   7.80 -> 4.38 ms
+//   HCP  11 x 9 x 7  (3)                 9.23 -> 5.56 ms
+//   BCC  10 x 10 x 7 (4; 269 clusters)   5.08 -> 2.79 ms
+//   BCC   7 x 9 x 8  (6)                 2.50 -> 1.64 ms
+//   BCC   8 x 8 x 10 (8)                 2.38 -> 1.79 ms
+//   HCP  10 x 9 x 9  (18)                1.92 -> 2.52 ms
+// so the line is drawn at 8 sites.
+static size_t spread_lds(const clexmc_handle *h, const HostSupercell &hs, size_t lds) {
+  const DevSupercell &d = hs.dev;
+  // (no slabs: asked for, or cut by themselves from 12,288 sites on)
+  if (h->binary || h->slabs >= 2 || (h->slabs == 0 && d.n_sites >= kMinSlabSites * 3 / 2)) return 0;
+  if (d.max_class > kSpreadMaxSites) return 0;
+  std::vector<int> variable(h->n_sublat);
+  for (int b = 0; b < h->n_sublat; ++b) variable[b] = h->n_occ[b] >= 2;
+  const int items = spread_items(variable, hs.gen_sub, hs.gen_prog);
+  if (items == 0) return 0;
+  const size_t extra = class_occ_bytes(d.max_class) + 16 +
+                       sizeof(float) * (size_t)d.max_class * h->n_func_max * spread_row_stride(items);
+  return (long long)(lds + extra) <= (long long)h->max_lds - 64 ? extra : 0;
 }
 
 // threads_override / packing_override: 0 = the handle's setting
@@ -1958,8 +1992,16 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
     P.sc_id = h->chain_sc[c0];
     P.one_shape = one_shape;
     const size_t fail = h->scs[h->chain_sc[c0]].jit_lds_fail;
-    if (h->specialize && !P.learned && one_shape && !fused_spec && (fail == 0 || lds < fail))
-      P.jit = jit_kernel(h, h->chain_sc[c0], kind, packed, P.lanes, P.threads);
+    if (h->specialize && !P.learned && one_shape && !fused_spec && (fail == 0 || lds < fail)) {
+      if (P.threads == 64 && kind != 2 && !packed && P.lanes == 1)
+        P.lds_spread = spread_lds(h, h->scs[h->chain_sc[c0]], P.lds);
+      if (P.lds_spread > 0) {
+        P.jit = jit_kernel(h, h->chain_sc[c0], kind, false, 1, 64, true);
+        P.spread = P.jit != nullptr;
+        if (P.spread) P.lds += P.lds_spread;
+      }
+      if (!P.jit) P.jit = jit_kernel(h, h->chain_sc[c0], kind, packed, P.lanes, P.threads);
+    }
   }
   if (!P.jit && !fused_spec) P.threads = std::min(P.threads, kAotMaxThreads);
   // the register-cube sweep: the specialised semi-grand canonical kernel's
@@ -1984,6 +2026,8 @@ static void drop_jit(clexmc_handle *h, RunPlan &P, int sc_id) {
   h->scs[sc_id].jit_lds_fail = P.lds;
   P.jit = nullptr;
   P.cube = false;
+  if (P.spread) P.lds -= P.lds_spread;
+  P.spread = false;
   P.threads = std::min(P.threads, kAotMaxThreads);
 }
 
@@ -2053,7 +2097,6 @@ static hipError_t plan_launch(const RunPlan &P, clexmc_handle *h, hipStream_t st
 // planes updated per launch), at most kMaxSlabs.  Requested (>= 2): that many
 // slabs where every slab keeps an updated plane.  Single-shape, plain
 // Metropolis launches with one lane per site only.
-static constexpr int kMinSlabSites = 8192;
 static constexpr int kMaxSlabs = 16;
 
 static hipError_t choose_slabs(clexmc_handle *h, const std::vector<RunPlan *> &plans) {

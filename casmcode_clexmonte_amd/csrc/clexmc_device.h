@@ -37,6 +37,13 @@ constexpr int kMaxAutoRounds = 1024; // canonical matchings per independent set 
 constexpr int kAotMaxThreads = 512;  // launch bound of the ahead-of-time Metropolis kernels
 constexpr int kMaxJitThreads = 1024; // launch bound of run-time specialised kernels for large classes
 
+// Spread fields (metropolis_body, SPREAD): floats between the rows of two site
+// functions or sites, for `items` clusters per lane.  16-byte reads; the 4 on
+// top start the summing lanes in different LDS banks.
+constexpr int spread_row_stride(int items) { return 64 * items + 4; }
+constexpr int kSpreadMaxSites = 8;  // sites of an independent set, at most
+static_assert(kSpreadMaxSites * kMaxFunc <= 64, "one lane adds the rows of one (site, function)");
+
 // Automatic canonical rounds of one independent set.  A random matching of
 // the set's n sites pairs a given site with each other site with probability
 // 1/n, so a round makes m / (2n) attempts between different occupants on

@@ -83,6 +83,7 @@ static void emit_field(std::ostringstream &o, const std::string &name, int n_sub
                        const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog, bool packed,
                        int max_threads, const CubeSpec *cube = nullptr) {
   o << "struct " << name << " {\n"
+    << "  static constexpr int kSpreadSub = 1, kSpreadItems = 1;  // see SpreadField\n"
     << "  template <class IMG>\n"
     << "  __device__ __forceinline__ static float bin(const FieldCtx &, const IMG &img, int b, int pa, int o,\n"
     << "                                              int (&K)[kMaxSlots]) {\n"
@@ -419,11 +420,76 @@ static void emit_cube(std::ostringstream &o, const BinSub &B, const std::vector<
   o << "  }\n";
 }
 
+int spread_items(const std::vector<int> &variable, const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog) {
+  int items = 0;
+  for (size_t b = 0; b < variable.size(); ++b) {
+    if (!variable[b]) continue;
+    const GenSub &S = gsubs[b];
+    items = std::max(items, (S.n_entries + 63) / 64);
+    int q = S.begin;
+    for (int e = 0; e < S.n_entries; ++e) {
+      const int k = gen_prog[q];
+      if (k > 3) return 0;
+      q += 2;
+      for (int i = 0; i < k; ++i, q += 2)
+        if (std::abs(gen_prog[q]) >= 1 << 23 || gen_prog[q + 1] < 0 || gen_prog[q + 1] > 255) return 0;
+    }
+  }
+  return variable.size() <= 4 && items * (int)variable.size() <= 16 ? items : 0;
+}
+
+// The spread kernel's field policy (the sweep's fields; JitField's for the
+// pair phases): cluster e of sublattice b as four words,
+// table offset, then (site offset << 8 | multiplier) three times; zeros (an
+// occupant times 0, the table's first row, stored and never added) fill up the
+// clusters' missing sites and the lanes' missing clusters.
+static void emit_spread(std::ostringstream &o, const std::vector<int> &variable, const std::vector<GenSub> &gsubs,
+                        const std::vector<int> &gen_prog) {
+  const int n_sublat = (int)variable.size(), items = spread_items(variable, gsubs, gen_prog);
+  o << "__device__ const int kSpreadDesc[" << n_sublat << "][" << 64 * items << "][4] = {\n";
+  for (int b = 0; b < n_sublat; ++b) {
+    o << "{";
+    int q = gsubs[b].begin;
+    for (int e = 0; e < 64 * items; ++e) {
+      int w[4] = {0, 0, 0, 0};
+      if (variable[b] && e < gsubs[b].n_entries) {
+        const int k = gen_prog[q];
+        w[0] = gen_prog[q + 1];
+        q += 2;
+        for (int i = 0; i < k; ++i, q += 2) w[1 + i] = gen_prog[q] * 256 + gen_prog[q + 1];
+      }
+      o << "{" << w[0] << "," << w[1] << "," << w[2] << "," << w[3] << "},";
+    }
+    o << "},\n";
+  }
+  o << "};\nstruct SpreadField : JitField {\n"
+    << "  static constexpr int kSpreadSub = " << n_sublat << ", kSpreadItems = " << items << ";\n"
+    << "  __device__ __forceinline__ static uint4 spread_desc(int b, int e) {\n"
+    << "    const int *d = kSpreadDesc[b][e];\n"
+    << "    return make_uint4((uint32_t)d[0], (uint32_t)d[1], (uint32_t)d[2], (uint32_t)d[3]);\n  }\n"
+    << "  __device__ static constexpr int spread_entries(int b) {\n    return 0";
+  for (int b = 0; b < n_sublat; ++b)
+    if (variable[b]) o << " + (b == " << b << " ? " << gsubs[b].n_entries << " : 0)";
+  o << ";\n  }\n  __device__ static constexpr int spread_func(int b) {\n    return 0";
+  for (int b = 0; b < n_sublat; ++b)
+    if (variable[b]) o << " + (b == " << b << " ? " << std::min(gsubs[b].nf, kMaxFunc) << " : 0)";
+  o << ";\n  }\n};\n";
+}
+
 std::string jit_source(int n_sublat, const std::vector<int> &variable, bool binary, const std::vector<BinSub> &subs,
                        const std::vector<int> &bin_off, int n_slots, const std::vector<GenSub> &gsubs,
                        const std::vector<int> &gen_prog, int kind, bool packed, int lanes, int max_threads,
-                       const CubeSpec *cube) {
+                       const CubeSpec *cube, bool spread) {
   std::ostringstream o;
+  if (spread) {
+    o << "#include \"clexmc_metropolis.h\"\nnamespace clexmc {\n";
+    emit_field(o, "JitField", n_sublat, variable, false, subs, bin_off, n_slots, gsubs, gen_prog, false, max_threads);
+    emit_spread(o, variable, gsubs, gen_prog);
+    o << "}  // namespace clexmc\nextern \"C\" __global__ __launch_bounds__(64) void " << jit_kernel_name(kind, false, 1)
+      << "(clexmc::RunArgs a) { clexmc::metropolis_body<false, " << kind
+      << ", false, clexmc::SpreadField, 1, false, true>(a, clexmc::BlockRole{(int)blockIdx.x, a.chain_map, a.slabs}); }\n";
+    return o.str();
+  }
   // the semi-grand canonical, unpacked, one-lane variant also carries the N-fold kernel
   const bool with_nfold = kind == 1 && !packed && lanes == 1;
   o << "#include \"clexmc_metropolis.h\"\n" << (with_nfold ? "#include \"clexmc_nfold.h\"\n" : "")

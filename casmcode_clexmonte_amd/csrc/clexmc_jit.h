@@ -33,11 +33,20 @@ struct CubeSpec {
 // One kernel per (kind, packed, lanes per site) variant; `max_threads` (512 or
 // 1024) is its launch bound.
 // `cube` (semi-grand canonical, unpacked, one-lane variant only; may be
-// nullptr) adds the register-cube sweep.
+// nullptr) adds the register-cube sweep.  `spread` (general, unpacked, one
+// lane per site, kinds 0 and 1, spread_items() > 0): the kernel for sets of a
+// few sites instead (metropolis_body, SPREAD).
 std::string jit_source(int n_sublat, const std::vector<int> &variable, bool binary, const std::vector<BinSub> &subs,
                        const std::vector<int> &bin_off, int n_slots, const std::vector<GenSub> &gsubs,
                        const std::vector<int> &gen_prog, int kind, bool packed, int lanes, int max_threads,
-                       const CubeSpec *cube = nullptr);
+                       const CubeSpec *cube = nullptr, bool spread = false);
+
+// Table rows that each lane of a wavefront forms per site in the spread kernel
+// (the largest program of a variable sublattice, over 64 lanes); 0 where its
+// descriptors cannot hold the programs (clusters of more than three other
+// sites, offsets of 2^23 or more, multipliers above 255), would take too many
+// registers (16 rows, all sublattices together) or for more than 4 sublattices.
+int spread_items(const std::vector<int> &variable, const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog);
 
 // One supercell shape of a fused launch: its site programs (as for
 // jit_source) and image format.

@@ -356,6 +356,7 @@ struct FieldCtx {
 
 struct GenericField {
   static constexpr bool kCube = false;
+  static constexpr int kSpreadSub = 1, kSpreadItems = 1;
   struct Cube {};
   template <class IMG>
   __device__ __forceinline__ static float bin(const FieldCtx &c, const IMG &img, int b, int pa, int o,
@@ -376,6 +377,12 @@ struct GenericField {
                                              float (&G)[kMaxFunc]) {
     general_field(img, pa, cst(c.sc->gen_sub + b), c.gen_prog, tab, G);
   }
+};
+
+// a sublattice as a type, for programs built in per sublattice
+template <int B>
+struct SublatIndex {
+  static constexpr int value = B;
 };
 
 // ---------------------------------------------------------------------------
@@ -400,8 +407,18 @@ struct BlockRole {
 
 // CUBE: the register-cube sweep instead of the class loop (the field policy
 // must provide it; semi-grand canonical binary one-lane unpacked only).
-template <bool BIN, int KIND, bool PACK, class FIELD, int SPLIT = 1, bool CUBE = false>
+// SPREAD: blocks of one wavefront whose independent sets hold a few sites only
+// (tables; small and ragged supercells).  With lane = site such a set's fields
+// are one long stream of instructions in two or three lanes.  Here lane =
+// cluster: every lane forms the table rows of its clusters (descriptors in its
+// registers, FIELD::spread_desc) for one site after the other into LDS, then
+// one lane per (site, function) adds its rows in cluster order, so the fields
+// are the same bit for bit.  Bound by the row latencies and by the additions, one
+// after the other: 64 ternary HCP chains of 11 x 9 x 7 (sets of 3 sites, 406
+// clusters), 10 passes, 18.5 ms -> 11.1 ms.
+template <bool BIN, int KIND, bool PACK, class FIELD, int SPLIT = 1, bool CUBE = false, bool SPREAD = false>
 __device__ __forceinline__ void metropolis_body(const RunArgs &args, const BlockRole role) {
+  static_assert(!SPREAD || (!BIN && !PACK && SPLIT == 1 && !CUBE && KIND != 2), "spread fields: tables, one-lane sweeps");
   extern __shared__ __align__(16) unsigned char smem[];
   // slabs > 1: this workgroup runs slab `slab` of its chain
   const int n_slabs = role.slabs > 1 ? role.slabs : 1;
@@ -458,6 +475,9 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
   // occupants of the class in canonical matchings (args.class_occ)
   uint8_t *cO = (uint8_t *)(cF + nfs * max_class);       // [max_class]
   static_assert(kMaxSlots == 8, "cluster sums of a site are 8 bytes");
+  // spread fields: the clusters' rows of the class's sites
+  const size_t off_r = off_b + (size_t)(BIN ? 8 * max_class : 0) + (size_t)nfs * max_class * 4 + (size_t)max_class;
+  [[maybe_unused]] float *cR = (float *)(smem + ((off_r + 15) & ~(size_t)15));
   auto pack_K = [](const int (&K)[kMaxSlots]) -> uint2 {
     return make_uint2(((uint32_t)K[0] & 255u) | ((uint32_t)K[1] & 255u) << 8 | ((uint32_t)K[2] & 255u) << 16 |
                           (uint32_t)K[3] << 24,
@@ -730,6 +750,86 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
                        (uint32_t)__builtin_amdgcn_readlane((int)x, l));
   };
 
+  // spread fields of a class (n sites, lane t has the t-th's address pa): lane
+  // v * nf + f returns function f of site v
+  [[maybe_unused]] uint4 desc[SPREAD ? FIELD::kSpreadSub : 1][SPREAD ? FIELD::kSpreadItems : 1];
+  if constexpr (SPREAD) {
+#pragma unroll
+    for (int q = 0; q < FIELD::kSpreadSub; ++q)
+#pragma unroll
+      for (int i = 0; i < FIELD::kSpreadItems; ++i) desc[q][i] = FIELD::spread_desc(q, lane + 64 * i);
+  }
+  [[maybe_unused]] auto spread_sub = [&](auto sub, int n, int pa) -> float {
+    float g = 0.0f;
+    if constexpr (SPREAD) {
+      constexpr int q = decltype(sub)::value, I = FIELD::kSpreadItems, stride = spread_row_stride(I),
+                    nf = FIELD::spread_func(q), ne = FIELD::spread_entries(q);
+      if (n <= 0 || nf == 0) return g;
+      int x[I][3];
+      auto occupants = [&](int v) {
+        const int pv = __builtin_amdgcn_readlane(pa, v);
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+          x[i][0] = img.get(pv + ((int)desc[q][i].y >> 8));
+          x[i][1] = img.get(pv + ((int)desc[q][i].z >> 8));
+          x[i][2] = img.get(pv + ((int)desc[q][i].w >> 8));
+        }
+      };
+      occupants(0);
+      for (int v = 0; v < n; ++v) {
+        float row[I][nf > 0 ? nf : 1];
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+          const uint4 d = desc[q][i];
+          // (occupants below 4, multipliers below 256: 24-bit products)
+          const int idx = (int)((x[i][0] & 3u) * (d.y & 255u) + (x[i][1] & 3u) * (d.z & 255u) +
+                                (x[i][2] & 3u) * (d.w & 255u));
+          const float *V = tabL + (int)d.x + idx * nf;
+#pragma unroll
+          for (int f = 0; f < nf; ++f) row[i][f] = V[f];
+        }
+        if (v + 1 < n) occupants(v + 1);  // on their way while the rows arrive and are stored
+        float *out = cR + v * nf * stride + lane;
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+          for (int f = 0; f < nf; ++f) out[f * stride + 64 * i] = row[i][f];
+      }
+      lds_barrier();
+      // eight reads of four rows on their way while the eight before are added
+      // (whole batches: at most the 64 I rows stored)
+      if (lane < n * nf) {
+        const float4 *r = (const float4 *)(cR + lane * stride);
+        constexpr int nb = (ne + 31) / 32;
+        float4 y[2][8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) y[0][u] = r[u];
+#pragma unroll
+        for (int e = 0; e < nb; ++e) {
+          if (e + 1 < nb)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) y[(e + 1) & 1][u] = r[8 * (e + 1) + u];
+          asm volatile("" : "+v"(g) : : "memory");
+#pragma unroll
+          for (int u = 0; u < 32; ++u) {
+            const float4 w = y[e & 1][u >> 2];
+            if (32 * e + u < ne) g += (u & 3) == 0 ? w.x : (u & 3) == 1 ? w.y : (u & 3) == 2 ? w.z : w.w;
+          }
+        }
+      }
+    }
+    return g;
+  };
+  [[maybe_unused]] auto spread_fields = [&](int b, int n, int pa) -> float {
+    if (b == 0) return spread_sub(SublatIndex<0>{}, n, pa);
+    if constexpr (SPREAD && FIELD::kSpreadSub > 1)
+      if (b == 1) return spread_sub(SublatIndex<1>{}, n, pa);
+    if constexpr (SPREAD && FIELD::kSpreadSub > 2)
+      if (b == 2) return spread_sub(SublatIndex<2>{}, n, pa);
+    if constexpr (SPREAD && FIELD::kSpreadSub > 3) return spread_sub(SublatIndex<3>{}, n, pa);
+    return 0.0f;
+  };
+
   ClassNums nums1{}, nums2{};
   ClassFirst first1{0, make_int2(0, 0)};
   if (!use_cube) {
@@ -836,7 +936,14 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               if (acc) img.set(pa, o, 1 - o);
             }
           }
-        } else
+        } else {
+        [[maybe_unused]] const int nf = SPREAD ? (int)gs->nf : 0;
+        [[maybe_unused]] float spread[kMaxFunc];
+        if constexpr (SPREAD) {
+          const float g = spread_fields(b, nR, first.pa);
+#pragma unroll
+          for (int f = 0; f < kMaxFunc; ++f) spread[f] = f < nf ? __shfl(g, (lane * nf + f) & 63) : 0.0f;
+        }
         for (int v = tid; v < nR; v += nthr) {
           const int pa = v == tid ? first.pa : sc->class_addr[R.at(v)];
           const int o = img.get(pa);
@@ -857,7 +964,12 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             if (acc) img.set(pa, o, 1 - o);
           } else {
             float G[kMaxFunc];
-            FIELD::gen(fctx, img, b, pa, tabL, G);
+            if constexpr (SPREAD) {
+#pragma unroll
+              for (int f = 0; f < kMaxFunc; ++f) G[f] = spread[f];
+            } else {
+              FIELD::gen(fctx, img, b, pa, tabL, G);
+            }
             const int no = sys->n_occ[b];
             const float u2 = rng.next();
             int r = (int)(u2 * (float)(no - 1));
@@ -875,6 +987,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               for (int q = 0; q < kMaxOcc; ++q) accN[q] += (q == nw) - (q == o);
             }
           }
+        }
         }
         lds_barrier();
       } else {
@@ -904,7 +1017,12 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
               cK[t] = pack_K(K);
             }
           }
-        } else
+        } else {
+        if constexpr (SPREAD) {
+          const int nf = gs->nf;
+          const float g = spread_fields(b, n, first.pa);
+          if (lane < n * nf) cF[(lane % nf) * max_class + lane / nf] = g;
+        }
         for (int t = tid; t < n; t += nthr) {
           const int pa = t == tid ? first.pa : sc->class_addr[R.at(t)];
           const int o = img.get(pa);
@@ -913,13 +1031,14 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
             int K[kMaxSlots];
             cF[t] = FIELD::bin(fctx, img, b, pa, o, K);
             cK[t] = pack_K(K);
-          } else {
+          } else if constexpr (!SPREAD) {
             float G[kMaxFunc];
             FIELD::gen(fctx, img, b, pa, tabL, G);
             cF[t] = G[0];
             if (nfs > 1) cF[max_class + t] = G[1];
             if (nfs > 2) cF[2 * max_class + t] = G[2];
           }
+        }
         }
         lds_barrier();
         for (int rd = 0; rd < n_rounds; ++rd) {
