@@ -1862,7 +1862,8 @@ static constexpr int kMinSlabSites = 8192;  // sites per workgroup of a slab, at
 // LDS of the spread kernel's rows for a launch of 64 threads per chain on
 // supercell hs, 0: the launch keeps lane = site.  A set then costs the same
 // whatever it holds (4.0 us: ternary HCP, 406 clusters), while spread fields
-// cost 1.8 us and 0.2 us per site: 5 passes of 64 chains, lane = site -> spread,
+// cost 1.8 us and 0.2 us per site: 5 passes of 64 chains, lane = site -> spread
+// (rows of one site after the other; three at a time take 2 % less at 3 sites),
 //   HCP   8 x 7 x 7  (2 sites per set)   7.80 -> 4.38 ms
 //   HCP  11 x 9 x 7  (3)                 9.23 -> 5.56 ms
 //   BCC  10 x 10 x 7 (4; 269 clusters)   5.08 -> 2.79 ms

@@ -379,10 +379,10 @@ struct GenericField {
   }
 };
 
-// a sublattice as a type, for programs built in per sublattice
-template <int B>
-struct SublatIndex {
-  static constexpr int value = B;
+// a number as a type (a sublattice whose program is built in, a loop's length)
+template <int N>
+struct IntConst {
+  static constexpr int value = N;
 };
 
 // ---------------------------------------------------------------------------
@@ -411,11 +411,12 @@ struct BlockRole {
 // (tables; small and ragged supercells).  With lane = site such a set's fields
 // are one long stream of instructions in two or three lanes.  Here lane =
 // cluster: every lane forms the table rows of its clusters (descriptors in its
-// registers, FIELD::spread_desc) for one site after the other into LDS, then
+// registers, FIELD::spread_desc) for three sites at a time into LDS, then
 // one lane per (site, function) adds its rows in cluster order, so the fields
 // are the same bit for bit.  Bound by the row latencies and by the additions, one
 // after the other: 64 ternary HCP chains of 11 x 9 x 7 (sets of 3 sites, 406
-// clusters), 10 passes, 18.5 ms -> 11.1 ms.
+// clusters), 10 passes, 18.5 ms -> 10.9 ms (rows of one site after the other:
+// 11.1 ms).
 template <bool BIN, int KIND, bool PACK, class FIELD, int SPLIT = 1, bool CUBE = false, bool SPREAD = false>
 __device__ __forceinline__ void metropolis_body(const RunArgs &args, const BlockRole role) {
   static_assert(!SPREAD || (!BIN && !PACK && SPLIT == 1 && !CUBE && KIND != 2), "spread fields: tables, one-lane sweeps");
@@ -765,36 +766,46 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
       constexpr int q = decltype(sub)::value, I = FIELD::kSpreadItems, stride = spread_row_stride(I),
                     nf = FIELD::spread_func(q), ne = FIELD::spread_entries(q);
       if (n <= 0 || nf == 0) return g;
-      int x[I][3];
-      auto occupants = [&](int v) {
-        const int pv = __builtin_amdgcn_readlane(pa, v);
+      // the rows of nv sites from v0 on: all occupants, then all rows, are on
+      // their way together
+      auto rows = [&](auto nv, int v0) {
+        constexpr int V = decltype(nv)::value;
+        int x[V][I][3];
 #pragma unroll
-        for (int i = 0; i < I; ++i) {
-          x[i][0] = img.get(pv + ((int)desc[q][i].y >> 8));
-          x[i][1] = img.get(pv + ((int)desc[q][i].z >> 8));
-          x[i][2] = img.get(pv + ((int)desc[q][i].w >> 8));
+        for (int v = 0; v < V; ++v) {
+          const int pv = __builtin_amdgcn_readlane(pa, v0 + v);
+#pragma unroll
+          for (int i = 0; i < I; ++i) {
+            x[v][i][0] = img.get(pv + ((int)desc[q][i].y >> 8));
+            x[v][i][1] = img.get(pv + ((int)desc[q][i].z >> 8));
+            x[v][i][2] = img.get(pv + ((int)desc[q][i].w >> 8));
+          }
         }
+        float row[V][I][nf > 0 ? nf : 1];
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+#pragma unroll
+          for (int i = 0; i < I; ++i) {
+            const uint4 d = desc[q][i];
+            // (occupants below 4, multipliers below 256: 24-bit products)
+            const int idx = (int)((x[v][i][0] & 3u) * (d.y & 255u) + (x[v][i][1] & 3u) * (d.z & 255u) +
+                                  (x[v][i][2] & 3u) * (d.w & 255u));
+            const float *T = tabL + (int)d.x + idx * nf;
+#pragma unroll
+            for (int f = 0; f < nf; ++f) row[v][i][f] = T[f];
+          }
+        float *out = cR + v0 * nf * stride + lane;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+#pragma unroll
+          for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int f = 0; f < nf; ++f) out[(v * nf + f) * stride + 64 * i] = row[v][i][f];
       };
-      occupants(0);
-      for (int v = 0; v < n; ++v) {
-        float row[I][nf > 0 ? nf : 1];
-#pragma unroll
-        for (int i = 0; i < I; ++i) {
-          const uint4 d = desc[q][i];
-          // (occupants below 4, multipliers below 256: 24-bit products)
-          const int idx = (int)((x[i][0] & 3u) * (d.y & 255u) + (x[i][1] & 3u) * (d.z & 255u) +
-                                (x[i][2] & 3u) * (d.w & 255u));
-          const float *V = tabL + (int)d.x + idx * nf;
-#pragma unroll
-          for (int f = 0; f < nf; ++f) row[i][f] = V[f];
-        }
-        if (v + 1 < n) occupants(v + 1);  // on their way while the rows arrive and are stored
-        float *out = cR + v * nf * stride + lane;
-#pragma unroll
-        for (int i = 0; i < I; ++i)
-#pragma unroll
-          for (int f = 0; f < nf; ++f) out[f * stride + 64 * i] = row[i][f];
-      }
+      int v = 0;
+      for (; v + 3 <= n; v += 3) rows(IntConst<3>{}, v);
+      if (n - v == 2) rows(IntConst<2>{}, v);
+      if (n - v == 1) rows(IntConst<1>{}, v);
       lds_barrier();
       // eight reads of four rows on their way while the eight before are added
       // (whole batches: at most the 64 I rows stored)
@@ -821,12 +832,12 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
     return g;
   };
   [[maybe_unused]] auto spread_fields = [&](int b, int n, int pa) -> float {
-    if (b == 0) return spread_sub(SublatIndex<0>{}, n, pa);
+    if (b == 0) return spread_sub(IntConst<0>{}, n, pa);
     if constexpr (SPREAD && FIELD::kSpreadSub > 1)
-      if (b == 1) return spread_sub(SublatIndex<1>{}, n, pa);
+      if (b == 1) return spread_sub(IntConst<1>{}, n, pa);
     if constexpr (SPREAD && FIELD::kSpreadSub > 2)
-      if (b == 2) return spread_sub(SublatIndex<2>{}, n, pa);
-    if constexpr (SPREAD && FIELD::kSpreadSub > 3) return spread_sub(SublatIndex<3>{}, n, pa);
+      if (b == 2) return spread_sub(IntConst<2>{}, n, pa);
+    if constexpr (SPREAD && FIELD::kSpreadSub > 3) return spread_sub(IntConst<3>{}, n, pa);
     return 0.0f;
   };
 
