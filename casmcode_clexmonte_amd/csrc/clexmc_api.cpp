@@ -2712,11 +2712,21 @@ clexmc_status clexmc_read_samples(clexmc_handle *h, int *n_samples, double *E, i
   ARG_CHECK(want >= ns, "output arrays too small for the recorded samples");
   if (ns == 0) return CLEXMC_OK;
   // chains share a contiguous copy per kPackBytes of samples; a chain with
-  // more than half of that (700,000 samples) is copied from its own row
+  // more than half of that (700,000 samples), or without memory for the
+  // buffer, is copied from its own row
   static constexpr size_t kPackBytes = 32u << 20;
   const size_t per_chain = (sizeof(double) + kMaxOcc * sizeof(int)) * (size_t)ns;
   const int group = (int)std::min<size_t>((size_t)h->n_chains, kPackBytes / per_chain);
-  if (group <= 1) {
+  if (group > 1 && h->pack_bytes < per_chain * group) {
+    hipFree(h->d_pack);
+    h->d_pack = nullptr;
+    h->pack_bytes = hipMalloc(&h->d_pack, per_chain * group) == hipSuccess ? per_chain * group : 0;
+    if (h->pack_bytes == 0) {
+      h->d_pack = nullptr;
+      (void)hipGetLastError();
+    }
+  }
+  if (group <= 1 || h->pack_bytes == 0) {
     for (int c = 0; c < h->n_chains; ++c) {
       if (E)
         HIP_TRY(hipMemcpyAsync(E + (size_t)c * ns, h->d_sampE + (size_t)c * h->sample_cap, sizeof(double) * ns,
@@ -2727,13 +2737,6 @@ clexmc_status clexmc_read_samples(clexmc_handle *h, int *n_samples, double *E, i
     }
     HIP_TRY(hipStreamSynchronize(h->stream));
     return CLEXMC_OK;
-  }
-  if (h->pack_bytes < per_chain * group) {
-    hipFree(h->d_pack);
-    h->d_pack = nullptr;
-    h->pack_bytes = 0;
-    HIP_TRY(hipMalloc(&h->d_pack, per_chain * group));
-    h->pack_bytes = per_chain * group;
   }
   for (int c0 = 0; c0 < h->n_chains; c0 += group) {
     const int nc = std::min(group, h->n_chains - c0);
