@@ -362,7 +362,6 @@ __global__ __launch_bounds__(1024) void learned_kernel(RunArgs args, LearnArgs l
   // `draw` is the counter of this wavefront's stream
   const int n_str = la.stream_threads >> 6;  // streams; two wavefronts each
   const int str = wave_u % n_str;
-  const int stream_tid = tid < la.stream_threads ? tid : tid - la.stream_threads;
 
   int accC[kMaxSlots];
 #pragma unroll
@@ -542,13 +541,15 @@ __global__ __launch_bounds__(1024) void learned_kernel(RunArgs args, LearnArgs l
                           (uint32_t)sc->n_pair_phases;
       const int pb = sc->pair_begin[ph], pe = sc->pair_begin[ph + 1];
       // (the pairs of a phase share no cluster: the threads of both halves
-      // take one each, with the words of thread tid mod stream_threads)
+      // take one each.  A pair's word is its own: the counter is the pair's
+      // place in the phase and the draw of the wavefront's stream.  Two pairs
+      // on one word would be accepted together more often than apart)
       for (int t = pb + tid; t < pe; t += nthr) {
         const int2 pq = sc->pair_addr[t];
         const int bpq = sc->pair_sublat[t];
         const int op = img[pq.x], oq = img[pq.y];
         if (op == oq) continue;
-        const uint4 ur = philox4x32_10(make_uint4((uint32_t)stream_tid, (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
+        const uint4 ur = philox4x32_10(make_uint4((uint32_t)(t - pb), (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
                                                  (uint32_t)chain), k0, k1);
         int Kp[kMaxSlots], Kq[kMaxSlots];
         const float Fp = binary_field_l(img, pq.x, op, cst(sc->bin_sub + (bpq & 0xFF)), bin_off, n_slots, Kp);
