@@ -44,6 +44,8 @@ struct HostSupercell {
   int jit_spread_state[2] = {};
   hipFunction_t jit_spread[2] = {};
   hipFunction_t jit_nfold = nullptr;  // N-fold kernel of the SGC (unpacked, one-lane) module
+  int jit_nfold_single_state = 0;     // the one for blocks of one wavefront, a module of its own
+  hipFunction_t jit_nfold_single = nullptr;
   hipFunction_t jit_cube[2] = {nullptr, nullptr};  // register-cube kernel of that module [block above 512]
   // register-cube sweep (binary, one sublattice, classes = the residues of
   // the cells mod 3 listed in block order): eligible, and its layout
@@ -1564,6 +1566,7 @@ clexmc_status clexmc_set_lds_row_pitch(clexmc_handle *h, int extra) {
 
 static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads,
                                 bool spread = false);
+static hipFunction_t jit_nfold_single(clexmc_handle *h, int sc_id);
 
 // Chains whose N-fold run stopped because their total rate vanished: the
 // flags are cleared and the run reported as failed (its blocks past the stop
@@ -1588,6 +1591,44 @@ static clexmc_status nfold_check_stalls(clexmc_handle *h) {
 
 static clexmc_status grow_samples(clexmc_handle *h, long long n_new_samples);
 
+// Threads of an N-fold block: those that make the events (asked for, or 256 or
+// 128) and the wavefront that keeps the books, or one wavefront for both (64).
+// A chain alone is fastest with the most threads, but a compute unit holds two
+// blocks of 256 + 64 threads at once (general expansions: one, they take more
+// registers), five (four) of 128 + 64 and twelve of one wavefront, fewer where
+// the LDS ends first.  So 256 as long as all chains run at once, then 128
+// where it takes no more turns than one wavefront does.  200 events, ms with
+// 256 + 64, 128 + 64, 64 + 64 and 64 threads (one block of 64 threads per chain
+// before there was a wavefront for the books, in brackets):
+//   FCC 12^3    512 chains   0.73   0.80   0.93   0.99  (0.98)
+//   FCC 12^3  1,024          1.97   0.95   0.96   1.03  (1.02)
+//   FCC 12^3  2,048          3.33   1.84   1.42   1.29  (1.37)
+//   FCC  8^3  8,192         12.65   5.84   5.03   3.81  (4.73)
+//   HCP  8^3    256          2.31   2.39   2.49   2.74  (2.73)
+//   HCP  8^3  1,024          9.12   3.92   3.86   4.59  (4.68)
+//   BCC  8^3  2,048         23.54  14.59  16.90  12.03 (16.11)
+//
+// The kernel that is not specialised reads a general expansion's programs from
+// memory for every rate: its time is that of the turns its threads take over
+// the neighbour list, and a wavefront for the books only takes room.  So one
+// thread per list entry, up to 128, own books: BCC 8^3 (113 neighbours), 1,536
+// chains 46.5 ms (one wavefront 70.7), 768 chains 43.4 ms (128 + 64: 46.0).
+static int nfold_block(const clexmc_handle *h, size_t lds, int nb_max, bool specialized, bool *own_books) {
+  *own_books = false;
+  if (h->nfold_threads > 0) return h->nfold_threads + 64;
+  if (!specialized && !h->binary) {
+    *own_books = true;
+    return nb_max > 64 ? 128 : 64;
+  }
+  const int n_cu = std::max(1, h->n_cu), fit = std::max(1, (int)((size_t)h->max_lds / lds));
+  const int want = (h->n_chains + n_cu - 1) / n_cu;
+  auto turns = [&](int resident) { return (want + std::min(fit, resident) - 1) / std::min(fit, resident); };
+  if (std::min(want, fit) <= (h->binary ? 2 : 1)) return 256 + 64;
+  if (turns(h->binary ? 5 : 4) <= turns(4 * kNfoldSingleWaves)) return 128 + 64;
+  *own_books = true;
+  return 64;
+}
+
 // The N-fold run; blocks_out receives kNfoldBlockSums moments per block.
 static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_per_block, double *blocks_out,
                                     int n_time_samples = 0, double sample_dt = 0.0) {
@@ -1598,7 +1639,9 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
   if (n_events == 0) return CLEXMC_OK;
   HIP_TRY(hipSetDevice(h->device));
   int max_pad = 0, max_sites = 0, nb_max = 1, nb_total = 1;
+  bool one_shape = true;
   for (int c = 0; c < h->n_chains; ++c) {
+    one_shape = one_shape && h->chain_sc[c] == h->chain_sc[0];
     const HostSupercell &hs = h->scs[h->chain_sc[c]];
     const DevSupercell &d = hs.dev;
     max_pad = std::max(max_pad, d.pad_bytes);
@@ -1609,11 +1652,6 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
   ARG_CHECK(max_sites <= 262144, "the N-fold kernel takes supercells of at most 262,144 sites");
   ARG_CHECK(h->n_mswaps == 0, "the N-fold kernel's events are single-site changes: clear the multiswaps");
   const size_t lds = nfold_lds_bytes(max_pad, max_sites, nb_max, nb_total, h->n_sublat);
-  // threads that make the events, and the wavefront that keeps the books.
-  // Automatic: 256, so that the group sums (four lanes per changed rate) take
-  // one turn; 1,000 events of 256 FCC 24^3 chains: 3.26 ms, 3.63 ms with 128,
-  // 4.16 ms with 64
-  const int nf_threads = (h->nfold_threads > 0 ? h->nfold_threads : 256) + 64;
   ARG_CHECK(lds <= 160 * 1024, "supercell too large for the N-fold kernel's LDS (image + one rate per site)");
   NfoldArgs na;
   memset(&na, 0, sizeof(na));
@@ -1647,13 +1685,13 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
   // every chain on one supercell: the run-time specialised N-fold kernel
   // (constant site-program offsets), else the generic one
   hipFunction_t jf = nullptr;
-  if (h->specialize) {
-    bool one_shape = true;
-    for (int c = 1; c < h->n_chains; ++c) one_shape = one_shape && h->chain_sc[c] == h->chain_sc[0];
-    if (one_shape) {
-      (void)jit_kernel(h, h->chain_sc[0], 1, false, 1, kAotMaxThreads);
-      jf = h->scs[h->chain_sc[0]].jit_nfold;
-    }
+  bool own_books = false;
+  int nf_threads = nfold_block(h, lds, nb_max, h->specialize && one_shape, &own_books);
+  if (h->specialize && one_shape && own_books) {
+    jf = jit_nfold_single(h, h->chain_sc[0]);
+  } else if (h->specialize && one_shape) {
+    (void)jit_kernel(h, h->chain_sc[0], 1, false, 1, kAotMaxThreads);
+    jf = h->scs[h->chain_sc[0]].jit_nfold;
   }
   hipError_t e = hipMemsetAsync(d_blocks, 0, nb * sizeof(double), h->stream);
   h->last_specialized = 0;
@@ -1670,7 +1708,10 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
       jf = nullptr;
     }
   }
-  if (e == hipSuccess && !jf) e = launch_nfold(na, h->binary != 0, h->n_chains, nf_threads, lds, h->stream);
+  if (!jf) nf_threads = nfold_block(h, lds, nb_max, false, &own_books);
+  h->last_threads = nf_threads;
+  if (e == hipSuccess && !jf)
+    e = launch_nfold(na, h->binary != 0, h->n_chains, nf_threads, own_books, lds, h->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(blocks_out, d_blocks, nb * sizeof(double), hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   hipFree(d_blocks);
@@ -1824,6 +1865,28 @@ static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool pack
     }
   }
   return state == 1 ? fn : nullptr;
+}
+
+// The specialised one-wavefront N-fold kernel of a supercell, compiled on first use.
+static hipFunction_t jit_nfold_single(clexmc_handle *h, int sc_id) {
+  HostSupercell &hs = h->scs[sc_id];
+  if (hs.jit_nfold_single_state == 0) {
+    hs.jit_nfold_single_state = -1;
+    std::vector<int> variable(h->n_sublat);
+    for (int b = 0; b < h->n_sublat; ++b) variable[b] = h->n_occ[b] >= 2;
+    hipModule_t mod = nullptr;
+    if (jit_compile_load(jit_source_nfold_single(h->n_sublat, variable, h->binary != 0, hs.bin_sub, hs.bin_off,
+                                                 h->n_slots, hs.gen_sub, hs.gen_prog),
+                         &mod, &h->jit_log) == hipSuccess) {
+      hs.jit_mods.push_back(mod);
+      if (hipModuleGetFunction(&hs.jit_nfold_single, mod, kJitNfoldSingleName) == hipSuccess)
+        hs.jit_nfold_single_state = 1;
+      else
+        hs.jit_nfold_single = nullptr;
+    }
+    if (hs.jit_nfold_single_state < 0) (void)hipGetLastError();
+  }
+  return hs.jit_nfold_single;
 }
 
 // Sample storage for n_new_samples more samples per chain.  The count in use

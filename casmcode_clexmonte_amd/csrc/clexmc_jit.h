@@ -41,6 +41,11 @@ std::string jit_source(int n_sublat, const std::vector<int> &variable, bool bina
                        const std::vector<int> &gen_prog, int kind, bool packed, int lanes, int max_threads,
                        const CubeSpec *cube = nullptr, bool spread = false);
 
+// The N-fold kernel for blocks of one wavefront (nfold_body, OWN_BOOKS).
+std::string jit_source_nfold_single(int n_sublat, const std::vector<int> &variable, bool binary,
+                                    const std::vector<BinSub> &subs, const std::vector<int> &bin_off, int n_slots,
+                                    const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog);
+
 // Table rows that each lane of a wavefront forms per site in the spread kernel
 // (the largest program of a variable sublattice, over 64 lanes); 0 where its
 // descriptors cannot hold the programs (clusters of more than three other
@@ -76,6 +81,7 @@ constexpr const char *kJitCubeName = "clexmc_jit_s_u8_cube";
 // The N-fold kernel in the module of the semi-grand canonical, unpacked,
 // one-lane variant.
 constexpr const char *kJitNfoldName = "clexmc_jit_nfold";
+constexpr const char *kJitNfoldSingleName = "clexmc_jit_nfold_single";  // one wavefront, its own books
 
 // Compiles `src` (hipRTC, gfx950) and loads it as a module; code objects are
 // cached per source text for the life of the process.

@@ -141,6 +141,8 @@ constexpr int kNfoldNbBeginBytes = ((kMaxSublat + 1) * 4 + 15) & ~15;
 // threads of the largest N-fold block: 256 that make the events and a
 // wavefront that keeps the books
 constexpr int kNfoldMaxThreads = 256 + 64;
+// wavefronts per SIMD that the registers of the one-wavefront N-fold kernel allow
+constexpr int kNfoldSingleWaves = 3;
 // LDS bytes of the current event's record (16 words and the total rate)
 constexpr int kNfoldSelBytes = 16 * 4 + 16;
 struct NfoldArgs {
@@ -195,7 +197,9 @@ hipError_t launch_philox(int n, const uint4 *ctr, const uint2 *key, uint4 *out, 
 // further LDS of a canonical launch that keeps the occupants of a class side by side
 inline size_t class_occ_bytes(int max_class) { return (size_t)((max_class + 15) & ~15); }
 size_t metropolis_lds_bytes(int pad_sites, int n_tab, bool binary, int n_func_max, int max_class, bool packed);
-hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st);
+// own_books: no wavefront for the books alone, at most 128 threads
+hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, bool own_books, size_t lds,
+                        hipStream_t st);
 // nb_total: neighbour-list entries of the supercell, all sublattices
 size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total, int n_sublat);
 

@@ -22,8 +22,8 @@
 //    recompute the rates of the site and of its interaction neighbours (each
 //    neighbour once), and the sum of every group holding one of them is
 //    formed again from its 64 rates, four lanes per group;
-//  * meanwhile one lane of the last wavefront weights the state the event
-//    leaves by its expected residence time w = n_mutable / R in Metropolis
+//  * meanwhile one lane of the last wavefront (OWN_BOOKS: afterwards one lane
+//    of the first) weights the state the event leaves by its expected residence time w = n_mutable / R in Metropolis
 //    steps (the jump chain visits states in proportion to pi(x) R(x); weights
 //    1/R recover pi) and keeps the counts (binary: exact integer cluster
 //    counts, general: FP64 energy).
@@ -109,6 +109,21 @@ __device__ __forceinline__ double group_rate_sum(const float *rate, int g, int q
   a += dpp_d<0xB1, 0xf>(a);
   return a + dpp_d<0x4E, 0xf>(a);
 }
+// the same sum, bit for bit, in one lane (in one or two wavefronts four lanes
+// per group would take four times the turns)
+__device__ __forceinline__ double group_rate_sum_lane(const float *rate, int g) {
+  const float4 *r = (const float4 *)(rate + g * 64);
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+#pragma unroll
+  for (int p = 0; p < 16; ++p) {
+    const float4 v = r[p ^ (g & 15)];
+    a0 += (double)v.x;
+    a1 += (double)v.y;
+    a2 += (double)v.z;
+    a3 += (double)v.w;
+  }
+  return (a0 + a1) + (a2 + a3);
+}
 
 // x / d for 0 <= x < 2^18 and 1 <= d < 2^14 or d > x, by one high product (on
 // the scalar unit for a uniform x): m = floor(2^32 / d) + 1 exceeds 2^32 / d
@@ -120,7 +135,140 @@ __device__ __forceinline__ int div_small(int x, uint32_t m) { return m ? (int)__
 // smallest total rate a chain may reach before it stops with an error
 constexpr double kNfoldMinTotalRate = 1e-30;
 
-template <bool BIN, class FIELD>
+// The books of a chain, kept by one lane: the energy and occupant counts of the
+// state it is in, the moments of the current block and the time samples.
+template <bool BIN>
+struct NfoldBooks {
+  long long C[kMaxSlots];        // binary: cluster-count changes per slot
+  long long cnt[kMaxOcc], n_done;
+  double E_run;                  // general: running energy
+  double mom[kNfoldBlockSums];   // residence-weighted moments (kNfoldBlockSums layout)
+  double n_mutable, T_now;
+  // binary: the weight of each slot's orbit, read once (the energy of a state
+  // is formed at every event), and the energy of the exact counts at launch
+  double wslot[kMaxSlots], E0;
+  int s_base, n_rec;
+
+  __device__ __forceinline__ void open(const NfoldArgs &na, cptr<DevSystem> sys, const ChainState *cs, int chain,
+                                       int n_cells) {
+    const RunArgs &args = na.a;
+#pragma unroll
+    for (int q = 0; q < kMaxOcc; ++q) cnt[q] = cs->counts[q];
+    E_run = cs->E;
+#pragma unroll
+    for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
+    n_done = 0;
+    n_mutable = 0.0;
+    for (int b = 0; b < sys->n_sublat; ++b)
+      if (sys->n_occ[b] >= 2) n_mutable += (double)n_cells;
+#pragma unroll
+    for (int j = 0; j < kMaxSlots; ++j) {
+      C[j] = 0;
+      wslot[j] = (BIN && j < sys->n_slots) ? sys->bin_w64[sys->slot_orbit[j]] : 0.0;
+    }
+    E0 = 0.0;
+    if (BIN) {
+      const long long *C0 = args.binC + (long long)chain * args.n_orbits;
+      for (int a = 0; a < args.n_orbits; ++a) E0 += sys->bin_w64[a] * (double)C0[a];
+    }
+    // (the sample storage is only passed in for time sampling)
+    s_base = na.n_time_samples > 0 ? args.sample_count[chain] : 0;
+    T_now = 0.0;
+    n_rec = 0;
+  }
+
+  // The state the event leaves, weighted by its expected Metropolis steps (R:
+  // its total rate); true: time sampling has taken every sample.
+  __device__ __forceinline__ bool leave(const NfoldArgs &na, int chain, int n_slots, double R) {
+    const RunArgs &args = na.a;
+    double E = E0;
+    if (BIN) {
+#pragma unroll
+      for (int j = 0; j < kMaxSlots; ++j)
+        if (j < n_slots) E += wslot[j] * (double)C[j];
+    } else {
+      E = E_run;
+    }
+    const double w = n_mutable / R;
+    // every sample time in this state's residence interval
+    // [T, T + w / n_mutable) (in passes) samples it
+    if (na.n_time_samples > 0) {
+      const double t1 = T_now + w / n_mutable;
+      while (n_rec < na.n_time_samples && (double)n_rec * na.sample_dt < t1) {
+        const long long so = (long long)chain * args.sample_cap + (s_base + n_rec);
+        args.sampE[so] = E;
+#pragma unroll
+        for (int q = 0; q < kMaxOcc; ++q) args.sampN[so * kMaxOcc + q] = (int)cnt[q];
+        ++n_rec;
+      }
+      T_now = t1;
+    }
+    mom[0] += w;
+    mom[1] += w * E;
+    mom[2] += w * E * E;
+    int t = 0;
+#pragma unroll
+    for (int o = 0; o < kMaxOcc; ++o) {
+      const double wn = w * (double)cnt[o];
+      mom[3 + o] += wn;
+      mom[17 + o] += wn * E;
+#pragma unroll
+      for (int q = o; q < kMaxOcc; ++q, ++t) mom[7 + t] += wn * (double)cnt[q];
+    }
+    return na.n_time_samples > 0 && n_rec >= na.n_time_samples;
+  }
+
+  // Event `ev` has been applied; sel: its record.
+  __device__ __forceinline__ void applied(const NfoldArgs &na, int chain, int ev, const int *sel) {
+    const int o = sel[4], nw = sel[5];
+    if (BIN) {
+      const int sk = o ? -2 : 2;
+#pragma unroll
+      for (int a = 0; a < kMaxSlots; ++a) C[a] += (long long)sk * sel[8 + a];
+    } else {
+      E_run += (double)__int_as_float(sel[6]);
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxOcc; ++q) cnt[q] += (q == nw ? 1 : 0) - (q == o ? 1 : 0);
+    ++n_done;
+    if ((ev + 1) % na.events_per_block == 0) {
+      const int blk = (ev + 1) / na.events_per_block - 1;
+      if (blk < na.n_blocks) {
+        double *out = na.blocks + ((long long)chain * na.n_blocks + blk) * kNfoldBlockSums;
+#pragma unroll
+        for (int q = 0; q < kNfoldBlockSums; ++q) out[q] = mom[q];
+      }
+#pragma unroll
+      for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
+    }
+  }
+
+  __device__ __forceinline__ void close(const NfoldArgs &na, cptr<DevSystem> sys, ChainState *cs, int chain,
+                                        int n_slots, unsigned long long ev0) const {
+    const RunArgs &args = na.a;
+    if (BIN) {
+      long long *Cg = args.binC + (long long)chain * args.n_orbits;
+#pragma unroll
+      for (int j = 0; j < kMaxSlots; ++j)
+        if (j < n_slots) Cg[sys->slot_orbit[j]] += C[j];
+      double E = 0.0;
+      for (int a = 0; a < args.n_orbits; ++a) E += sys->bin_w64[a] * (double)Cg[a];
+      cs->E = E;
+    } else {
+      cs->E = E_run;
+    }
+#pragma unroll
+    for (int q = 0; q < kMaxOcc; ++q) cs->counts[q] = cnt[q];
+    if (na.n_time_samples > 0) args.sample_count[chain] = s_base + n_rec;
+    cs->n_attempt += n_done;
+    cs->n_accept += n_done;
+    cs->pass_base = ev0 + (unsigned long long)na.n_events;
+  }
+};
+
+// OWN_BOOKS: the first wavefront keeps the books as well, after each event,
+// instead of a wavefront of their own (many chains per compute unit).
+template <bool BIN, class FIELD, bool OWN_BOOKS = false>
 __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   extern __shared__ __align__(16) unsigned char smem[];
   const RunArgs &args = na.a;
@@ -264,77 +412,17 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   // The event's record (sel[4..15]) stands until the next flip, after the next
   // A, so the books take it in while the next event is being chosen.
   auto list_in_first_wave = [&](int sb) { return distinct && nbB[sb + 1] - nbB[sb] <= 64; };
-  if (wave == n_waves - 1) {
-    long long C[kMaxSlots] = {0, 0, 0, 0, 0, 0, 0, 0};  // binary: cluster-count changes per slot
-    long long cnt[kMaxOcc];
-    for (int q = 0; q < kMaxOcc; ++q) cnt[q] = cs->counts[q];
-    double E_run = cs->E;  // general: running energy
-    // residence-weighted moments of the current block (kNfoldBlockSums layout)
-    double mom[kNfoldBlockSums];
-#pragma unroll
-    for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
-    long long n_done = 0;
-    double n_mutable = 0.0;
-    for (int b = 0; b < sys->n_sublat; ++b)
-      if (sys->n_occ[b] >= 2) n_mutable += (double)n_cells;
-    // binary: the weight of each slot's orbit, read once (the energy of a
-    // state is formed at every event)
-    double wslot[kMaxSlots];
-#pragma unroll
-    for (int j = 0; j < kMaxSlots; ++j) wslot[j] = (BIN && j < n_slots) ? sys->bin_w64[sys->slot_orbit[j]] : 0.0;
-    double E0 = 0.0;  // binary: energy of the exact counts at launch
-    if (BIN) {
-      const long long *C0 = args.binC + (long long)chain * args.n_orbits;
-      for (int a = 0; a < args.n_orbits; ++a) E0 += sys->bin_w64[a] * (double)C0[a];
-    }
-    // (the sample storage is only passed in for time sampling)
-    const int s_base = n_tsamp > 0 ? args.sample_count[chain] : 0;
-    double T_now = 0.0;
-    int n_rec = 0;
+  if (!OWN_BOOKS && wave == n_waves - 1) {
+    NfoldBooks<BIN> books;
+    books.open(na, sys, cs, chain, n_cells);
     for (int ev = 0; ev < na.n_events; ++ev) {
       __syncthreads();  // A
       const int site = __builtin_amdgcn_readfirstlane(sel[0]);
       if (site < 0) break;
-      // the state the event leaves, weighted by its expected Metropolis steps;
-      // in time sampling before the event is applied
+      // in time sampling the state is left before the event is applied
       for (int turn = 0; turn < 2; ++turn) {
-        if (lane == 0 && turn == (n_tsamp > 0 ? 0 : 1)) {
-          double E = E0;
-          if (BIN) {
-#pragma unroll
-            for (int j = 0; j < kMaxSlots; ++j)
-              if (j < n_slots) E += wslot[j] * (double)C[j];
-          } else {
-            E = E_run;
-          }
-          const double w = n_mutable / *selR;
-          // every sample time in this state's residence interval
-          // [T, T + w / n_mutable) (in passes) samples it
-          if (n_tsamp > 0) {
-            const double t1 = T_now + w / n_mutable;
-            while (n_rec < n_tsamp && (double)n_rec * na.sample_dt < t1) {
-              const long long so = (long long)chain * args.sample_cap + (s_base + n_rec);
-              args.sampE[so] = E;
-#pragma unroll
-              for (int q = 0; q < kMaxOcc; ++q) args.sampN[so * kMaxOcc + q] = (int)cnt[q];
-              ++n_rec;
-            }
-            T_now = t1;
-            if (n_rec >= n_tsamp) sel[3] = 1;  // every sample taken: stop before this event
-          }
-          mom[0] += w;
-          mom[1] += w * E;
-          mom[2] += w * E * E;
-          int t = 0;
-#pragma unroll
-          for (int o = 0; o < kMaxOcc; ++o) {
-            const double wn = w * (double)cnt[o];
-            mom[3 + o] += wn;
-            mom[17 + o] += wn * E;
-#pragma unroll
-            for (int q = o; q < kMaxOcc; ++q, ++t) mom[7 + t] += wn * (double)cnt[q];
-          }
-        }
+        if (lane == 0 && turn == (n_tsamp > 0 ? 0 : 1))
+          if (books.leave(na, chain, n_slots, *selR)) sel[3] = 1;  // stop before this event
         if (turn == 0) {
           if (n_tsamp > 0) __syncthreads();  // T
           if (n_tsamp > 0 && __builtin_amdgcn_readfirstlane(sel[3])) break;
@@ -344,48 +432,13 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
       if (n_tsamp > 0 && __builtin_amdgcn_readfirstlane(sel[3])) break;  // (uniform across the workgroup)
       __syncthreads();  // C
       __syncthreads();  // D
-      if (lane == 0) {
-        const int o = sel[4], nw = sel[5];
-        if (BIN) {
-          const int sk = o ? -2 : 2;
-#pragma unroll
-          for (int a = 0; a < kMaxSlots; ++a) C[a] += (long long)sk * sel[8 + a];
-        } else {
-          E_run += (double)__int_as_float(sel[6]);
-        }
-#pragma unroll
-        for (int q = 0; q < kMaxOcc; ++q) cnt[q] += (q == nw ? 1 : 0) - (q == o ? 1 : 0);
-        ++n_done;
-        if ((ev + 1) % na.events_per_block == 0) {
-          const int blk = (ev + 1) / na.events_per_block - 1;
-          if (blk < na.n_blocks) {
-            double *out = na.blocks + ((long long)chain * na.n_blocks + blk) * kNfoldBlockSums;
-#pragma unroll
-            for (int q = 0; q < kNfoldBlockSums; ++q) out[q] = mom[q];
-          }
-#pragma unroll
-          for (int q = 0; q < kNfoldBlockSums; ++q) mom[q] = 0.0;
-        }
-      }
+      if (lane == 0) books.applied(na, chain, ev, sel);
     }
-    if (lane == 0) {
-      if (BIN) {
-        long long *Cg = args.binC + (long long)chain * args.n_orbits;
-        for (int j = 0; j < n_slots; ++j) Cg[sys->slot_orbit[j]] += C[j];
-        double E = 0.0;
-        for (int a = 0; a < args.n_orbits; ++a) E += sys->bin_w64[a] * (double)Cg[a];
-        cs->E = E;
-      } else {
-        cs->E = E_run;
-      }
-      for (int q = 0; q < kMaxOcc; ++q) cs->counts[q] = cnt[q];
-      if (n_tsamp > 0) args.sample_count[chain] = s_base + n_rec;
-      cs->n_attempt += n_done;
-      cs->n_accept += n_done;
-      cs->pass_base = ev0 + (unsigned long long)na.n_events;
-    }
+    if (lane == 0) books.close(na, sys, cs, chain, n_slots, ev0);
   } else {
-    const int n_work = nthr - 64;  // threads that make the events
+    const int n_work = OWN_BOOKS ? nthr : nthr - 64;  // threads that make the events
+    NfoldBooks<BIN> books;
+    if (OWN_BOOKS && wave == 0) books.open(na, sys, cs, chain, n_cells);
     // this lane's periodic copy in a flip: shift 0, +1 or -1 period per axis
     const int cpk = lane / 9, cpj = (lane / 3) % 3, cpi = lane % 3;
     const bool near = h <= L1 && h <= L2 && h <= L3;  // a coordinate wraps by one period at most
@@ -467,6 +520,8 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
         break;
       }
       if (n_tsamp > 0) {
+        if (OWN_BOOKS && tid == 0)
+          if (books.leave(na, chain, n_slots, *selR)) sel[3] = 1;
         __syncthreads();  // T
         if (__builtin_amdgcn_readfirstlane(sel[3])) break;  // time sampling complete (uniform across the workgroup)
       }
@@ -594,6 +649,12 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
         // the groups of the changed rates, summed again from their 64 rates by
         // four lanes each (several quads may form one group's sum: they write
         // the same value)
+        if constexpr (OWN_BOOKS) {
+          for (int t = tid; t < nb1 - nb0; t += n_work) {
+            const int g = aff[t] >> 6;
+            G[g] = group_rate_sum_lane(rate, g);
+          }
+        } else
         for (int w = tid; w < 4 * (nb1 - nb0); w += n_work) {
           const int g = aff[w >> 2] >> 6;
           const double s = group_rate_sum(rate, g, w & 3);
@@ -601,7 +662,12 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
         }
         __syncthreads();  // D
       }
+      if (OWN_BOOKS && tid == 0) {
+        if (n_tsamp == 0) (void)books.leave(na, chain, n_slots, *selR);
+        books.applied(na, chain, ev, sel);
+      }
     }
+    if (OWN_BOOKS && tid == 0) books.close(na, sys, cs, chain, n_slots, ev0);
   }
 
   // ---- write back: occupation, exact counts, energy, counters

@@ -19,14 +19,18 @@ __global__ __launch_bounds__(kNfoldMaxThreads) void nfold_kernel(NfoldArgs na) {
   nfold_body<BIN, GenericField>(na);
 }
 
-hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, size_t lds, hipStream_t st) {
-  const void *fn = binary ? (const void *)nfold_kernel<true> : (const void *)nfold_kernel<false>;
-  hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+template <bool BIN>
+__global__ __launch_bounds__(128, kNfoldSingleWaves) void nfold_own_books_kernel(NfoldArgs na) {
+  nfold_body<BIN, GenericField, true>(na);
+}
+
+hipError_t launch_nfold(const NfoldArgs &a, bool binary, int n_chains, int threads, bool own_books, size_t lds,
+                        hipStream_t st) {
+  void (*fn)(NfoldArgs) = own_books ? (binary ? nfold_own_books_kernel<true> : nfold_own_books_kernel<false>)
+                                    : (binary ? nfold_kernel<true> : nfold_kernel<false>);
+  hipError_t e = hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  if (binary)
-    hipLaunchKernelGGL(nfold_kernel<true>, dim3(n_chains), dim3(threads), lds, st, a);
-  else
-    hipLaunchKernelGGL(nfold_kernel<false>, dim3(n_chains), dim3(threads), lds, st, a);
+  hipLaunchKernelGGL(fn, dim3(n_chains), dim3(threads), lds, st, a);
   return hipGetLastError();
 }
 

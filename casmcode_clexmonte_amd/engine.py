@@ -365,8 +365,8 @@ class Engine:
         self._check(lib().clexmc_set_block_size(self.h, C.c_int(threads)), "clexmc_set_block_size")
 
     def set_nfold_block_size(self, threads: int):
-        """Threads per chain that make the N-fold kernel's events: 64, 128,
-        256, or 0 (default) for 256."""
+        """Threads per chain that make the N-fold kernel's events: 64, 128 or
+        256, or 0 (default) to choose by the number of chains."""
         self._check(lib().clexmc_set_nfold_block_size(self.h, C.c_int(threads)), "clexmc_set_nfold_block_size")
 
     def read_samples(self):

@@ -243,11 +243,14 @@ clexmc_status clexmc_last_run_ms(clexmc_handle *h, double *ms);
 clexmc_status clexmc_set_block_size(clexmc_handle *h, int threads);
 
 /* Threads per chain that make the N-fold kernel's events (clexmc_nfold_run*):
- * 64, 128 or 256, or 0 (default) for 256; one more wavefront keeps the
- * chain's books.  An event's select and flip run in the first wavefront, its
- * neighbours' rates one per thread, the sums of the changed groups of rates
- * four threads each.  Results do not depend on it.  No counterpart in the reference
- * (its nfold loop, include/casm/clexmonte/nfold/nfold_impl.hh:18-98, runs
+ * 64, 128 or 256 and one more wavefront that keeps the chain's books, or 0
+ * (default) to choose by the number of chains: 256 while all of them run at
+ * once, 128 or one wavefront for events and books beyond.  An event's select
+ * and flip run in the first wavefront, its neighbours' rates one per thread,
+ * the sums of the changed groups of rates four threads each (one in the
+ * one-wavefront form).  Results do not depend on it.
+ * clexmc_last_run_info gives the block an N-fold run took, books included.
+ * No counterpart in the reference (its nfold loop, include/casm/clexmonte/nfold/nfold_impl.hh:18-98, runs
  * on one CPU thread). */
 clexmc_status clexmc_set_nfold_block_size(clexmc_handle *h, int threads);
 
