@@ -2047,6 +2047,7 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
   P.n_blocks = n_sel;
   P.la.mlp = h->d_mlp;
   P.la.rounds_per_group = h->rounds_per_group;
+  P.la.twice = n_sel <= h->n_cu ? 1 : 0;
   // specialised kernel when every chain uses the same supercell
   P.jit = nullptr;
   {

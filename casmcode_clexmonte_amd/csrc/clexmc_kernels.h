@@ -93,6 +93,7 @@ struct LearnArgs {
   const MlpDev *mlp;
   int rounds_per_group;
   int stream_threads;  // threads whose random streams the chain uses (set by launch_learned)
+  int twice;           // twice as many threads in the launch
 };
 
 struct CollectArgs {

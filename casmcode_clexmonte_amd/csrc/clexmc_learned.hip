@@ -290,16 +290,28 @@ __device__ __forceinline__ float binary_field_l(const uint8_t *img, int pa, int 
 // Grouped-proposal Metropolis kernel (binary path).  KIND 0 canonical, 1 SGC;
 // WEIGHTS 0 uniform, 1 learned network, 2 informed (exact Barker weights).
 // ---------------------------------------------------------------------------
-// The launch has twice the threads of the chain's random streams
-// (la.stream_threads: the block size asked for): wavefront w draws from stream
+// The launch has the threads of the chain's random streams (la.stream_threads:
+// the block size asked for) or twice as many: wavefront w draws from stream
 // w mod (stream_threads / 64), whose groups are the same ones with either
 // count, so the results do not depend on it.  A group is a chain of dependent
 // shuffles, scans and ballots (half of all wave cycles waited with 8
-// wavefronts per chain).  128 chains of FCC 32^3, 16 rounds, 4 passes: 7.5 ms;
-// 5.5 ms with twice the wavefronts and DPP in place of most shuffles, 4.5 ms
-// with both halves in the pair phases and the inputs built two to a word.
-template <int KIND, int WEIGHTS>
-__global__ __launch_bounds__(1024) void learned_kernel(RunArgs args, LearnArgs la) {
+// wavefronts per chain), so as long as every chain has a compute unit to
+// itself it takes twice the wavefronts; with more chains the further
+// wavefronts would keep other chains out.  4 passes of 128 chains of FCC 32^3,
+// 16 rounds: 7.5 ms before; 5.5 ms with twice the wavefronts and DPP in place
+// of most shuffles, 4.7 ms with both halves in the pair phases and the inputs
+// built two to a word.  2 passes, ms with twice and once the threads (before):
+//   FCC 32^3    256 chains   2.45   3.57  (3.88)
+//   FCC 24^3    256          1.72   1.72  (1.82)
+//   FCC 24^3    512          3.32   2.15  (2.33)
+//   FCC 32^3    512          4.74   4.57  (5.02)
+//   FCC 12^3  4,096          4.42   3.42  (3.74)
+// TWICE: the launch with twice the threads.  The other, for many chains, keeps
+// to the registers of 6 wavefronts per SIMD without the network, so that three
+// chains of 512 threads share a compute unit instead of two (768 chains of FCC
+// 24^3, informed: 2.52 ms, 2.11 ms so).
+template <int KIND, int WEIGHTS, bool TWICE>
+__global__ __launch_bounds__(TWICE ? 1024 : 512, TWICE || WEIGHTS == 1 ? 4 : 6) void learned_kernel(RunArgs args, LearnArgs la) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int chain = blockIdx.x;
   const int tid = threadIdx.x;
@@ -360,7 +372,7 @@ __global__ __launch_bounds__(1024) void learned_kernel(RunArgs args, LearnArgs l
          (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)draw);
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   // `draw` is the counter of this wavefront's stream
-  const int n_str = la.stream_threads >> 6;  // streams; two wavefronts each
+  const int n_str = la.stream_threads >> 6;  // streams, one or two wavefronts each
   const int str = wave_u % n_str;
 
   int accC[kMaxSlots];
@@ -1103,11 +1115,11 @@ __global__ void mlp_publish_kernel(const float *p, MlpDev *m, int n_env, float e
 template <int KIND, int WEIGHTS>
 static hipError_t launch_l(const RunArgs &args, const LearnArgs &la, int n_chains, int threads, size_t lds,
                            hipStream_t st, bool launch) {
-  auto kern = learned_kernel<KIND, WEIGHTS>;
+  auto kern = la.twice ? learned_kernel<KIND, WEIGHTS, true> : learned_kernel<KIND, WEIGHTS, false>;
   if (!launch) return hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   LearnArgs l2 = la;
   l2.stream_threads = threads;
-  hipLaunchKernelGGL(kern, dim3(n_chains), dim3(2 * threads), lds, st, args, l2);
+  hipLaunchKernelGGL(kern, dim3(n_chains), dim3(la.twice ? 2 * threads : threads), lds, st, args, l2);
   return hipGetLastError();
 }
 
