@@ -2775,31 +2775,37 @@ clexmc_status clexmc_read_samples(clexmc_handle *h, int *n_samples, double *E, i
   if (!E && !counts) return CLEXMC_OK;
   ARG_CHECK(want >= ns, "output arrays too small for the recorded samples");
   if (ns == 0) return CLEXMC_OK;
-  // chains share a contiguous copy per kPackBytes of samples; a chain with
-  // more than half of that (700,000 samples), or without memory for the
-  // buffer, is copied from its own row
+  // Short rows of several chains are put side by side on the device and copied
+  // at once, up to kPackBytes of them.  A row takes about 6 us to copy by
+  // itself; one large copy to pageable memory pins its pages instead.  Chains x
+  // samples, us row by row and at once: 3 x 500 87 and 64, 4 x 8,000 147 and 97,
+  // 16 x 16,000 582 and 455, 128 x 8,000 3,200 and 1,750; 2 x 500 72 and 73,
+  // 4 x 40,000 295 and 326, 32 x 40,000 2,077 and 2,294.  So long rows, and all
+  // but short ones of two or three chains, are copied one by one.
   static constexpr size_t kPackBytes = 32u << 20;
+  static constexpr int kPackSamples = 16384, kPackFewSamples = 512;
   const size_t per_chain = (sizeof(double) + kMaxOcc * sizeof(int)) * (size_t)ns;
   const int group = (int)std::min<size_t>((size_t)h->n_chains, kPackBytes / per_chain);
-  if (group > 1 && h->pack_bytes < per_chain * group) {
+  const bool side_by_side = group > 1 && ns <= (h->n_chains >= 4 ? kPackSamples : kPackFewSamples);
+  if (side_by_side && h->pack_bytes < per_chain * group) {
+    // (doubled: a program that reads as its samples grow does not allocate each time)
+    size_t bytes = 1u << 16;
+    while (bytes < per_chain * group) bytes *= 2;
     hipFree(h->d_pack);
     h->d_pack = nullptr;
-    h->pack_bytes = hipMalloc(&h->d_pack, per_chain * group) == hipSuccess ? per_chain * group : 0;
+    h->pack_bytes = hipMalloc(&h->d_pack, bytes) == hipSuccess ? bytes : 0;
     if (h->pack_bytes == 0) {
       h->d_pack = nullptr;
       (void)hipGetLastError();
     }
   }
-  if (group <= 1 || h->pack_bytes == 0) {
-    for (int c = 0; c < h->n_chains; ++c) {
-      if (E)
-        HIP_TRY(hipMemcpyAsync(E + (size_t)c * ns, h->d_sampE + (size_t)c * h->sample_cap, sizeof(double) * ns,
-                               hipMemcpyDeviceToHost, h->stream));
-      if (counts)
-        HIP_TRY(hipMemcpyAsync(counts + (size_t)c * ns * kMaxOcc, h->d_sampN + (size_t)c * h->sample_cap * kMaxOcc,
-                               sizeof(int) * kMaxOcc * ns, hipMemcpyDeviceToHost, h->stream));
-    }
-    HIP_TRY(hipStreamSynchronize(h->stream));
+  if (!side_by_side || h->pack_bytes == 0) {
+    if (E)
+      HIP_TRY(hipMemcpy2D(E, sizeof(double) * ns, h->d_sampE, sizeof(double) * h->sample_cap, sizeof(double) * ns,
+                          h->n_chains, hipMemcpyDeviceToHost));
+    if (counts)
+      HIP_TRY(hipMemcpy2D(counts, sizeof(int) * kMaxOcc * ns, h->d_sampN, sizeof(int) * kMaxOcc * h->sample_cap,
+                          sizeof(int) * kMaxOcc * ns, h->n_chains, hipMemcpyDeviceToHost));
     return CLEXMC_OK;
   }
   for (int c0 = 0; c0 < h->n_chains; c0 += group) {
