@@ -2800,12 +2800,15 @@ clexmc_status clexmc_read_samples(clexmc_handle *h, int *n_samples, double *E, i
     }
   }
   if (!side_by_side || h->pack_bytes == 0) {
+    // (on the handle's stream: a copy on the null stream would make the next
+    // free wait for that one too, 0.1 ms)
     if (E)
-      HIP_TRY(hipMemcpy2D(E, sizeof(double) * ns, h->d_sampE, sizeof(double) * h->sample_cap, sizeof(double) * ns,
-                          h->n_chains, hipMemcpyDeviceToHost));
+      HIP_TRY(hipMemcpy2DAsync(E, sizeof(double) * ns, h->d_sampE, sizeof(double) * h->sample_cap, sizeof(double) * ns,
+                               h->n_chains, hipMemcpyDeviceToHost, h->stream));
     if (counts)
-      HIP_TRY(hipMemcpy2D(counts, sizeof(int) * kMaxOcc * ns, h->d_sampN, sizeof(int) * kMaxOcc * h->sample_cap,
-                          sizeof(int) * kMaxOcc * ns, h->n_chains, hipMemcpyDeviceToHost));
+      HIP_TRY(hipMemcpy2DAsync(counts, sizeof(int) * kMaxOcc * ns, h->d_sampN, sizeof(int) * kMaxOcc * h->sample_cap,
+                               sizeof(int) * kMaxOcc * ns, h->n_chains, hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
     return CLEXMC_OK;
   }
   for (int c0 = 0; c0 < h->n_chains; c0 += group) {
