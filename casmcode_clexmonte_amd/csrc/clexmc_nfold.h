@@ -75,6 +75,15 @@ __device__ __forceinline__ double lane_d(double x, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// Orders the wavefront's LDS accesses: what any lane stored before, every lane
+// reads after.  (No instruction: a wavefront's LDS operations are in order; the
+// compiler must keep them so.)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // first lane whose inclusive prefix exceeds t; if rounding leaves none, the
 // last lane with a positive value (-1 if there is none)
 __device__ __forceinline__ int pick_lane(double incl, double v, double t) {
@@ -558,7 +567,7 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
           if (lane == 0) sel[6] = __float_as_int(general_dE(sys, b, o, nw, Gf));
         }
         // every lane has read the site before a copy of it is written
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         if (lane == 0) {
           sel[4] = o;
           sel[5] = nw;
@@ -589,6 +598,10 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
             }
           }
         }
+        // the copies, written by many lanes, are there for every lane of this
+        // wavefront (barrier B is for the others, and left out where only this
+        // one reads them)
+        wave_sync();
       }
       // ---- rates of the site and its interaction neighbours
       {
