@@ -1652,7 +1652,7 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
   ARG_CHECK(max_sites <= 262144, "the N-fold kernel takes supercells of at most 262,144 sites");
   ARG_CHECK(h->n_mswaps == 0, "the N-fold kernel's events are single-site changes: clear the multiswaps");
   const size_t lds = nfold_lds_bytes(max_pad, max_sites, nb_max, nb_total, h->n_sublat);
-  ARG_CHECK(lds <= 160 * 1024, "supercell too large for the N-fold kernel's LDS (image + one rate per site)");
+  ARG_CHECK(lds <= (size_t)kNfoldMaxLds, "supercell too large for the N-fold kernel's LDS (image + one rate per site)");
   NfoldArgs na;
   memset(&na, 0, sizeof(na));
   na.a.sys = h->d_sys;

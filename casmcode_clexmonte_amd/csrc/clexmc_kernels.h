@@ -144,6 +144,10 @@ constexpr int kNfoldNbBeginBytes = ((kMaxSublat + 1) * 4 + 15) & ~15;
 constexpr int kNfoldMaxThreads = 256 + 64;
 // wavefronts per SIMD that the registers of the one-wavefront N-fold kernel allow
 constexpr int kNfoldSingleWaves = 3;
+// LDS of an N-fold workgroup, at most.  With an image and four bytes per site in
+// it there are fewer than 2^15 sites and a halo of at most 26 cells, so that the
+// offsets of a neighbour fit a byte each.
+constexpr int kNfoldMaxLds = 160 * 1024;
 // LDS bytes of the current event's record (16 words and the total rate)
 constexpr int kNfoldSelBytes = 16 * 4 + 16;
 struct NfoldArgs {

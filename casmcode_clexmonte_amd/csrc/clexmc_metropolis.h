@@ -172,7 +172,7 @@ struct PadWalk {
 // selects; h and L are the same in every lane).  Bytes past L + 2h in a row
 // (the unused part of a padded row pitch) are clamped to a valid cell: their
 // image value is never read, but the global read of it must stay in bounds.
-__device__ __forceinline__ int pad_wrap(int q, int h, int L) {
+__host__ __device__ __forceinline__ int pad_wrap(int q, int h, int L) {
   int x = q - h;
   if (h <= L) {
     x = x < 0 ? x + L : x;

@@ -41,7 +41,41 @@
 
 namespace clexmc {
 
-__host__ __device__ inline size_t nfold_align16(size_t x) { return (x + 15) & ~(size_t)15; }
+// LDS of an N-fold workgroup: byte offsets behind the padded image
+struct NfoldLds {
+  size_t rate;   // [n_groups * 64] FP32 rates, zero past n_sites (rate_at)
+  size_t G;      // [n_groups] FP64 group sums
+  size_t aff;    // [nb_max] linear indices of the sites whose rates change
+  size_t affp;   // [nb_max] their padded addresses
+  size_t sel;    // the event's record (kNfoldSelBytes)
+  size_t nb_begin;  // [n_sublat + 1] starts of the neighbour lists
+  size_t nb;     // [nb_total] sublattice, di, dj, dk of a neighbour, a byte each
+  size_t n_occ;  // [n_sublat]
+  size_t chem;   // [n_sublat][kMaxOcc]
+  size_t bytes;
+};
+__host__ __device__ inline NfoldLds nfold_lds(int pad_sites, int n_sites, int nb_max, int nb_total, int n_sublat) {
+  auto up = [](size_t x) { return (x + 15) & ~(size_t)15; };
+  const size_t n_groups = (size_t)((n_sites + 63) / 64);
+  NfoldLds o;
+  o.rate = (size_t)image_bytes(pad_sites, false);
+  o.G = o.rate + n_groups * 64 * 4;
+  o.aff = o.G + up(n_groups * 8);
+  o.affp = o.aff + up((size_t)nb_max * 4);
+  o.sel = o.affp + up((size_t)nb_max * 4);
+  o.nb_begin = o.sel + kNfoldSelBytes;
+  o.nb = o.nb_begin + kNfoldNbBeginBytes;
+  o.n_occ = o.nb + up((size_t)nb_total * 4);
+  o.chem = o.n_occ + (size_t)n_sublat * 4;
+  o.bytes = o.chem + (size_t)n_sublat * kMaxOcc * 4;
+  return o;
+}
+__host__ __device__ inline uint32_t nfold_pack_nb(int b, int di, int dj, int dk) {
+  return (uint32_t)(b & 0xff) | (uint32_t)(di & 0xff) << 8 | (uint32_t)(dj & 0xff) << 16 | (uint32_t)(dk & 0xff) << 24;
+}
+__host__ __device__ inline int4 nfold_unpack_nb(uint32_t v) {
+  return make_int4((int)(v & 0xff), (int)(int8_t)(v >> 8), (int)(int8_t)(v >> 16), (int)v >> 24);
+}
 
 // x of the lane that DPP control CTRL names (0 where it names none, and in
 // the rows ROW_MASK leaves out), the two halves moved separately
@@ -102,7 +136,7 @@ __device__ __forceinline__ double u01_53(uint32_t a, uint32_t b) {
 // blocks of four are permuted by the group number, so that lanes that walk
 // different groups in step read different LDS banks (with plain rows every
 // group's block q lies in the same four banks: 860 conflict cycles per event)
-__device__ __forceinline__ int rate_at(int l) {
+__host__ __device__ __forceinline__ int rate_at(int l) {
   return (l & ~63) | ((((l >> 2) ^ (l >> 6)) & 15) << 2) | (l & 3);
 }
 
@@ -137,9 +171,53 @@ __device__ __forceinline__ double group_rate_sum_lane(const float *rate, int g) 
 // x / d for 0 <= x < 2^18 and 1 <= d < 2^14 or d > x, by one high product (on
 // the scalar unit for a uniform x): m = floor(2^32 / d) + 1 exceeds 2^32 / d
 // by at most 1, so x m / 2^32 exceeds x / d by less than 2^-14 < 1 / d (and
-// by less than 2^-14 below 1 for d > x); d = 1 has m = 0
-__device__ __forceinline__ uint32_t div_magic(int d) { return d > 1 ? (uint32_t)(4294967296ull / (uint32_t)d) + 1u : 0u; }
-__device__ __forceinline__ int div_small(int x, uint32_t m) { return m ? (int)__umulhi((uint32_t)x, m) : x; }
+// by less than 2^-14 below 1 for d > x); d = 1 has m = 0.  Fewer than 2^15
+// sites (kNfoldMaxLds) keep x and d there: a d of 2^14 or more is the cells of
+// the one sublattice, or an axis longer than the site's index.
+__host__ __device__ __forceinline__ uint32_t div_magic(int d) {
+  return d > 1 ? (uint32_t)(4294967296ull / (uint32_t)d) + 1u : 0u;
+}
+__host__ __device__ __forceinline__ int div_small(int x, uint32_t m) {
+  return m ? (int)(((unsigned long long)(uint32_t)x * m) >> 32) : x;
+}
+
+// The padded image of a supercell (cells of one sublattice after the other)
+struct NfoldShape {
+  int L1, L2, L3, h, P1, P12, S, n_cells;
+  bool near;  // h <= L on every axis: a coordinate wraps by one period at most
+};
+// Neighbour o (nfold_unpack_nb; offsets within the halo) of the site in cell
+// (i, j, k): its linear index and its address in the padded image.
+__host__ __device__ __forceinline__ void nfold_place(const NfoldShape &g, const int4 &o, int i, int j, int k, int &lt,
+                                                     int &pt) {
+  int it = i + o.y, jt = j + o.z, kt = k + o.w;
+  if (g.near) {
+    it += it < 0 ? g.L1 : 0;
+    jt += jt < 0 ? g.L2 : 0;
+    kt += kt < 0 ? g.L3 : 0;
+    it -= it >= g.L1 ? g.L1 : 0;
+    jt -= jt >= g.L2 ? g.L2 : 0;
+    kt -= kt >= g.L3 ? g.L3 : 0;
+  } else {
+    it = pad_wrap(it + g.h, g.h, g.L1);
+    jt = pad_wrap(jt + g.h, g.h, g.L2);
+    kt = pad_wrap(kt + g.h, g.h, g.L3);
+  }
+  lt = o.x * g.n_cells + it + g.L1 * (jt + g.L2 * kt);
+  pt = o.x * g.S + (kt + g.h) * g.P12 + (jt + g.h) * g.P1 + (it + g.h);
+}
+// Address a of a copy of the site in cell (i, j, k) of sublattice b, per axis
+// shifted by 0 (digit 0), +1 (1) or -1 (2) period, and whether the image has
+// such a copy (near shapes only).
+__host__ __device__ __forceinline__ bool nfold_copy(const NfoldShape &g, int cpi, int cpj, int cpk, int b, int i, int j,
+                                                   int k, int &a) {
+  const int qi = i + g.h + (cpi == 1 ? g.L1 : (cpi == 2 ? -g.L1 : 0)), qj = j + g.h + (cpj == 1 ? g.L2 : (cpj == 2 ? -g.L2 : 0)),
+            qk = k + g.h + (cpk == 1 ? g.L3 : (cpk == 2 ? -g.L3 : 0));
+  const bool vi = cpi == 0 || (cpi == 1 ? i < g.h : i >= g.L1 - g.h), vj = cpj == 0 || (cpj == 1 ? j < g.h : j >= g.L2 - g.h),
+             vk = cpk == 0 || (cpk == 1 ? k < g.h : k >= g.L3 - g.h);
+  a = b * g.S + qk * g.P12 + qj * g.P1 + qi;
+  return vi && vj && vk;
+}
 
 // smallest total rate a chain may reach before it stops with an error
 constexpr double kNfoldMinTotalRate = 1e-30;
@@ -300,33 +378,24 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
 
   ImgU8 img;
   img.p = (uint8_t *)smem;
-  size_t off = nfold_align16((size_t)image_bytes(pad_bytes, false));
-  float *rate = (float *)(smem + off);  // [n_groups * 64], zero past n_sites
-  off += nfold_align16((size_t)n_groups * 64 * 4);
-  double *G = (double *)(smem + off);   // [n_groups]
-  off += nfold_align16((size_t)n_groups * 8);
-  int *aff = (int *)(smem + off);    // linear indices of the sites whose rates change
-  off += nfold_align16((size_t)sc->nb_max * 4);
-  int *affp = (int *)(smem + off);   // their padded addresses
-  off += nfold_align16((size_t)sc->nb_max * 4);
+  const NfoldLds lds = nfold_lds(pad_bytes, n_sites, sc->nb_max, sc->nb_begin[sys->n_sublat], sys->n_sublat);
+  float *rate = (float *)(smem + lds.rate);
+  double *G = (double *)(smem + lds.G);
+  int *aff = (int *)(smem + lds.aff);
+  int *affp = (int *)(smem + lds.affp);
   // the event: [0] site (-2: stopped), [1], [2] random words, [3] time
   // sampling complete, [4], [5] old and new occupant, [6] energy change (FP32,
   // general), [8..] cluster sums of the flipped site, and the total rate
-  int *sel = (int *)(smem + off);
+  int *sel = (int *)(smem + lds.sel);
   double *selR = (double *)(sel + 16);
-  off += kNfoldSelBytes;
   // the interaction-neighbour offsets of every sublattice, staged once: an
   // event reads them right after its flip
-  int *nbB = (int *)(smem + off);     // [n_sublat + 1] list starts
-  off += kNfoldNbBeginBytes;
-  // sublattice, di, dj, dk of a neighbour, a byte each (an image that fits in
-  // LDS has a halo of at most 26 cells)
-  int *nbL = (int *)(smem + off);
-  off += nfold_align16((size_t)(sc->nb_begin[sys->n_sublat]) * 4);
+  int *nbB = (int *)(smem + lds.nb_begin);
+  uint32_t *nbL = (uint32_t *)(smem + lds.nb);
   // occupant counts and chemical potentials per sublattice: the rate of a
   // neighbour reads them for its sublattice (a per-lane index)
-  int *noccL = (int *)(smem + off);                 // [n_sublat]
-  float *chemL = (float *)(noccL + sys->n_sublat);  // [n_sublat][kMaxOcc]
+  int *noccL = (int *)(smem + lds.n_occ);
+  float *chemL = (float *)(smem + lds.chem);
 
   // ---- padded image, neighbour lists
   const int8_t *__restrict__ occG = args.occ + cp->occ_offset;
@@ -342,7 +411,7 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
     const int nb_tot = sc->nb_begin[n_sub];
     for (int t = tid; t < nb_tot; t += nthr) {
       const int4 o = sc->nb_cell[t];
-      nbL[t] = (o.x & 0xff) | (o.y & 0xff) << 8 | (o.z & 0xff) << 16 | (o.w & 0xff) << 24;
+      nbL[t] = nfold_pack_nb(o.x, o.y, o.z, o.w);
     }
     if (tid <= n_sub) nbB[tid] = sc->nb_begin[tid];
     if (tid < n_sub) noccL[tid] = sys->n_occ[tid];
@@ -350,11 +419,6 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
   }
   __syncthreads();
   const int P3 = S / P12;
-  auto neighbour = [&](int t) {
-    const int v = nbL[t];
-    return make_int4(v & 0xff, (int)(int8_t)(v >> 8), (int)(int8_t)(v >> 16), v >> 24);
-  };
-
   const float beta = cp->beta;
   cptr<int> bin_off = cst(sc->bin_off);
   auto main_addr = [&](int l) {
@@ -445,12 +509,12 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
     }
     if (lane == 0) books.close(na, sys, cs, chain, n_slots, ev0);
   } else {
+    const NfoldShape shape{L1, L2, L3, h, P1, P12, S, n_cells, h <= L1 && h <= L2 && h <= L3};
     const int n_work = OWN_BOOKS ? nthr : nthr - 64;  // threads that make the events
     NfoldBooks<BIN> books;
     if (OWN_BOOKS && wave == 0) books.open(na, sys, cs, chain, n_cells);
-    // this lane's periodic copy in a flip: shift 0, +1 or -1 period per axis
+    // this lane's periodic copy in a flip
     const int cpk = lane / 9, cpj = (lane / 3) % 3, cpi = lane % 3;
-    const bool near = h <= L1 && h <= L2 && h <= L3;  // a coordinate wraps by one period at most
     uint4 rv = make_uint4(0u, 0u, 0u, 0u);  // wavefront 0: the random words of events ev0 + 64 m + lane
     for (int ev = 0; ev < na.n_events; ++ev) {
       // ---- select an event (wavefront 0)
@@ -574,14 +638,11 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
         }
         // the site and every periodic copy of it in the padded image: padded
         // coordinate (i + h) + d L for every d that stays inside [0, L + 2h)
-        if (near) {
+        if (shape.near) {
           // d in {0, +1 (i < h), -1 (i >= L - h)}: at most three per axis, one
           // combination per lane
-          const int qi = ci + h + (cpi == 1 ? L1 : (cpi == 2 ? -L1 : 0)), qj = cj + h + (cpj == 1 ? L2 : (cpj == 2 ? -L2 : 0)),
-                    qk = ck + h + (cpk == 1 ? L3 : (cpk == 2 ? -L3 : 0));
-          const bool vi = cpi == 0 || (cpi == 1 ? ci < h : ci >= L1 - h), vj = cpj == 0 || (cpj == 1 ? cj < h : cj >= L2 - h),
-                     vk = cpk == 0 || (cpk == 1 ? ck < h : ck >= L3 - h);
-          if (lane < 27 && vi && vj && vk) img.p[b * S + qk * P12 + qj * P1 + qi] = (uint8_t)nw;
+          int copy;
+          if (nfold_copy(shape, cpi, cpj, cpk, b, ci, cj, ck, copy) && lane < 27) img.p[copy] = (uint8_t)nw;
         } else if (lane == 0) {
           const int m1 = (h + L1 - 1) / L1, m2 = (h + L2 - 1) / L2, m3 = (h + L3 - 1) / L3;
           for (int dk = -m3; dk <= m3; ++dk) {
@@ -605,31 +666,14 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
       }
       // ---- rates of the site and its interaction neighbours
       {
-        const int i = ci, j = cj, k = ck;
         const int nb0 = nbB[sb], nb1 = nbB[sb + 1];
-        // the neighbour o of the site: linear index and padded address
-        // (neighbour offsets are within the halo width h)
-        auto place = [&](const int4 &o, int &lt, int &pt) {
-          int it = i + o.y, jt = j + o.z, kt = k + o.w;
-          if (near) {
-            it += it < 0 ? L1 : 0;
-            jt += jt < 0 ? L2 : 0;
-            kt += kt < 0 ? L3 : 0;
-            it -= it >= L1 ? L1 : 0;
-            jt -= jt >= L2 ? L2 : 0;
-            kt -= kt >= L3 ? L3 : 0;
-          } else {
-            it = pad_wrap(it + h, h, L1);
-            jt = pad_wrap(jt + h, h, L2);
-            kt = pad_wrap(kt + h, h, L3);
-          }
-          lt = o.x * n_cells + it + L1 * (jt + L2 * kt);
-          pt = o.x * S + (kt + h) * P12 + (jt + h) * P1 + (it + h);
+        auto place = [&](int t, int &lt, int &pt) {
+          nfold_place(shape, nfold_unpack_nb(nbL[nb0 + t]), ci, cj, ck, lt, pt);
         };
         if (!distinct)
           for (int t = tid; t < nb1 - nb0; t += n_work) {
             int lt, pt;
-            place(neighbour(nb0 + t), lt, pt);
+            place(t, lt, pt);
             aff[t] = lt;
             affp[t] = pt;
           }
@@ -639,7 +683,7 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
         for (int t = tid; t < nb1 - nb0; t += n_work) {
           int lt, pt;
           if (distinct) {
-            place(neighbour(nb0 + t), lt, pt);
+            place(t, lt, pt);
           } else {
             lt = aff[t];
             pt = affp[t];
@@ -650,7 +694,7 @@ __device__ __forceinline__ void nfold_body(const NfoldArgs &na) {
           if (distinct) aff[t] = lt;  // the groups to sum again below
           if (!dup) {
             int K[kMaxSlots];
-            rate[rate_at(lt)] = site_rate_at(nbL[nb0 + t] & 0xff, pt, K);
+            rate[rate_at(lt)] = site_rate_at((int)(nbL[nb0 + t] & 0xff), pt, K);
             if (BIN && t == 0) {
               // the flipped site itself (first in the list): its cluster sums
 #pragma unroll

@@ -8,10 +8,7 @@
 namespace clexmc {
 
 size_t nfold_lds_bytes(int pad_sites, int n_sites, int nb_max, int nb_total, int n_sublat) {
-  const int n_groups = (n_sites + 63) / 64;
-  return nfold_align16((size_t)image_bytes(pad_sites, false)) + nfold_align16((size_t)n_groups * 64 * 4) +
-         nfold_align16((size_t)n_groups * 8) + 2 * nfold_align16((size_t)nb_max * 4) + kNfoldSelBytes +
-         kNfoldNbBeginBytes + nfold_align16((size_t)nb_total * 4) + (size_t)n_sublat * (1 + kMaxOcc) * 4;
+  return nfold_lds(pad_sites, n_sites, nb_max, nb_total, n_sublat).bytes;
 }
 
 template <bool BIN>
