@@ -361,6 +361,8 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
   long long n_bins = 0;
   for (int a = 0; a < s->n_orbits; ++a) {
     const int k = s->orbit_k[a], ne = s->corr_orbit_begin[a + 1] - s->corr_orbit_begin[a];
+    bin0[a] = (int)n_bins;
+    if (s->orbit_nfunc[a] <= 0) continue;  // nothing to count
     h->max_elem = std::max(h->max_elem, ne);
     for (int e = 0; e < ne; ++e) {
       long long n = 1;
@@ -369,13 +371,12 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
         ARG_CHECK(es[0] >= 0 && es[0] < s->n_sublat, "orbit element sublattice out of range");
         n *= s->n_occ[es[0]];
         for (int c = 1; c < 4; ++c) h->elem_reach = std::max(h->elem_reach, std::abs(es[c]));
-        ARG_CHECK(n < (1ll << 28), "orbit with too many decorations");
+        ARG_CHECK(n < (1ll << 31), "orbit with too many decorations");  // (nor does its table's offset go further)
       }
       ntau[a] = std::max(ntau[a], (int)n);
     }
-    bin0[a] = (int)n_bins;
     n_bins += ntau[a];
-    ARG_CHECK(n_bins < (1ll << 30), "too many cluster decorations");
+    ARG_CHECK(n_bins < (1ll << 31), "too many cluster decorations");
     h->max_ntau = std::max(h->max_ntau, ntau[a]);
   }
   h->n_bins = (int)n_bins;
@@ -1241,17 +1242,25 @@ static clexmc_status run_corr(clexmc_handle *h, int chain0, int n, double *out_h
   a.direct = corr_direct(max_cells, h->max_elem, h->max_ntau) ? 1 : 0;
   a.cells_per_block = a.direct ? (int)max_cells
                                : corr_cells_per_block(max_cells, h->max_elem, h->n_orbits, n, h->n_cu);
+  // the counters of as many chains as kCorrHistBytes holds, at least one's
+  static constexpr size_t kCorrHistBytes = 256u << 20;
+  const size_t chain_bytes = a.direct ? 0 : sizeof(unsigned long long) * (size_t)h->n_bins;
+  const int slice = chain_bytes ? (int)std::min<size_t>((size_t)n, std::max<size_t>(1, kCorrHistBytes / chain_bytes)) : n;
   DevBufs B;
-  const size_t out_bytes = sizeof(double) * h->n_corr * (size_t)n;
-  const size_t hist_bytes = a.direct ? 0 : sizeof(unsigned long long) * h->n_bins * (size_t)n;
+  const size_t out_bytes = sizeof(double) * h->n_corr * (size_t)n, hist_bytes = chain_bytes * slice;
   unsigned char *buf;
   HIP_TRY(B.alloc(&buf, out_bytes + hist_bytes));
-  a.out = (double *)buf;
-  a.hist = a.direct ? nullptr : (unsigned long long *)(buf + out_bytes);
   // (also the correlations: functions of an orbit without clusters stay 0)
   hipError_t e = hipMemsetAsync(buf, 0, out_bytes + hist_bytes, h->stream);
-  if (e == hipSuccess) e = launch_corr(a, max_cells, h->n_orbits, n, h->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(out_host, a.out, out_bytes, hipMemcpyDeviceToHost, h->stream);
+  double *const out = (double *)buf;
+  a.hist = a.direct ? nullptr : (unsigned long long *)(buf + out_bytes);
+  for (int c = 0; c < n && e == hipSuccess; c += slice) {
+    if (c > 0) e = hipMemsetAsync(a.hist, 0, hist_bytes, h->stream);
+    a.chain0 = chain0 + c;
+    a.out = out + (size_t)c * h->n_corr;
+    if (e == hipSuccess) e = launch_corr(a, max_cells, h->n_orbits, std::min(slice, n - c), h->stream);
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(out_host, out, out_bytes, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
   if (e != hipSuccess) {
     h->err = std::string("correlations: ") + hipGetErrorString(e);

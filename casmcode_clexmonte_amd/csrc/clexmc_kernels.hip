@@ -131,11 +131,12 @@ __global__ __launch_bounds__(256) void delta_batch_kernel(DeltaArgs a) {
 // with exact integer counts, and the FP64 sum runs over decorations.
 //
 // corr_count_kernel: a block counts the decorations of one orbit over a range
-// of cells of one chain (grid: cell ranges x orbits x chains) in LDS, with up
+// of cells of one chain (grid: orbits x cell ranges x chains) in LDS, with up
 // to 16 copies of every counter (by lane) so that the few decorations of a
 // pair do not serialise the lanes.  `direct` (a chain's cells in one block):
 // it forms the correlations at once.  Else the counts go to a.hist and
-// corr_finish_kernel forms them.  Orbits with more than kCorrLdsBins
+// corr_finish_kernel forms them, by the same sum (corr_sum): a chain's
+// correlations do not depend on the form, and so not on the chains beside it.  Orbits with more than kCorrLdsBins
 // decorations count in global memory.  Bound by the address arithmetic of the
 // cluster sites (about 10 VALU operations per site).
 // BCC quaternary 32^3, 8 chains loaded and every correlation read one chain
@@ -185,17 +186,45 @@ __device__ __forceinline__ void corr_count(cptr<DevSystem> sys, const DevSuperce
   }
 }
 
+// Correlation f of an orbit from its decoration counts (count(t) occurrences of
+// decoration t), one wavefront: products and sums carry their rounding errors
+// along (Dekker's two-product by fma, Knuth's two-sum), so that the sum is
+// rounded once before the division by the multiplicity.
+template <class COUNT>
+__device__ __forceinline__ double corr_sum(int ntau, const double *T, int nf, int f, int mult, COUNT count) {
+#pragma clang fp contract(off)
+  double hi = 0.0, lo = 0.0;
+  auto add = [&](double p, double err) {
+#pragma clang fp contract(off)
+    const double s = hi + p, q = s - hi;
+    lo += ((hi - (s - q)) + (p - q)) + err;
+    hi = s;
+  };
+  for (int t = threadIdx.x & 63; t < ntau; t += 64) {
+    const unsigned long long c = count(t);
+    if (c) {
+      const double n = (double)c, v = T[t * nf + f], p = n * v;
+      add(p, __builtin_fma(n, v, -p));
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const double h2 = __shfl_xor(hi, o), l2 = __shfl_xor(lo, o);
+    add(h2, l2);
+  }
+  return (hi + lo) / (double)mult;
+}
+
 __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
   __shared__ unsigned bins[kCorrLdsBins];
   const int tid = threadIdx.x;
-  const int orb = blockIdx.y;
+  const int orb = blockIdx.x;
   const int chain = a.chain0 + blockIdx.z;
   cptr<DevSystem> sys = cst(a.sys);
   const ChainParams &cp = a.params[chain];
   const DevSupercell &sc = a.scs[cp.sc];
   const int8_t *__restrict__ occ = a.occ + cp.occ_offset;
   const int nf = sys->orbit_nfunc[orb];
-  const int c0 = (int)blockIdx.x * a.cells_per_block;
+  const int c0 = (int)blockIdx.y * a.cells_per_block;
   if (nf <= 0 || c0 >= sc.n_cells) return;
   const int c1 = min(c0 + a.cells_per_block, sc.n_cells);
   const int k = sys->orbit_k_all[orb];
@@ -204,7 +233,7 @@ __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
   const int ntau = sys->orbit_ntau[orb];
   const bool in_lds = ntau <= kCorrLdsBins;
   int copies = 1;
-  while (copies < 16 && ntau * copies * 2 <= kCorrLdsBins) copies *= 2;
+  while (in_lds && copies < 16 && ntau * copies * 2 <= kCorrLdsBins) copies *= 2;
   unsigned long long *hist = a.hist ? a.hist + (long long)blockIdx.z * a.n_bins + sys->orbit_bin0[orb] : nullptr;
   if (in_lds)
     for (int t = tid; t < ntau * copies; t += kCorrThreads) bins[t] = 0u;
@@ -229,14 +258,12 @@ __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
     const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
     const int f0 = sys->orbit_func_begin[orb];
     for (int f = tid >> 6; f < nf; f += kCorrThreads / 64) {
-      double acc = 0.0;
-      for (int t = tid & 63; t < ntau; t += 64) {
-        unsigned v = 0u;
-        for (int q = 0; q < copies; ++q) v += bins[t * copies + q];
-        if (v) acc += (double)v * T[t * nf + f];
-      }
-      acc = wave_sum(acc);
-      if ((tid & 63) == 0) a.out[(long long)blockIdx.z * a.n_corr + f0 + f] = acc / (double)sys->orbit_mult[orb];
+      const double v = corr_sum(ntau, T, nf, f, sys->orbit_mult[orb], [&](int t) -> unsigned long long {
+        unsigned n = 0u;
+        for (int q = 0; q < copies; ++q) n += bins[t * copies + q];
+        return n;
+      });
+      if ((tid & 63) == 0) a.out[(long long)blockIdx.z * a.n_corr + f0 + f] = v;
     }
     return;
   }
@@ -248,33 +275,16 @@ __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
 }
 
 // correlations from the decoration counts: one block per (orbit, chain), one
-// wavefront per function.  Products and sums carry their rounding errors along
-// (Dekker's two-product by fma, Knuth's two-sum), so the sum is rounded once.
+// wavefront per function
 __global__ __launch_bounds__(1024) void corr_finish_kernel(CorrArgs a) {
-  const int orb = blockIdx.x, lane = threadIdx.x & 63;
+  const int orb = blockIdx.x;
   cptr<DevSystem> sys = cst(a.sys);
   const int nf = sys->orbit_nfunc[orb], f0 = sys->orbit_func_begin[orb], ntau = sys->orbit_ntau[orb];
   const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
   const unsigned long long *hist = a.hist + (long long)blockIdx.y * a.n_bins + sys->orbit_bin0[orb];
   for (int f = threadIdx.x >> 6; f < nf; f += 16) {
-#pragma clang fp contract(off)
-    double hi = 0.0, lo = 0.0;
-    auto add = [&](double p, double err) {
-#pragma clang fp contract(off)
-      const double s = hi + p, q = s - hi;
-      lo += ((hi - (s - q)) + (p - q)) + err;
-      hi = s;
-    };
-    for (int t = lane; t < ntau; t += 64) {
-      const double n = (double)hist[t], v = T[t * nf + f], p = n * v;
-      if (hist[t]) add(p, __builtin_fma(n, v, -p));
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-      const double h2 = __shfl_xor(hi, o), l2 = __shfl_xor(lo, o);
-      add(h2, l2);
-    }
-    if (lane == 0)
-      a.out[(long long)blockIdx.y * a.n_corr + f0 + f] = (hi + lo) / (double)sys->orbit_mult[orb];
+    const double v = corr_sum(ntau, T, nf, f, sys->orbit_mult[orb], [&](int t) { return hist[t]; });
+    if ((threadIdx.x & 63) == 0) a.out[(long long)blockIdx.y * a.n_corr + f0 + f] = v;
   }
 }
 
@@ -513,6 +523,7 @@ bool corr_direct(long long max_cells, int max_elem, int max_ntau) {
 // fewer while that leaves the device short of blocks, at least one per thread
 int corr_cells_per_block(long long max_cells, int max_elem, int n_orbits, int n_chains, int n_cu) {
   long long cells = std::max(1, 65536 / std::max(1, max_elem));
+  cells = std::max(cells, (max_cells + 32767) / 32768);  // (the grid's y extent is bounded)
   while (cells > kCorrThreads && (max_cells + cells - 1) / cells * n_orbits * n_chains < 4ll * n_cu) cells /= 2;
   return (int)((cells + kCorrThreads - 1) / kCorrThreads * kCorrThreads);
 }
@@ -526,7 +537,7 @@ hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int
     s.out = a.out + (long long)z0 * a.n_corr;
     if (a.hist) s.hist = a.hist + (long long)z0 * a.n_bins;
     const unsigned gx = a.direct ? 1u : (unsigned)((max_cells + a.cells_per_block - 1) / a.cells_per_block);
-    hipLaunchKernelGGL(corr_count_kernel, dim3(gx, n_orbits, nz), dim3(kCorrThreads), 0, st, s);
+    hipLaunchKernelGGL(corr_count_kernel, dim3(n_orbits, gx, nz), dim3(kCorrThreads), 0, st, s);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && !a.direct) {
       hipLaunchKernelGGL(corr_finish_kernel, dim3(n_orbits, nz), dim3(1024), 0, st, s);
