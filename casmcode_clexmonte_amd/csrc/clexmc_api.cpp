@@ -73,6 +73,7 @@ struct clexmc_handle {
   // correlations: elements of the largest orbit, largest site offset of an
   // element, decorations of an orbit (largest) and of all orbits
   int max_elem = 1, elem_reach = 0, max_ntau = 1, n_bins = 0;
+  bool corr_owned = false;  // every function belongs to one orbit
   DevSystem dsys{};
   DevSystem *d_sys = nullptr;
   std::vector<void *> sys_allocs;
@@ -358,11 +359,13 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
   }
   // correlations
   std::vector<int> ntau(s->n_orbits, 1), bin0(s->n_orbits, 0);
+  std::set<int> owned;
   long long n_bins = 0;
   for (int a = 0; a < s->n_orbits; ++a) {
     const int k = s->orbit_k[a], ne = s->corr_orbit_begin[a + 1] - s->corr_orbit_begin[a];
     bin0[a] = (int)n_bins;
     if (s->orbit_nfunc[a] <= 0) continue;  // nothing to count
+    for (int i = 0; i < s->orbit_nfunc[a]; ++i) owned.insert(s->orbit_func_begin[a] + i);
     h->max_elem = std::max(h->max_elem, ne);
     for (int e = 0; e < ne; ++e) {
       long long n = 1;
@@ -380,6 +383,7 @@ clexmc_status clexmc_create(const clexmc_system_desc *s, int device, clexmc_hand
     h->max_ntau = std::max(h->max_ntau, ntau[a]);
   }
   h->n_bins = (int)n_bins;
+  h->corr_owned = (int)owned.size() == s->n_corr && *owned.begin() == 0 && *owned.rbegin() == s->n_corr - 1;
   HIP_TRY(upload(h, A, s->orbit_k, (size_t)s->n_orbits, (int **)&d.orbit_k_all));
   HIP_TRY(upload(h, A, s->orbit_mult, (size_t)s->n_orbits, (int **)&d.orbit_mult));
   HIP_TRY(upload(h, A, s->orbit_nfunc, (size_t)s->n_orbits, (int **)&d.orbit_nfunc));
@@ -1250,8 +1254,10 @@ static clexmc_status run_corr(clexmc_handle *h, int chain0, int n, double *out_h
   const size_t out_bytes = sizeof(double) * h->n_corr * (size_t)n, hist_bytes = chain_bytes * slice;
   unsigned char *buf;
   HIP_TRY(B.alloc(&buf, out_bytes + hist_bytes));
-  // (also the correlations: functions of an orbit without clusters stay 0)
-  hipError_t e = hipMemsetAsync(buf, 0, out_bytes + hist_bytes, h->stream);
+  // (also the correlations, for functions that belong to no orbit; the
+  // one-block form writes all the others)
+  hipError_t e = hipSuccess;
+  if (!a.direct || !h->corr_owned) e = hipMemsetAsync(buf, 0, out_bytes + hist_bytes, h->stream);
   double *const out = (double *)buf;
   a.hist = a.direct ? nullptr : (unsigned long long *)(buf + out_bytes);
   for (int c = 0; c < n && e == hipSuccess; c += slice) {

@@ -85,6 +85,7 @@ struct CorrArgs {
   int n_bins;            // decoration counters per chain, all orbits
   unsigned long long *hist;  // [n_chains][n_bins], zero before the launch (direct: not used)
   int cells_per_block;
+  int n_ranges;          // cell ranges of the largest chain (set by launch_corr)
   int direct;            // every chain's cells in one block per orbit
   int elem_reach;        // largest cell offset of an orbit element's site
 };

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void delta_batch_kernel(DeltaArgs a) {
 // with exact integer counts, and the FP64 sum runs over decorations.
 //
 // corr_count_kernel: a block counts the decorations of one orbit over a range
-// of cells of one chain (grid: orbits x cell ranges x chains) in LDS, with up
+// of cells of one chain (grid: cell ranges of one orbit after the other, chains) in LDS, with up
 // to 16 copies of every counter (by lane) so that the few decorations of a
 // pair do not serialise the lanes.  `direct` (a chain's cells in one block):
 // it forms the correlations at once.  Else the counts go to a.hist and
@@ -147,17 +147,23 @@ constexpr int kCorrThreads = 512;
 constexpr int kCorrLdsBins = 8192;  // counters in LDS (32 KB)
 
 // decoration counts of one orbit over the cells [c0, c1); K: sites per
-// cluster (-1: any), NEAR: every site offset is at most one period
-template <int K, bool NEAR, class ADD>
+// cluster (-1: any), NEAR: every site offset is at most one period.  SHARE
+// (fewer cells than threads): groups of wavefronts share the orbit's elements;
+// one cell's elements one after the other are a chain of load latencies (BCC
+// 8^3, correlations of one chain: 54 us, 35 us so with the sums below)
+template <int K, bool NEAR, bool SHARE, class ADD>
 __device__ __forceinline__ void corr_count(cptr<DevSystem> sys, const DevSupercell &sc, const int8_t *__restrict__ occ,
                                            const int4 *elem_sites, int ne, int k_rt, int c0, int c1, ADD add) {
   const int k = K >= 0 ? K : k_rt;
   const int L1 = sc.L1, L2 = sc.L2, L3 = sc.L3, n_cells = sc.n_cells;
   cptr<int4> es = cst(elem_sites);
-  for (int c = c0 + (int)threadIdx.x; c < c1; c += kCorrThreads) {
+  const int w = SHARE ? (c1 - c0 + 63) & ~63 : kCorrThreads, groups = SHARE ? kCorrThreads / w : 1;
+  const int group = SHARE ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / w) : 0;
+  if (group >= groups) return;
+  for (int c = c0 + (int)threadIdx.x - group * w; c < c1; c += w) {
     const int i0 = c % L1, j0 = (c / L1) % L2, k0 = c / (L1 * L2);
 #pragma unroll 2
-    for (int e = 0; e < ne; ++e) {
+    for (int e = group; e < ne; e += groups) {
       int tau = 0, mul = 1;
 #pragma unroll
       for (int q = 0; q < k; ++q) {
@@ -200,12 +206,10 @@ __device__ __forceinline__ double corr_sum(int ntau, const double *T, int nf, in
     lo += ((hi - (s - q)) + (p - q)) + err;
     hi = s;
   };
+#pragma unroll 4
   for (int t = threadIdx.x & 63; t < ntau; t += 64) {
-    const unsigned long long c = count(t);
-    if (c) {
-      const double n = (double)c, v = T[t * nf + f], p = n * v;
-      add(p, __builtin_fma(n, v, -p));
-    }
+    const double n = (double)count(t), v = T[t * nf + f], p = n * v;
+    if (n > 0.0) add(p, __builtin_fma(n, v, -p));
   }
   for (int o = 32; o > 0; o >>= 1) {
     const double h2 = __shfl_xor(hi, o), l2 = __shfl_xor(lo, o);
@@ -217,14 +221,14 @@ __device__ __forceinline__ double corr_sum(int ntau, const double *T, int nf, in
 __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
   __shared__ unsigned bins[kCorrLdsBins];
   const int tid = threadIdx.x;
-  const int orb = blockIdx.x;
-  const int chain = a.chain0 + blockIdx.z;
+  const int orb = (int)blockIdx.x / a.n_ranges;
+  const int chain = a.chain0 + blockIdx.y;
   cptr<DevSystem> sys = cst(a.sys);
   const ChainParams &cp = a.params[chain];
   const DevSupercell &sc = a.scs[cp.sc];
   const int8_t *__restrict__ occ = a.occ + cp.occ_offset;
   const int nf = sys->orbit_nfunc[orb];
-  const int c0 = (int)blockIdx.y * a.cells_per_block;
+  const int c0 = ((int)blockIdx.x - orb * a.n_ranges) * a.cells_per_block;
   if (nf <= 0 || c0 >= sc.n_cells) return;
   const int c1 = min(c0 + a.cells_per_block, sc.n_cells);
   const int k = sys->orbit_k_all[orb];
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
   const bool in_lds = ntau <= kCorrLdsBins;
   int copies = 1;
   while (in_lds && copies < 16 && ntau * copies * 2 <= kCorrLdsBins) copies *= 2;
-  unsigned long long *hist = a.hist ? a.hist + (long long)blockIdx.z * a.n_bins + sys->orbit_bin0[orb] : nullptr;
+  unsigned long long *hist = a.hist ? a.hist + (long long)blockIdx.y * a.n_bins + sys->orbit_bin0[orb] : nullptr;
   if (in_lds)
     for (int t = tid; t < ntau * copies; t += kCorrThreads) bins[t] = 0u;
   __syncthreads();
@@ -242,35 +246,39 @@ __global__ __launch_bounds__(kCorrThreads) void corr_count_kernel(CorrArgs a) {
   if (in_lds) {
     unsigned *mine = bins + (tid & (copies - 1));
     auto add = [&](int tau) { atomicAdd(&mine[tau * copies], 1u); };
-    if (!near) corr_count<-1, false>(sys, sc, occ, es, ne, k, c0, c1, add);
-    else if (k == 1) corr_count<1, true>(sys, sc, occ, es, ne, k, c0, c1, add);
-    else if (k == 2) corr_count<2, true>(sys, sc, occ, es, ne, k, c0, c1, add);
-    else if (k == 3) corr_count<3, true>(sys, sc, occ, es, ne, k, c0, c1, add);
-    else if (k == 4) corr_count<4, true>(sys, sc, occ, es, ne, k, c0, c1, add);
-    else corr_count<-1, true>(sys, sc, occ, es, ne, k, c0, c1, add);
+    auto count = [&](auto share) {
+      constexpr bool S = decltype(share)::value;
+      if (!near) corr_count<-1, false, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+      else if (k == 1) corr_count<1, true, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+      else if (k == 2) corr_count<2, true, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+      else if (k == 3) corr_count<3, true, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+      else if (k == 4) corr_count<4, true, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+      else corr_count<-1, true, S>(sys, sc, occ, es, ne, k, c0, c1, add);
+    };
+    if (c1 - c0 <= kCorrThreads / 2) count(std::true_type{});
+    else count(std::false_type{});
   } else {
     auto add = [&](int tau) { atomicAdd(&hist[tau], 1ull); };
-    corr_count<-1, false>(sys, sc, occ, es, ne, k, c0, c1, add);
+    corr_count<-1, false, false>(sys, sc, occ, es, ne, k, c0, c1, add);
   }
   __syncthreads();
   if (!in_lds) return;
-  if (a.direct) {
-    const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
-    const int f0 = sys->orbit_func_begin[orb];
-    for (int f = tid >> 6; f < nf; f += kCorrThreads / 64) {
-      const double v = corr_sum(ntau, T, nf, f, sys->orbit_mult[orb], [&](int t) -> unsigned long long {
-        unsigned n = 0u;
-        for (int q = 0; q < copies; ++q) n += bins[t * copies + q];
-        return n;
-      });
-      if ((tid & 63) == 0) a.out[(long long)blockIdx.z * a.n_corr + f0 + f] = v;
-    }
-    return;
-  }
+  // the copies of a counter, added from another one on in every lane (lanes a
+  // multiple of the copies apart would read one LDS bank)
   for (int t = tid; t < ntau; t += kCorrThreads) {
     unsigned v = 0u;
-    for (int q = 0; q < copies; ++q) v += bins[t * copies + q];
-    if (v) atomicAdd(&hist[t], (unsigned long long)v);
+    for (int q = 0; q < copies; ++q) v += bins[t * copies + ((q + t) & (copies - 1))];
+    if (a.direct) bins[t * copies] = v;
+    else if (v) atomicAdd(&hist[t], (unsigned long long)v);
+  }
+  if (!a.direct) return;
+  __syncthreads();
+  const double *T = sys->orbit_tables + sys->orbit_table_offset[orb];
+  const int f0 = sys->orbit_func_begin[orb];
+  for (int f = tid >> 6; f < nf; f += kCorrThreads / 64) {
+    const double v = corr_sum(ntau, T, nf, f, sys->orbit_mult[orb],
+                              [&](int t) -> unsigned long long { return bins[t * copies]; });
+    if ((tid & 63) == 0) a.out[(long long)blockIdx.y * a.n_corr + f0 + f] = v;
   }
 }
 
@@ -523,21 +531,21 @@ bool corr_direct(long long max_cells, int max_elem, int max_ntau) {
 // fewer while that leaves the device short of blocks, at least one per thread
 int corr_cells_per_block(long long max_cells, int max_elem, int n_orbits, int n_chains, int n_cu) {
   long long cells = std::max(1, 65536 / std::max(1, max_elem));
-  cells = std::max(cells, (max_cells + 32767) / 32768);  // (the grid's y extent is bounded)
+  cells = std::max(cells, max_cells * n_orbits >> 30);  // (the grid is bounded)
   while (cells > kCorrThreads && (max_cells + cells - 1) / cells * n_orbits * n_chains < 4ll * n_cu) cells /= 2;
   return (int)((cells + kCorrThreads - 1) / kCorrThreads * kCorrThreads);
 }
 
 hipError_t launch_corr(const CorrArgs &a, long long max_cells, int n_orbits, int n_chains, hipStream_t st) {
-  // the grid's z extent is bounded: chains in slices
+  // the grid's y extent is bounded: chains in slices
   for (int z0 = 0; z0 < n_chains; z0 += 32768) {
     CorrArgs s = a;
     const int nz = std::min(32768, n_chains - z0);
     s.chain0 = a.chain0 + z0;
     s.out = a.out + (long long)z0 * a.n_corr;
     if (a.hist) s.hist = a.hist + (long long)z0 * a.n_bins;
-    const unsigned gx = a.direct ? 1u : (unsigned)((max_cells + a.cells_per_block - 1) / a.cells_per_block);
-    hipLaunchKernelGGL(corr_count_kernel, dim3(n_orbits, gx, nz), dim3(kCorrThreads), 0, st, s);
+    s.n_ranges = a.direct ? 1 : (int)((max_cells + a.cells_per_block - 1) / a.cells_per_block);
+    hipLaunchKernelGGL(corr_count_kernel, dim3((unsigned)s.n_ranges * n_orbits, nz), dim3(kCorrThreads), 0, st, s);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && !a.direct) {
       hipLaunchKernelGGL(corr_finish_kernel, dim3(n_orbits, nz), dim3(1024), 0, st, s);
