@@ -37,7 +37,7 @@ struct HostSupercell {
   // specialised kernels per (kind, packed, lanes, launch bound 512 / 1024):
   // 0 not tried, 1 loaded, -1 unavailable
   int jit_state[3][2][2][2] = {};
-  size_t jit_lds_fail = 0;  // smallest dynamic LDS size at which a specialised launch was refused
+  JitRefusals jit_refused;
   std::vector<hipModule_t> jit_mods;
   hipFunction_t jit_fn[3][2][2][2] = {};  // [kind][packed][lanes][block above 512]
   // the same for sets of a few sites (spread fields) [kind 0, 1]
@@ -2071,9 +2071,9 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
     for (int i = 1; i < n_sel; ++i) one_shape = one_shape && h->chain_sc[subset ? (*subset)[i] : i] == h->chain_sc[c0];
     P.sc_id = h->chain_sc[c0];
     P.one_shape = one_shape;
-    const size_t fail = h->scs[h->chain_sc[c0]].jit_lds_fail;
-    if (h->specialize && !P.learned && one_shape && !fused_spec && (fail == 0 || lds < fail)) {
-      if (P.threads == 64 && kind != 2 && !packed && P.lanes == 1)
+    const JitRefusals &refused = h->scs[h->chain_sc[c0]].jit_refused;
+    if (h->specialize && !P.learned && one_shape && !fused_spec && refused.allows(lds)) {
+      if (P.threads == 64 && kind != 2 && !packed && P.lanes == 1 && refused.allows_spread(kind))
         P.lds_spread = spread_lds(h, h->scs[h->chain_sc[c0]], P.lds);
       if (P.lds_spread > 0) {
         P.jit = jit_kernel(h, h->chain_sc[c0], kind, false, 1, 64, true);
@@ -2099,16 +2099,21 @@ static clexmc_status plan_run(clexmc_handle *h, int kind, int n_passes, int samp
 }
 
 // The runtime refused a specialised launch (dynamic LDS of a module kernel
-// above its limit): remember the LDS size and fall back to the ahead-of-time
-// kernel, whose block size is bounded at 512 threads.
+// above its limit): remember it and go on to the next kernel, the ordinary
+// specialised one after the spread one, then the ahead-of-time kernel, whose
+// block size is bounded at 512 threads.
 static void drop_jit(clexmc_handle *h, RunPlan &P, int sc_id) {
   (void)hipGetLastError();
-  h->scs[sc_id].jit_lds_fail = P.lds;
+  JitRefusals &refused = h->scs[sc_id].jit_refused;
+  refused.refused(P.kind, P.lds, P.spread ? P.lds_spread : 0);
   P.jit = nullptr;
   P.cube = false;
-  if (P.spread) P.lds -= P.lds_spread;
-  P.spread = false;
-  P.threads = std::min(P.threads, kAotMaxThreads);
+  if (P.spread) {
+    P.spread = false;
+    P.lds -= P.lds_spread;
+    if (refused.allows(P.lds)) P.jit = jit_kernel(h, sc_id, P.kind, P.packed, P.lanes, P.threads);
+  }
+  if (!P.jit) P.threads = std::min(P.threads, kAotMaxThreads);
 }
 
 // attribute setting (not a stream operation) and the launch, separately, so
@@ -2445,7 +2450,7 @@ static clexmc_status run_grouped(clexmc_handle *h, int kind, int n_passes, int s
     RunPlan &P = plans[g];
     hipStream_t st = h->side[stream_of[g]];
     hipError_t le = plan_launch(P, h, st);
-    if (le != hipSuccess && P.jit) {
+    while (le != hipSuccess && P.jit) {
       drop_jit(h, P, P.sc_id);
       HIP_TRY(plan_attributes(P, h));
       le = plan_launch(P, h, st);
@@ -2523,9 +2528,9 @@ static clexmc_status run_passes_impl(clexmc_handle *h, int kind, int n_passes, i
   HIP_TRY(plan_attributes(P, h));
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
   hipError_t le = plan_launch(P, h);
-  if (le != hipSuccess && P.jit) {
+  while (le != hipSuccess && P.jit) {
     drop_jit(h, P, h->chain_sc[0]);
-    h->last_specialized = 0;
+    h->last_specialized = P.jit ? 1 : 0;
     h->last_threads = P.threads;
     HIP_TRY(plan_attributes(P, h));
     le = plan_launch(P, h);
@@ -2570,14 +2575,14 @@ clexmc_status clexmc_graph_capture(clexmc_handle *h, int kind, int passes_per_re
   HIP_TRY(hipStreamSynchronize(h->stream));
   hipError_t e = hipSuccess;
   hipGraph_t g = nullptr;
-  for (int attempt = 0; attempt < 2; ++attempt) {
+  for (int attempt = 0; attempt < 3; ++attempt) {
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     e = plan_launch(P, h);
     g = nullptr;
     hipError_t e2 = hipStreamEndCapture(h->stream, &g);
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess || !P.jit) break;
-    // specialised launch refused: capture the generic kernel instead
+    // specialised launch refused: capture the next kernel instead
     if (g) hipGraphDestroy(g);
     g = nullptr;
     drop_jit(h, P, h->chain_sc[0]);

@@ -53,6 +53,23 @@ std::string jit_source_nfold_single(int n_sublat, const std::vector<int> &variab
 // registers (16 rows, all sublattices together) or for more than 4 sublattices.
 int spread_items(const std::vector<int> &variable, const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog);
 
+// Specialised launches of a supercell that the runtime refused (their dynamic
+// LDS).  The spread kernels, which take LDS of their own, are remembered by
+// themselves: a refusal of theirs says nothing of the ordinary kernel's launch
+// with less LDS, which is the next to try.
+struct JitRefusals {
+  size_t lds = 0;           // smallest dynamic LDS of a refused ordinary launch (0: none)
+  bool spread[2] = {};      // spread kernel refused [kind 0, 1]
+  bool allows(size_t bytes) const { return lds == 0 || bytes < lds; }
+  bool allows_spread(int kind) const { return !spread[kind]; }
+  // a refused launch with `bytes` of LDS, `spread_bytes` of them the spread
+  // kernel's (0: the ordinary kernel)
+  void refused(int kind, size_t bytes, size_t spread_bytes) {
+    if (spread_bytes > 0) spread[kind] = true;
+    else if (allows(bytes)) lds = bytes;
+  }
+};
+
 // One supercell shape of a fused launch: its site programs (as for
 // jit_source) and image format.
 struct JitShape {
