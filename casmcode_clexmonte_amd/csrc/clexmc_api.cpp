@@ -118,6 +118,7 @@ struct clexmc_handle {
   int packing = 0;                  // LDS image: 0 automatic, 1 int8, 2 packed 2-bit
   bool last_packed = false;
   int last_specialized = 0, last_threads = 0, last_lanes = 1, last_slabs = 1, last_fused = 0, last_cube = 0;
+  int last_spread = 0, last_class_occ = 0;
   int fuse = 1;  // chains on several supercell shapes: one fused launch (1) or one launch per shape (0)
   int cube = 1;  // register-cube sweep where the specialised kernel has one (1) or the class loop (0)
   int slabs = 0;  // slabs per chain: 0 automatic, 1 off, >= 2 requested
@@ -1803,6 +1804,13 @@ clexmc_status clexmc_last_run_info(clexmc_handle *h, int *specialized, int *pack
   return CLEXMC_OK;
 }
 
+clexmc_status clexmc_last_run_routes(clexmc_handle *h, int *spread, int *class_occ) {
+  if (!h) return CLEXMC_ERR_ARG;
+  if (spread) *spread = h->last_spread;
+  if (class_occ) *class_occ = h->last_class_occ;
+  return CLEXMC_OK;
+}
+
 clexmc_status clexmc_last_run_lanes(clexmc_handle *h, int *lanes_per_site) {
   if (!h || !lanes_per_site) return CLEXMC_ERR_ARG;
   *lanes_per_site = h->last_lanes;
@@ -2372,6 +2380,8 @@ static bool run_fused(clexmc_handle *h, int kind, int n_passes, int sample_perio
   h->last_slabs = max_slabs;
   h->last_fused = 1;
   h->last_cube = 0;
+  h->last_spread = 0;
+  h->last_class_occ = a.class_occ;
   return true;
 }
 
@@ -2472,6 +2482,8 @@ static clexmc_status run_grouped(clexmc_handle *h, int kind, int n_passes, int s
   h->last_packed = any_packed;
   h->last_threads = plans[0].threads;
   h->last_lanes = plans[0].lanes;
+  h->last_spread = plans[0].spread ? 1 : 0;
+  h->last_class_occ = plans[0].a.class_occ;
   h->last_slabs = max_slabs;
   return CLEXMC_OK;
 }
@@ -2525,6 +2537,8 @@ static clexmc_status run_passes_impl(clexmc_handle *h, int kind, int n_passes, i
   h->last_slabs = P.slabs;
   h->last_fused = 0;
   h->last_cube = P.cube && P.slabs <= 1 ? 1 : 0;
+  h->last_spread = P.spread ? 1 : 0;
+  h->last_class_occ = P.a.class_occ;
   HIP_TRY(plan_attributes(P, h));
   HIP_TRY(hipEventRecord(h->ev0, h->stream));
   hipError_t le = plan_launch(P, h);
@@ -2532,6 +2546,7 @@ static clexmc_status run_passes_impl(clexmc_handle *h, int kind, int n_passes, i
     drop_jit(h, P, h->chain_sc[0]);
     h->last_specialized = P.jit ? 1 : 0;
     h->last_threads = P.threads;
+    h->last_spread = 0;
     HIP_TRY(plan_attributes(P, h));
     le = plan_launch(P, h);
   }

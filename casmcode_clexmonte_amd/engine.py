@@ -76,7 +76,7 @@ def lib():
                      "clexmc_set_lds_row_pitch", "clexmc_nfold_run",
                      "clexmc_reanchor_energies", "clexmc_graph_capture", "clexmc_graph_replay",
                      "clexmc_graph_release", "clexmc_autotune", "clexmc_set_specialization",
-                     "clexmc_last_run_info", "clexmc_specialization_log", "clexmc_lds_probe",
+                     "clexmc_last_run_info", "clexmc_last_run_routes", "clexmc_specialization_log", "clexmc_lds_probe",
                      "clexmc_set_lanes_per_site", "clexmc_last_run_lanes", "clexmc_set_slabs", "clexmc_last_run_slabs",
                      "clexmc_set_fused_launch", "clexmc_last_run_fused", "clexmc_nfold_run_moments",
                      "clexmc_nfold_run_time", "clexmc_set_register_cube", "clexmc_last_run_cube",
@@ -103,7 +103,7 @@ def exported_symbols() -> List[str]:
             "clexmc_set_lds_row_pitch", "clexmc_nfold_run",
             "clexmc_reanchor_energies", "clexmc_graph_capture", "clexmc_graph_replay",
             "clexmc_graph_release", "clexmc_autotune", "clexmc_set_specialization",
-            "clexmc_last_run_info", "clexmc_specialization_log", "clexmc_lds_probe",
+            "clexmc_last_run_info", "clexmc_last_run_routes", "clexmc_specialization_log", "clexmc_lds_probe",
             "clexmc_set_lanes_per_site", "clexmc_last_run_lanes", "clexmc_set_slabs", "clexmc_last_run_slabs",
             "clexmc_set_fused_launch", "clexmc_last_run_fused", "clexmc_nfold_run_moments",
             "clexmc_nfold_run_time", "clexmc_set_register_cube", "clexmc_last_run_cube",
@@ -620,6 +620,14 @@ class Engine:
         self._check(lib().clexmc_last_run_lanes(self.h, C.byref(ln)), "clexmc_last_run_lanes")
         return {"specialized": bool(sp.value), "packed": bool(pk.value), "threads": th.value,
                 "lanes_per_site": ln.value}
+
+    def last_run_routes(self):
+        """Whether the last run_passes spread a site's clusters over the lanes
+        (sets of a few sites) and kept a set's occupants side by side in LDS
+        (canonical matchings)."""
+        spread, occ = C.c_int(), C.c_int()
+        self._check(lib().clexmc_last_run_routes(self.h, C.byref(spread), C.byref(occ)), "clexmc_last_run_routes")
+        return {"spread": bool(spread.value), "class_occ": bool(occ.value)}
 
     def set_lanes_per_site(self, lanes: int):
         self._check(lib().clexmc_set_lanes_per_site(self.h, C.c_int(lanes)), "clexmc_set_lanes_per_site")

@@ -400,6 +400,12 @@ clexmc_status clexmc_specialization_log(clexmc_handle *h, char *buf, int cap);
  * packed image (0/1), block size. */
 clexmc_status clexmc_last_run_info(clexmc_handle *h, int *specialized, int *packed, int *threads);
 
+/* Routes of the last clexmc_run_passes (the first launch's, where there are
+ * several): spread fields for sets of a few sites (0/1), the occupants of a
+ * set side by side in LDS during canonical matchings (0/1).  Results do not
+ * depend on them. */
+clexmc_status clexmc_last_run_routes(clexmc_handle *h, int *spread, int *class_occ);
+
 /* Binary expansions: lanes per site in the class sweeps (2: the two lanes of
  * a pair each sum half of every orbit's clusters, doubling the wavefronts per
  * chain, at the cost of neighbour reads the two halves both need).  0
