@@ -1008,9 +1008,10 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(TrainArgs a) {
       db2 += (double)dl;
 #pragma unroll
       for (int tn = 0; tn < 4; ++tn) {
-        const float D = h[tn][r] > 0.f ? dl * W2[tn] : 0.0f;
+        // (a row past the batch adds zeros, also where a parameter is not finite)
+        const float D = in_b[r] && h[tn][r] > 0.f ? dl * W2[tn] : 0.0f;
         db1[tn] += (double)D;
-        dW2[tn] += (double)(dl * fmaxf(h[tn][r], 0.f));
+        dW2[tn] += in_b[r] ? (double)(dl * fmaxf(h[tn][r], 0.f)) : 0.0;
 #pragma unroll
         for (int tk = 0; tk < 3; ++tk)
           dW1[tn][tk] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)D, (double)xb[r][tk], dW1[tn][tk], 0, 0, 0);
@@ -1076,7 +1077,10 @@ __global__ __launch_bounds__(1024) void mlp_reduce_kernel(TrainArgs a, AdamArgs 
     return;
   }
   const float inv = 1.0f / (float)a.n;
-  const float grad = (float)(v * inv);
+  // inputs past n_env take no part, also in a sample that is not finite (whose
+  // products with their zeros are NaN)
+  const bool unused = p < kHidden * kEnvMax && p % kEnvMax >= a.n_env;
+  const float grad = unused ? 0.0f : (float)(v * inv);
   if (a.grad) a.grad[p] = grad;
   if (ad.p) {
     const float m = ad.b1m * ad.m[p] + (1.0f - ad.b1m) * grad;
