@@ -111,7 +111,7 @@ struct clexmc_handle {
   long long samples_bound = 0;
   int max_lds = 0, n_cu = 0;        // device attributes, read at creation
   unsigned char *h_stage = nullptr, *d_stage = nullptr;  // delta-energy staging (pinned host, device)
-  size_t stage_bytes = 0;
+  size_t h_stage_bytes = 0, d_stage_bytes = 0;
   unsigned char *noalloc = nullptr; // the device's staging array (clexmc_delta_energy_batch_noalloc)
   int block_size = 0;
   int nfold_threads = 0;  // N-fold kernel block size (0: automatic)
@@ -1336,26 +1336,34 @@ static hipError_t delta_batch_staged(clexmc_handle *h, int n_prop, const int32_t
   return e;
 }
 
-// Staging of the delta-energy calls: pinned host memory and a device buffer of
-// the same size, grown in powers of two to at most kDeltaSlice proposals'
-// bytes (2.5 MiB each), kept until the handle goes.
+// Staging of the delta-energy calls: pinned host memory and, beyond
+// kDeltaDirect proposals, a device buffer, grown in powers of two to at most
+// kDeltaSlice proposals' bytes (2.5 MiB each), kept until the handle goes.
 static constexpr int kDeltaSlice = 65536;
 // proposals up to which the kernel reads and writes the pinned memory itself:
 // the two copies' launches (about 10 us) cost more than its reads over the bus.
 // One proposed swap, the whole call: 226 us with four allocations, three
 // copies in and one out; 26 us so.
 static constexpr int kDeltaDirect = 256;
-static hipError_t delta_stage(clexmc_handle *h, size_t bytes) {
-  if (h->stage_bytes >= bytes) return hipSuccess;
+static hipError_t delta_stage(clexmc_handle *h, size_t bytes, bool device) {
   size_t cap = 4096;
   while (cap < bytes) cap *= 2;
-  (void)hipHostFree(h->h_stage);
-  (void)hipFree(h->d_stage);
-  h->h_stage = h->d_stage = nullptr;
-  h->stage_bytes = 0;
-  hipError_t e = hipHostMalloc((void **)&h->h_stage, cap, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc((void **)&h->d_stage, cap);
-  if (e == hipSuccess) h->stage_bytes = cap;
+  cap = std::min(cap, sizeof(int) * (size_t)kDeltaSlice * (2 + 2 * kMaxSitesPerProp));
+  hipError_t e = hipSuccess;
+  if (h->h_stage_bytes < bytes) {
+    (void)hipHostFree(h->h_stage);
+    h->h_stage = nullptr;
+    h->h_stage_bytes = 0;
+    e = hipHostMalloc((void **)&h->h_stage, cap, hipHostMallocDefault);
+    if (e == hipSuccess) h->h_stage_bytes = cap;
+  }
+  if (e == hipSuccess && device && h->d_stage_bytes < bytes) {
+    (void)hipFree(h->d_stage);
+    h->d_stage = nullptr;
+    h->d_stage_bytes = 0;
+    e = hipMalloc((void **)&h->d_stage, cap);
+    if (e == hipSuccess) h->d_stage_bytes = cap;
+  }
   return e;
 }
 
@@ -1364,13 +1372,13 @@ static hipError_t delta_stage(clexmc_handle *h, size_t bytes) {
 static hipError_t delta_slice(clexmc_handle *h, int n, const int32_t *chain, const int32_t *sites,
                               const int32_t *new_occ, int m, int include_chem, float *dE_out) {
   const size_t nb = sizeof(int) * (size_t)n, in_bytes = nb + 2 * nb * m;
-  hipError_t e = delta_stage(h, nb + in_bytes);
+  const bool direct = n <= kDeltaDirect;
+  hipError_t e = delta_stage(h, nb + in_bytes, !direct);
   if (e != hipSuccess) return e;
   unsigned char *hs = h->h_stage;
   memcpy(hs + nb, chain, nb);
   memcpy(hs + 2 * nb, sites, nb * m);
   memcpy(hs + 2 * nb + nb * m, new_occ, nb * m);
-  const bool direct = n <= kDeltaDirect;
   unsigned char *ds = direct ? hs : h->d_stage;
   if (!direct) e = hipMemcpyAsync(ds + nb, hs + nb, in_bytes, hipMemcpyHostToDevice, h->stream);
   if (e == hipSuccess)
