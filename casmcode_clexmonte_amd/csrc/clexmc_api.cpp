@@ -44,7 +44,7 @@ struct HostSupercell {
   int jit_spread_state[2] = {};
   hipFunction_t jit_spread[2] = {};
   hipFunction_t jit_nfold = nullptr;  // N-fold kernel of the SGC (unpacked, one-lane) module
-  int jit_nfold_single_state = 0;     // the one for blocks of one wavefront, a module of its own
+  int jit_nfold_state[2] = {};        // modules of its own: the same kernel, blocks of one wavefront
   hipFunction_t jit_nfold_single = nullptr;
   hipFunction_t jit_cube[2] = {nullptr, nullptr};  // register-cube kernel of that module [block above 512]
   // register-cube sweep (binary, one sublattice, classes = the residues of
@@ -1590,7 +1590,7 @@ clexmc_status clexmc_set_lds_row_pitch(clexmc_handle *h, int extra) {
 
 static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool packed, int lanes, int threads,
                                 bool spread = false);
-static hipFunction_t jit_nfold_single(clexmc_handle *h, int sc_id);
+static hipFunction_t jit_nfold_kernel(clexmc_handle *h, int sc_id, bool own_books);
 
 // Chains whose N-fold run stopped because their total rate vanished: the
 // flags are cleared and the run reported as failed (its blocks past the stop
@@ -1711,12 +1711,7 @@ static clexmc_status nfold_run_impl(clexmc_handle *h, int n_events, int events_p
   hipFunction_t jf = nullptr;
   bool own_books = false;
   int nf_threads = nfold_block(h, lds, nb_max, h->specialize && one_shape, &own_books);
-  if (h->specialize && one_shape && own_books) {
-    jf = jit_nfold_single(h, h->chain_sc[0]);
-  } else if (h->specialize && one_shape) {
-    (void)jit_kernel(h, h->chain_sc[0], 1, false, 1, kAotMaxThreads);
-    jf = h->scs[h->chain_sc[0]].jit_nfold;
-  }
+  if (h->specialize && one_shape) jf = jit_nfold_kernel(h, h->chain_sc[0], own_books);
   hipError_t e = hipMemsetAsync(d_blocks, 0, nb * sizeof(double), h->stream);
   h->last_specialized = 0;
   if (e == hipSuccess && jf) {
@@ -1898,26 +1893,28 @@ static hipFunction_t jit_kernel(clexmc_handle *h, int sc_id, int kind, bool pack
   return state == 1 ? fn : nullptr;
 }
 
-// The specialised one-wavefront N-fold kernel of a supercell, compiled on first use.
-static hipFunction_t jit_nfold_single(clexmc_handle *h, int sc_id) {
+// The specialised N-fold kernel of a supercell, compiled on first use by itself
+// where no semi-grand canonical module has brought it along (sets of a few
+// sites run another module; the one-wavefront kernel is in none).
+static hipFunction_t jit_nfold_kernel(clexmc_handle *h, int sc_id, bool own_books) {
   HostSupercell &hs = h->scs[sc_id];
-  if (hs.jit_nfold_single_state == 0) {
-    hs.jit_nfold_single_state = -1;
+  hipFunction_t &fn = own_books ? hs.jit_nfold_single : hs.jit_nfold;
+  int &state = hs.jit_nfold_state[own_books ? 1 : 0];
+  if (!fn && state == 0) {
+    state = -1;
     std::vector<int> variable(h->n_sublat);
     for (int b = 0; b < h->n_sublat; ++b) variable[b] = h->n_occ[b] >= 2;
     hipModule_t mod = nullptr;
-    if (jit_compile_load(jit_source_nfold_single(h->n_sublat, variable, h->binary != 0, hs.bin_sub, hs.bin_off,
-                                                 h->n_slots, hs.gen_sub, hs.gen_prog),
+    if (jit_compile_load(jit_source_nfold(h->n_sublat, variable, h->binary != 0, hs.bin_sub, hs.bin_off, h->n_slots,
+                                          hs.gen_sub, hs.gen_prog, own_books),
                          &mod, &h->jit_log) == hipSuccess) {
       hs.jit_mods.push_back(mod);
-      if (hipModuleGetFunction(&hs.jit_nfold_single, mod, kJitNfoldSingleName) == hipSuccess)
-        hs.jit_nfold_single_state = 1;
-      else
-        hs.jit_nfold_single = nullptr;
+      if (hipModuleGetFunction(&fn, mod, own_books ? kJitNfoldSingleName : kJitNfoldName) == hipSuccess) state = 1;
+      else fn = nullptr;
     }
-    if (hs.jit_nfold_single_state < 0) (void)hipGetLastError();
+    if (state < 0) (void)hipGetLastError();
   }
-  return hs.jit_nfold_single;
+  return fn;
 }
 
 // Sample storage for n_new_samples more samples per chain.  The count in use

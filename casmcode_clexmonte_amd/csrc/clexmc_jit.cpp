@@ -512,15 +512,17 @@ std::string jit_source(int n_sublat, const std::vector<int> &variable, bool bina
   return o.str();
 }
 
-std::string jit_source_nfold_single(int n_sublat, const std::vector<int> &variable, bool binary,
-                                    const std::vector<BinSub> &subs, const std::vector<int> &bin_off, int n_slots,
-                                    const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog) {
+std::string jit_source_nfold(int n_sublat, const std::vector<int> &variable, bool binary,
+                             const std::vector<BinSub> &subs, const std::vector<int> &bin_off, int n_slots,
+                             const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog, bool own_books) {
   std::ostringstream o;
   o << "#include \"clexmc_metropolis.h\"\n#include \"clexmc_nfold.h\"\nnamespace clexmc {\n";
-  emit_field(o, "JitField", n_sublat, variable, binary, subs, bin_off, n_slots, gsubs, gen_prog, false, 64);
-  o << "}  // namespace clexmc\nextern \"C\" __global__ __launch_bounds__(64, " << kNfoldSingleWaves << ") void "
-    << kJitNfoldSingleName << "(clexmc::NfoldArgs na) { clexmc::nfold_body<" << (binary ? "true" : "false")
-    << ", clexmc::JitField, true>(na); }\n";
+  emit_field(o, "JitField", n_sublat, variable, binary, subs, bin_off, n_slots, gsubs, gen_prog, false, kAotMaxThreads);
+  o << "}  // namespace clexmc\nextern \"C\" __global__ __launch_bounds__(";
+  if (own_books) o << "64, " << kNfoldSingleWaves;
+  else o << kNfoldMaxThreads;
+  o << ") void " << (own_books ? kJitNfoldSingleName : kJitNfoldName) << "(clexmc::NfoldArgs na) { clexmc::nfold_body<"
+    << (binary ? "true" : "false") << ", clexmc::JitField, " << (own_books ? "true" : "false") << ">(na); }\n";
   return o.str();
 }
 

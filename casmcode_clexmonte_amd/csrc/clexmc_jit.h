@@ -41,10 +41,11 @@ std::string jit_source(int n_sublat, const std::vector<int> &variable, bool bina
                        const std::vector<int> &gen_prog, int kind, bool packed, int lanes, int max_threads,
                        const CubeSpec *cube = nullptr, bool spread = false);
 
-// The N-fold kernel for blocks of one wavefront (nfold_body, OWN_BOOKS).
-std::string jit_source_nfold_single(int n_sublat, const std::vector<int> &variable, bool binary,
-                                    const std::vector<BinSub> &subs, const std::vector<int> &bin_off, int n_slots,
-                                    const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog);
+// The N-fold kernel alone (kJitNfoldName); own_books: the one for blocks of one
+// wavefront (kJitNfoldSingleName).
+std::string jit_source_nfold(int n_sublat, const std::vector<int> &variable, bool binary,
+                             const std::vector<BinSub> &subs, const std::vector<int> &bin_off, int n_slots,
+                             const std::vector<GenSub> &gsubs, const std::vector<int> &gen_prog, bool own_books);
 
 // Table rows that each lane of a wavefront forms per site in the spread kernel
 // (the largest program of a variable sublattice, over 64 lanes); 0 where its
