@@ -242,9 +242,9 @@ static void emit_field(std::ostringstream &o, const std::string &name, int n_sub
     // rows in flight, and every add waits out most of an LDS latency.  The
     // empty asm statements order the batches (the sums pass through them, so
     // a batch's adds stay behind the next batch's loads).  The adds keep the
-    // entry order.  BCC 64^3, quaternary: 7.30 ms -> 6.94 ms per 8 passes (3 to
-    // 12 rows: 6.8 to 7.1); one wavefront per chain, ternary HCP 11 x 9 x 7:
-    // 23.3 ms -> 18.3 ms.  (Rows padded to 16 bytes, one ds_read_b96 each
+    // entry order.  32 chains of BCC 64^3, quaternary, 8 passes with the reads:
+    // 7.48 ms -> 7.10 ms (3 to 12 rows within 3 %); one wavefront per chain,
+    // ternary HCP 11 x 9 x 7: 23.7 ms -> 18.5 ms.  (Rows padded to 16 bytes, one ds_read_b96 each
     // instead of two reads, took 8.5 ms on BCC: the LDS is busy longer.)
     // Blocks above 512 threads have half the registers per lane
     // and keep the sites of large fields out of them: one batch, no order.

@@ -928,11 +928,14 @@ __global__ __launch_bounds__(kCollectThreads) void mlp_collect_kernel(CollectArg
 // [h > 0], so that nothing passes through memory between the two directions.
 // The products are formed in FP32 and summed in FP64.  Each block leaves its
 // FP64 sums in `part`; mlp_reduce_kernel adds the blocks in a fixed order.
-// A step moves 57 bytes per sample and is bound by the FP64 matrix rate
-// (48 MFMAs of 64 cycles per 16 samples).  Collection and 10 Adam steps on
-// 65,536 samples take 1.51 ms; one thread per sample forward and one per
-// parameter walking all samples (3,201 threads, every term read through
-// memory: 11.1 ms per step) took 116.1 ms.
+// A step moves 57 bytes per sample and is bound by latency at one wavefront per
+// SIMD: 65,536 samples take 46 us, of which the matrix units are busy 18 % (48
+// FP64 and 48 FP32 MFMAs per 16 samples) and the vector units issue 33 %; the
+// wavefronts wait for the samples' bytes 37 % of the time, and the blocks end
+// with four wavefronts adding their sums one after the other.  Collection and
+// 10 Adam steps on 65,536 samples take 0.90 ms; one thread per sample forward
+// and one per parameter walking all samples (3,201 threads, every term read
+// through memory: 11.1 ms per step) took 116.1 ms.
 // ---------------------------------------------------------------------------
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
