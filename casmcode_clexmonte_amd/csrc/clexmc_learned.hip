@@ -556,13 +556,15 @@ __global__ __launch_bounds__(TWICE ? 1024 : 512, TWICE || WEIGHTS == 1 ? 4 : 6) 
       // take one each.  A pair's word is its own: the counter is the pair's
       // place in the phase and the draw of the wavefront's stream.  Two pairs
       // on one word would be accepted together more often than apart)
-      for (int t = pb + tid; t < pe; t += nthr) {
-        const int2 pq = sc->pair_addr[t];
-        const int bpq = sc->pair_sublat[t];
+      for (int i = tid; i < pe - pb; i += nthr) {
+        const int2 pq = sc->pair_addr[pb + i];
+        const int bpq = sc->pair_sublat[pb + i];
+        // (the words while the pair's addresses are on their way)
+        uint4 ur = philox4x32_10(make_uint4((uint32_t)i, (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
+                                           (uint32_t)chain), k0, k1);
+        asm volatile("" : "+v"(ur.x), "+v"(ur.y));
         const int op = img[pq.x], oq = img[pq.y];
         if (op == oq) continue;
-        const uint4 ur = philox4x32_10(make_uint4((uint32_t)(t - pb), (uint32_t)draw, (uint32_t)(draw >> 32) | 0x80000000u,
-                                                 (uint32_t)chain), k0, k1);
         int Kp[kMaxSlots], Kq[kMaxSlots];
         const float Fp = binary_field_l(img, pq.x, op, cst(sc->bin_sub + (bpq & 0xFF)), bin_off, n_slots, Kp);
         const float Fq = binary_field_l(img, pq.y, oq, cst(sc->bin_sub + (bpq >> 8)), bin_off, n_slots, Kq);
@@ -996,6 +998,13 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(TrainArgs a) {
 #pragma unroll
       for (int tn = 0; tn < 4; ++tn) h[tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[ks], Wf[ks][tn], h[tn], 0, 0, 0);
     // lane (g, c) register r: sample s0 + 4 g + r, unit 16 tn + c
+    if (s0 + 16 > a.n) {
+      // rows past the batch add zeros, also where a parameter is not finite
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn) h[tn][r] = in_b[r] ? h[tn][r] : 0.0f;
+    }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float z = 0.0f;
@@ -1011,10 +1020,9 @@ __global__ __launch_bounds__(256) void mlp_step_kernel(TrainArgs a) {
       db2 += (double)dl;
 #pragma unroll
       for (int tn = 0; tn < 4; ++tn) {
-        // (a row past the batch adds zeros, also where a parameter is not finite)
-        const float D = in_b[r] && h[tn][r] > 0.f ? dl * W2[tn] : 0.0f;
+        const float D = h[tn][r] > 0.f ? dl * W2[tn] : 0.0f;
         db1[tn] += (double)D;
-        dW2[tn] += in_b[r] ? (double)(dl * fmaxf(h[tn][r], 0.f)) : 0.0;
+        dW2[tn] += (double)(dl * fmaxf(h[tn][r], 0.f));
 #pragma unroll
         for (int tk = 0; tk < 3; ++tk)
           dW1[tn][tk] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)D, (double)xb[r][tk], dW1[tn][tk], 0, 0, 0);
