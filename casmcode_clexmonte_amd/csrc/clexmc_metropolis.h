@@ -655,8 +655,13 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
   };
   // (Not in binary semi-grand canonical sweeps, which are bound by issue where
   // many chains fill the device: 20 passes of FCC 8^3, 2,048 chains, 1.83 ms
-  // ahead and 1.73 ms without; 16^3, 256 chains, 0.53 and 0.50 ms.)
-  constexpr bool kAhead = !(BIN && KIND == 1);
+  // ahead and 1.73 ms without; 16^3, 256 chains, 0.53 and 0.50 ms.  Nor with
+  // multiswaps, whose serial attempts would hold the values all along: one
+  // attempt per site, FCC 12^3, 2 passes of one chain, 15.6 ms ahead and
+  // 15.0 ms without; 8 attempts and 4 rounds per pass, 20 passes of 128 chains,
+  // FCC 16^3 3.71 and 3.52 ms, ternary HCP 6^3 9.42 and 8.96 ms, quaternary
+  // BCC 8^3 16.7 and 16.8 ms.)
+  constexpr bool kAhead = KIND == 0 || (KIND == 1 && !BIN);
   auto halo_at = [](const ClassNums &q, int t) -> int { return t < q.na ? q.a0 + t : q.b0 + (t - q.na); };
   auto class_first = [&](const ClassNums &q) -> ClassFirst {
     ClassFirst f{0, make_int2(0, 0)};
@@ -1047,7 +1052,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
           if (lane < n * nf) cF[(lane % nf) * max_class + lane / nf] = g;
         }
         for (int t = tid; t < n; t += nthr) {
-          const int pa = t == tid ? first.pa : sc->class_addr[R.at(t)];
+          const int pa = kAhead && t == tid ? first.pa : sc->class_addr[R.at(t)];
           const int o = img.get(pa);
           if (local) cO[t] = (uint8_t)o;
           if (BIN) {
@@ -1135,7 +1140,7 @@ __device__ __forceinline__ void metropolis_body(const RunArgs &args, const Block
         }
         if (local) {
           for (int t = tid; t < n; t += nthr) {
-            const int pa = t == tid ? first.pa : sc->class_addr[R.at(t)];
+            const int pa = kAhead && t == tid ? first.pa : sc->class_addr[R.at(t)];
             if constexpr (PACK) {
               const int o = img.get(pa), nw = cO[t];
               if (o != nw) img.set(pa, o, nw);
